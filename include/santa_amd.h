@@ -277,6 +277,14 @@ int santa_prop_decode_paged(const void* q, const void* K_pages, const void* V_pa
  * [M, storage, KVH, D]); bit for bit santa_rt_rope_write of santa_rt_linear's
  * output, without writing that output.  D even; the santa_rt_linear limits
  * on M and K.
+ * santa_rt_causal_attention: exact causal GQA attention of a prefill, D = 128
+ * (the HF model's own attention in the reference's prefill,
+ * tutorial_code/runtime_common.py:501-571): q [B, P, H, D], k, v [B, P, KVH,
+ * D], out [B, P, H, D] of one 16-bit type (enum santa_dtype); strides: 12 host
+ * values, the batch, position and head strides in elements of q, k, v, out
+ * (multiples of 8, the last dimension contiguous, the tensors 16-byte
+ * aligned).  Scores, softmax and sums in float32, the probabilities rounded
+ * to the 16-bit type for the second product.
  * santa_rt_argmax: out[r] (int64) = the index of the maximum of row r of
  * x [rows, n] (float32), torch.argmax's choice: NaN above any number, the
  * first index among equal values; the greedy step's token choice
@@ -291,6 +299,8 @@ int santa_rt_linear_rope(const void* x, const void* w, int M, int K, const void*
                          void* k_cache, void* v_cache, int H, int KVH, int D, long long storage, int pos,
                          hipStream_t stream);
 int santa_rt_argmax(const float* x, int rows, int n, long long* out, hipStream_t stream);
+int santa_rt_causal_attention(const void* q, const void* k, const void* v, void* out, int dtype, int B, int P, int H,
+                              int KVH, int D, const long long* strides, hipStream_t stream);
 
 #ifdef __cplusplus
 }

@@ -24,6 +24,7 @@ from dataclasses import dataclass
 from typing import Dict, List, Optional
 
 import torch
+import torch.autograd.forward_ad as fwAD
 import torch.nn.functional as F
 
 __all__ = ["LlamaShape", "LLAMA_3_1_8B", "RandomLlama", "NHDCache", "ExactDecodeBackend", "causal_attention",
@@ -87,6 +88,8 @@ class _FusedOps:
             L.santa_rt_linear_rope.argtypes = [ctypes.c_void_p] * 2 + [ctypes.c_int] * 2 + [ctypes.c_void_p] * 5 + [
                 ctypes.c_int] * 3 + [ctypes.c_longlong, ctypes.c_int, ctypes.c_void_p]
             L.santa_rt_argmax.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p]
+            L.santa_rt_causal_attention.argtypes = [ctypes.c_void_p] * 4 + [ctypes.c_int] * 6 + [
+                ctypes.POINTER(ctypes.c_longlong), ctypes.c_void_p]
             cls._lib = L
         return cls._lib
 
@@ -175,6 +178,28 @@ class _FusedOps:
         cls._check(cls.lib().santa_rt_argmax(logits.data_ptr(), rows, n, out.data_ptr(), cls._stream(logits)))
         return out
 
+    @staticmethod
+    def _attention_strides_fit(t: torch.Tensor) -> bool:
+        """Whether the attention kernels can address t [..., heads, 128]:
+        last dimension contiguous, the other strides multiples of 8 elements,
+        16-byte aligned storage."""
+        return (t.stride(-1) == 1 and all(s % 8 == 0 and s < 1 << 24 for s in t.stride()[1:-1])
+                and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0)
+
+    @classmethod
+    def causal_attention(cls, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> torch.Tensor:
+        """causal_attention of [B, P, heads, 128] tensors as one kernel."""
+        q, k, v = (t if cls._attention_strides_fit(t) else t.contiguous() for t in (q, k, v))
+        q, k, v = (t if t.data_ptr() % 16 == 0 else t.clone() for t in (q, k, v))
+        B, P, H, D = q.shape
+        out = torch.empty(B, P, H, D, dtype=q.dtype, device=q.device)
+        strides = (ctypes.c_longlong * 12)(*(s for t in (q, k, v, out) for s in t.stride()[:3]))
+        with torch.cuda.device(q.device):
+            cls._check(cls.lib().santa_rt_causal_attention(
+                q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), int(q.dtype == torch.float16), B, P, H,
+                k.shape[2], D, strides, cls._stream(q)))
+        return out
+
     @classmethod
     def silu_mul(cls, gu: torch.Tensor) -> torch.Tensor:
         assert gu.is_contiguous()
@@ -202,15 +227,40 @@ def _apply_rope(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.
     return x * cos + _rotate_half(x) * sin
 
 
+def _plain(*ts: torch.Tensor) -> bool:
+    """Ordinary tensors outside autograd, forward-mode differentiation,
+    functorch transforms and tracing: what a kernel behind raw pointers may
+    take in place of torch operations."""
+    if torch.is_grad_enabled() and any(t.requires_grad for t in ts):
+        return False
+    if torch.compiler.is_compiling() or torch.jit.is_tracing():
+        return False
+    return all(type(t) is torch.Tensor and not torch._C._functorch.is_functorch_wrapped_tensor(t)
+               and (fwAD._current_level < 0 or fwAD.unpack_dual(t).tangent is None) for t in ts)
+
+
+def _causal_kernel_takes(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> bool:
+    """Whether causal_attention runs as the library's kernel: bf16 or f16
+    tensors of head_dim 128 on one GPU."""
+    return (q.is_cuda and q.dtype in (torch.bfloat16, torch.float16) and k.dtype == q.dtype and v.dtype == q.dtype
+            and k.device == q.device and v.device == q.device and q.dim() == 4 and q.shape[-1] == 128
+            and k.shape == v.shape and k.shape[:2] == q.shape[:2] and k.shape[-1] == 128
+            and q.numel() > 0 and k.shape[2] > 0 and q.shape[2] % k.shape[2] == 0 and _plain(q, k, v))
+
+
 def causal_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, chunk: int = 512) -> torch.Tensor:
     """Exact causal GQA attention for a prefill: q [B, P, H, D], k/v
-    [B, P, KVH, D] -> [B, P, H, D].  Query chunks of `chunk` positions; the
-    products run on contiguous operands only (K is transposed once per call
-    into a contiguous copy and every chunk is scored against all of it, the
-    future positions masked), scores in the input dtype, softmax in float32."""
+    [B, P, KVH, D] -> [B, P, H, D].  bf16 and f16 tensors of head_dim 128 on a
+    GPU run as one kernel (float32 scores and softmax).  Otherwise, and under
+    autograd, query chunks of `chunk` positions; the products run on contiguous
+    operands only (K is transposed once per call into a contiguous copy and
+    every chunk is scored against all of it, the future positions masked),
+    scores in the input dtype, softmax in float32."""
     B, P, H, D = q.shape
     KVH = k.shape[2]
     GH = H // KVH
+    if chunk > 0 and _causal_kernel_takes(q, k, v):
+        return _FusedOps.causal_attention(q, k, v)
     scale = 1.0 / math.sqrt(D)
     kt = k.permute(0, 2, 3, 1).reshape(B * KVH, D, P).contiguous()      # [B*KVH, D, P]
     vv = v.permute(0, 2, 1, 3).reshape(B * KVH, P, D).contiguous()      # [B*KVH, P, D]
