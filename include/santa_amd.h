@@ -285,6 +285,13 @@ int santa_prop_decode_paged(const void* q, const void* K_pages, const void* V_pa
  * (multiples of 8, the last dimension contiguous, the tensors 16-byte
  * aligned).  Scores, softmax and sums in float32, the probabilities rounded
  * to the 16-bit type for the second product.
+ * santa_rt_exact_decode: exact decode attention in float32, D = 128: q, out
+ * [B, H, D] contiguous, k, v [B, L.., KVH, D] of which the first L positions
+ * count, one 16-bit type (enum santa_dtype); strides: 6 host values, the
+ * batch, position and head strides in elements of k and v (multiples of 8, the
+ * last dimension contiguous, the tensors 16-byte aligned).  workspace:
+ * santa_rt_exact_decode_workspace_size bytes, 16-byte aligned, needing no
+ * initialization.
  * santa_rt_argmax: out[r] (int64) = the index of the maximum of row r of
  * x [rows, n] (float32), torch.argmax's choice: NaN above any number, the
  * first index among equal values; the greedy step's token choice
@@ -301,6 +308,10 @@ int santa_rt_linear_rope(const void* x, const void* w, int M, int K, const void*
 int santa_rt_argmax(const float* x, int rows, int n, long long* out, hipStream_t stream);
 int santa_rt_causal_attention(const void* q, const void* k, const void* v, void* out, int dtype, int B, int P, int H,
                               int KVH, int D, const long long* strides, hipStream_t stream);
+size_t santa_rt_exact_decode_workspace_size(int B, int L, int H, int KVH);
+int santa_rt_exact_decode(const void* q, const void* k, const void* v, void* out, int dtype, int B, int L, int H,
+                          int KVH, int D, const long long* strides, void* workspace, size_t workspace_bytes,
+                          hipStream_t stream);
 
 #ifdef __cplusplus
 }

@@ -1,7 +1,8 @@
 // santa_attn.hip -- exact attention of the model-level runtime
-// (santa_amd/runtime.py) at head_dim 128: the causal attention of a prefill.
-// The reference leaves it to the HF model's own attention
-// (tutorial_code/runtime_common.py:501-571).
+// (santa_amd/runtime.py) at head_dim 128: the causal attention of a prefill and
+// the decode attention of the exact comparator.  The reference leaves both to
+// torch's and the HF model's own attention (tutorial_code/runtime_common.py:
+// 501-571, tutorial_code/attention_backends.py:70-89).
 #include "santa_device.h"
 #include "santa_amd.h"
 #include "santa_internal.h"
@@ -13,6 +14,7 @@ namespace attn {
 
 constexpr int kD = 128;
 constexpr int kBufWord3 = 0x00020000;  // raw buffer descriptor, gfx9 family
+constexpr int kBufNontemporal = 2;     // the "nt" cache-policy bit
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -265,6 +267,244 @@ __global__ __launch_bounds__(64 * NW, 2) void causal_attention_kernel(
     }
 }
 
+// ------------------------------------------------------------ exact decode
+// Exact decode attention: one query row per sequence over its first L cached
+// positions, everything in float32 (the 16-bit operands are exact; products,
+// scores, probabilities and sums are float32).
+//
+// A wave takes one item, a chunk of positions of one (sequence, KV head, up to
+// GHP of its query heads).  16 lanes hold a K or V row (16 bytes each), so a
+// load instruction covers 4 rows and a step 32 positions: the scores are
+// v_dot2 chains over the lane's 8 dims summed over the row's 16 lanes by
+// halving exchanges (each head's score ends in 16 / GHP of them), the step's
+// maximum meets across the 4 rows, and each probability goes back to its row's
+// lanes by a DPP broadcast for the V sums.  Matrix cores would not help: at GH
+// query rows the call reads 2 bytes per 2 GH multiply-adds.  The next step's
+// K rows are loaded once this step's scores are formed and its V rows once
+// this step's are summed, so 8 to 16 KiB per wave are in flight throughout.
+// The KV heads of a chunk are neighbours in launch order (8 waves of a
+// workgroup), so whole NHD rows are read at about the same time.  Bound by
+// reading K and V once: B = 8, 32k, 32q/8kv takes 171 us with its merge (6.27
+// TB/s), 32q/32kv at 8k 168 us (6.39 TB/s); eight heads per KV head double the
+// vector work per row (219 us, 4.90 TB/s).  B = 4, 4k: 21 us against 155 us for
+// the torch products on float32 copies of both caches it replaces.
+constexpr int kDecWaves = 8;
+constexpr int kDecStep = 32;              // positions per step
+constexpr int kPartStride = kD + 2;       // chunk partial: max (log2 units), mass, numerator[128]
+constexpr int kMaxChunks = 256;           // chunks per sequence (the merge holds one per thread)
+
+template <bool BF16>
+__device__ __forceinline__ float dot8(u32x4 a, u32x4 b) {
+  typedef typename Half8<BF16>::T H8;
+  const H8 x = __builtin_bit_cast(H8, a), y = __builtin_bit_cast(H8, b);
+  float acc = 0.0f;
+  if constexpr (BF16) {
+    acc = __builtin_amdgcn_fdot2_f32_bf16(x.s01, y.s01, acc, false);
+    acc = __builtin_amdgcn_fdot2_f32_bf16(x.s23, y.s23, acc, false);
+    acc = __builtin_amdgcn_fdot2_f32_bf16(x.s45, y.s45, acc, false);
+    return __builtin_amdgcn_fdot2_f32_bf16(x.s67, y.s67, acc, false);
+  } else {
+    acc = __builtin_amdgcn_fdot2(x.s01, y.s01, acc, false);
+    acc = __builtin_amdgcn_fdot2(x.s23, y.s23, acc, false);
+    acc = __builtin_amdgcn_fdot2(x.s45, y.s45, acc, false);
+    return __builtin_amdgcn_fdot2(x.s67, y.s67, acc, false);
+  }
+}
+
+// v of lane N of this lane's 16-lane row.
+template <int N>
+__device__ __forceinline__ float row_bcast(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + N, 0xF, 0xF, true));
+}
+// f(integral_constant<int, 0>) ... f(integral_constant<int, N - 1>).
+template <int N, class F, int I = 0>
+__device__ __forceinline__ void static_for(F f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    static_for<N, F, I + 1>(f);
+  }
+}
+
+template <bool BF16, int GHP>
+__global__ __launch_bounds__(64 * kDecWaves) void exact_decode_kernel(
+    const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K, const uint16_t* __restrict__ V, Strides sk,
+    Strides sv, int L, int H, int KVH, int GH, int groups, int chunk, int cpg, long long items, float scale_log2,
+    float* __restrict__ part) {
+  constexpr int SH = GHP == 1 ? 0 : GHP == 2 ? 1 : GHP == 4 ? 2 : 3;
+  const int lane = threadIdx.x & 63;
+  const long long item =
+      static_cast<long long>(blockIdx.x) * kDecWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (item >= items) return;
+  // items: (sequence, chunk, KV head, head group), the last fastest
+  const int grp = static_cast<int>(item % groups);
+  const int kv = static_cast<int>(item / groups % KVH);
+  const int c = static_cast<int>(item / groups / KVH % cpg);
+  const int b = static_cast<int>(item / groups / KVH / cpg);
+  const int h0 = kv * GH + grp * GHP;
+  const int nh = min(GHP, GH - grp * GHP);
+  const int n_begin = c * chunk, n_end = min(L, n_begin + chunk);
+  const int r = lane >> 4, p = lane & 15;
+
+  u32x4 q[GHP];
+#pragma unroll
+  for (int g = 0; g < GHP; ++g)
+    q[g] = *reinterpret_cast<const u32x4*>(Q + (static_cast<size_t>(b) * H + h0 + min(g, nh - 1)) * kD + 8 * p);
+
+  const char* Kg = reinterpret_cast<const char*>(K + b * sk.b + kv * sk.h);
+  const char* Vg = reinterpret_cast<const char*>(V + b * sv.b + kv * sv.h);
+  const uint32_t k_row = static_cast<uint32_t>(sk.p * 2), v_row = static_cast<uint32_t>(sv.p * 2);
+  // rows n .. n + 31, 4 per load; rows at or past the chunk's end read as zero
+  auto load = [&](u32x4 (&w)[8], const char* base, uint32_t row, int n) {
+    const int nvalid = min(n_end - n, kDecStep);
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<char*>(base) + static_cast<size_t>(nvalid > 0 ? n : n_begin) * row, static_cast<short>(0),
+        nvalid > 0 ? static_cast<int>((nvalid - 1) * row + 2 * kD) : 0, kBufWord3);
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      w[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, (4 * i + r) * row + 16 * p, 0,
+                                                                             kBufNontemporal));
+  };
+  u32x4 kw[8], vw[8];
+  load(kw, Kg, k_row, n_begin);
+  load(vw, Vg, v_row, n_begin);
+
+  float o[GHP][8];
+#pragma unroll
+  for (int g = 0; g < GHP; ++g)
+#pragma unroll
+    for (int d = 0; d < 8; ++d) o[g][d] = 0.0f;
+  // of the head whose scores end in this lane: running max (raw scores) and
+  // the mass of this row's positions
+  float m = -__builtin_inff(), l = 0.0f;
+
+  for (int n = n_begin; n < n_end; n += kDecStep) {
+    float s[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      typedef float acc_t __attribute__((ext_vector_type(GHP == 1 ? 2 : GHP)));
+      acc_t a = {};
+#pragma unroll
+      for (int g = 0; g < GHP; ++g) a[g] = dot8<BF16>(kw[i], q[g]);
+      lane_reduce<GHP, 8>(a, lane);
+      s[i] = (n + 4 * i + r < n_end) ? a[0] : -__builtin_inff();
+    }
+    load(kw, Kg, k_row, n + kDecStep);
+    float mx = s[0];
+#pragma unroll
+    for (int i = 1; i < 8; ++i) mx = fmaxf(mx, s[i]);
+    mx = fmaxf(mx, fxor<16>(mx, lane));
+    mx = fmaxf(mx, fxor<32>(mx, lane));
+    const float m_new = fmaxf(m, mx);
+    if (__any(m_new > m)) {
+      const float a = __builtin_amdgcn_exp2f((m - m_new) * scale_log2);
+      l *= a;
+      static_for<GHP>([&](auto gc) {
+        constexpr int g = decltype(gc)::value;
+        const float ag = row_bcast<g << (4 - SH)>(a);
+#pragma unroll
+        for (int d = 0; d < 8; ++d) o[g][d] *= ag;
+      });
+      m = m_new;
+    }
+    const float mc = m * scale_log2;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      s[i] = __builtin_amdgcn_exp2f(fmaf(s[i], scale_log2, -mc));
+      l += s[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      float v[8];
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        v[2 * d] = lo16_to_f32<BF16>(vw[i][d]);
+        v[2 * d + 1] = hi16_to_f32<BF16>(vw[i][d]);
+      }
+      static_for<GHP>([&](auto gc) {
+        constexpr int g = decltype(gc)::value;
+        const float pg = row_bcast<g << (4 - SH)>(s[i]);
+#pragma unroll
+        for (int d = 0; d < 8; ++d) o[g][d] = fmaf(pg, v[d], o[g][d]);
+      });
+    }
+    load(vw, Vg, v_row, n + kDecStep);
+  }
+  // the 4 rows' sums
+  l += fxor<16>(l, lane);
+  l += fxor<32>(l, lane);
+  static_for<GHP>([&](auto gc) {
+    constexpr int g = decltype(gc)::value;
+#pragma unroll
+    for (int d = 0; d < 8; ++d) {
+      o[g][d] += fxor<16>(o[g][d], lane);
+      o[g][d] += fxor<32>(o[g][d], lane);
+    }
+    const float mg = row_bcast<g << (4 - SH)>(m), lg = row_bcast<g << (4 - SH)>(l);
+    if (g < nh && r == (g & 3)) {
+      // partials [sequence, head, chunk]
+      float* pp = part + ((static_cast<size_t>(b) * H + h0 + g) * cpg + c) * kPartStride;
+      if (p == 0) *reinterpret_cast<float2*>(pp) = make_float2(mg * scale_log2, lg);
+#pragma unroll
+      for (int d = 0; d < 8; d += 2) *reinterpret_cast<float2*>(pp + 2 + 8 * p + d) = make_float2(o[g][d], o[g][d + 1]);
+    }
+  });
+}
+
+// out[d] = sum_c w_c num_c[d] / sum_c w_c mass_c, w_c = 2^(max_c - max), per
+// (sequence, head): 256 threads, thread c weighing chunk c, then two threads
+// per dim over the even and the odd chunks.
+template <bool BF16>
+__global__ __launch_bounds__(256) void exact_merge_kernel(const float* __restrict__ part, int cpg,
+                                                          uint16_t* __restrict__ out) {
+  __shared__ float s_w[kMaxChunks];
+  __shared__ float s_red[8];
+  __shared__ float s_o[kD];
+  const size_t bh = blockIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const float* pb = part + bh * cpg * kPartStride;
+  float2 ml = make_float2(-__builtin_inff(), 0.0f);
+  if (tid < cpg) ml = *reinterpret_cast<const float2*>(pb + static_cast<size_t>(tid) * kPartStride);
+  float mx = ml.x;
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) mx = fmaxf(mx, __shfl_xor(mx, d, 64));
+  if (lane == 0) s_red[wave] = mx;
+  __syncthreads();
+  mx = fmaxf(fmaxf(s_red[0], s_red[1]), fmaxf(s_red[2], s_red[3]));
+  const float w = tid < cpg ? __builtin_amdgcn_exp2f(ml.x - mx) : 0.0f;
+  s_w[tid] = w;
+  float z = tid < cpg ? w * ml.y : 0.0f;
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) z += __shfl_xor(z, d, 64);
+  if (lane == 0) s_red[4 + wave] = z;
+  __syncthreads();
+  z = (s_red[4] + s_red[5]) + (s_red[6] + s_red[7]);
+  const int d = tid & (kD - 1);
+  float acc = 0.0f;
+#pragma unroll 16
+  for (int c = tid >> 7; c < cpg; c += 2) acc = fmaf(s_w[c], pb[static_cast<size_t>(c) * kPartStride + 2 + d], acc);
+  if (tid >= kD) s_o[d] = acc;
+  __syncthreads();
+  if (tid < kD) out[bh * kD + d] = f32_to_h16<BF16>((acc + s_o[d]) / z);
+}
+
+// Chunks of the exact decode: about one resident round of waves (two per SIMD,
+// what the widest form's registers hold), at least 64 positions each, at most
+// kMaxChunks per sequence.
+void plan_decode(int B, int L, int KVH, int groups, int* chunk, int* cpg) {
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+    cus = 256;
+  const long long per_seq = static_cast<long long>(KVH) * groups * B;
+  const long long want = (8LL * cus + per_seq - 1) / per_seq;  // chunks per sequence
+  const long long n = want < 1 ? 1 : want > kMaxChunks ? kMaxChunks : want;
+  long long len = (L + n - 1) / n;
+  len = (len + kDecStep - 1) / kDecStep * kDecStep;
+  if (len < 64) len = 64;
+  *chunk = static_cast<int>(len);
+  *cpg = static_cast<int>((L + len - 1) / len);
+}
+
 }  // namespace attn
 }  // namespace santa
 
@@ -310,5 +550,63 @@ extern "C" int santa_rt_causal_attention(const void* q, const void* k, const voi
                        static_cast<int>(W), scale_log2);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return set_error(SANTA_ERR_HIP, "causal_attention launch failed: %s", hipGetErrorString(e));
+  return clear_error();
+}
+
+extern "C" size_t santa_rt_exact_decode_workspace_size(int B, int L, int H, int KVH) {
+  if (B <= 0 || L <= 0 || KVH <= 0 || H <= 0 || H % KVH != 0) return 0;
+  int chunk, cpg;
+  attn::plan_decode(B, L, KVH, (H / KVH + 7) / 8, &chunk, &cpg);
+  return static_cast<size_t>(B) * H * cpg * attn::kPartStride * sizeof(float);
+}
+
+extern "C" int santa_rt_exact_decode(const void* q, const void* k, const void* v, void* out, int dtype, int B, int L,
+                                     int H, int KVH, int D, const long long* strides, void* workspace,
+                                     size_t workspace_bytes, hipStream_t stream) {
+  if (!q || !k || !v || !out || !strides || !workspace || (dtype != SANTA_BF16 && dtype != SANTA_F16) || B <= 0 ||
+      L <= 0 || KVH <= 0 || H <= 0 || H % KVH != 0)
+    return set_error(SANTA_ERR_INVALID, "bad exact_decode arguments");
+  if (D != attn::kD) return set_error(SANTA_ERR_UNSUPPORTED, "exact_decode: D must be 128. Got D=%d", D);
+  const attn::Strides sk{strides[0], strides[1], strides[2]}, sv{strides[3], strides[4], strides[5]};
+  if (reinterpret_cast<uintptr_t>(q) % 16 != 0 || !strides_fit(sk, k) || !strides_fit(sv, v))
+    return set_error(SANTA_ERR_INVALID, "exact_decode: strides must be multiples of 8 elements (the position stride "
+                                        "below 2^24) and the tensors 16-byte aligned");
+  if (workspace_bytes < santa_rt_exact_decode_workspace_size(B, L, H, KVH))
+    return set_error(SANTA_ERR_WORKSPACE, "exact_decode: workspace too small");
+  const int GH = H / KVH, groups = (GH + 7) / 8;
+  int chunk, cpg;
+  attn::plan_decode(B, L, KVH, groups, &chunk, &cpg);
+  const long long items = static_cast<long long>(B) * KVH * groups * cpg;
+  const long long grid = (items + attn::kDecWaves - 1) / attn::kDecWaves;
+  if (grid > 0x7fffffffLL || static_cast<long long>(B) * H > 0x7fffffffLL)
+    return set_error(SANTA_ERR_INVALID, "exact_decode: batch too large");
+  const float scale_log2 = 1.44269504088896340736f / sqrtf(static_cast<float>(D));
+  const uint16_t *qp = static_cast<const uint16_t*>(q), *kp = static_cast<const uint16_t*>(k),
+                 *vp = static_cast<const uint16_t*>(v);
+  float* part = static_cast<float*>(workspace);
+  auto launch = [&](auto bf, auto ghp) {
+    constexpr bool BF16 = decltype(bf)::value;
+    constexpr int GHP = decltype(ghp)::value;
+    hipLaunchKernelGGL((attn::exact_decode_kernel<BF16, GHP>), dim3(static_cast<unsigned>(grid)),
+                       dim3(64 * attn::kDecWaves), 0, stream, qp, kp, vp, sk, sv, L, H, KVH, GH, groups, chunk, cpg,
+                       items, scale_log2, part);
+  };
+  auto pick = [&](auto bf) {
+    if (GH == 1) launch(bf, std::integral_constant<int, 1>{});
+    else if (GH == 2) launch(bf, std::integral_constant<int, 2>{});
+    else if (GH <= 4) launch(bf, std::integral_constant<int, 4>{});
+    else launch(bf, std::integral_constant<int, 8>{});
+  };
+  if (dtype == SANTA_BF16) {
+    pick(std::true_type{});
+    hipLaunchKernelGGL(attn::exact_merge_kernel<true>, dim3(static_cast<unsigned>(B) * H), dim3(256), 0, stream, part,
+                       cpg, static_cast<uint16_t*>(out));
+  } else {
+    pick(std::false_type{});
+    hipLaunchKernelGGL(attn::exact_merge_kernel<false>, dim3(static_cast<unsigned>(B) * H), dim3(256), 0, stream, part,
+                       cpg, static_cast<uint16_t*>(out));
+  }
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return set_error(SANTA_ERR_HIP, "exact_decode launch failed: %s", hipGetErrorString(e));
   return clear_error();
 }

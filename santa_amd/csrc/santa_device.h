@@ -486,6 +486,36 @@ __device__ __forceinline__ int lane_xor(int v, int lane) {
   }
 }
 
+template <int J>
+__device__ __forceinline__ float fxor(float v, int lane) {
+  return __int_as_float(lane_xor<J>(__float_as_int(v), lane));
+}
+
+// Sums of V per-lane values over the wave, each ending in its own lanes.
+// Halving exchanges at distance D = 32, 16, ...: both lanes of a pair add
+// the pair's copies of both halves and keep the half their bit D selects
+// (upper for the lane with the bit set), so after log2(V) steps the lane's
+// element 0 is index lane >> (6 - log2 V); the remaining distances then sum
+// it over the other lanes.  Every index goes through the same tree of
+// lanes, so a value's sum does not depend on its index.
+template <int V, int D, typename T>
+__device__ __forceinline__ void lane_reduce(T& acc, int lane) {
+  if constexpr (V > 1) {
+    constexpr int H = V / 2;
+    const bool hi = (lane & D) != 0;
+#pragma unroll
+    for (int i = 0; i < H; ++i) {
+      const float lo = acc[i] + fxor<D>(acc[i], lane);
+      const float up = acc[i + H] + fxor<D>(acc[i + H], lane);
+      acc[i] = hi ? up : lo;
+    }
+    lane_reduce<H, D / 2>(acc, lane);
+  } else if constexpr (D >= 1) {
+    acc[0] += fxor<D>(acc[0], lane);
+    lane_reduce<1, D / 2>(acc, lane);
+  }
+}
+
 // Chunk sums of the finalize kernels: s += fv(c) and e += fe(c) (fe only
 // where with_e) over chunks c = 0 .. n - 1 in ascending order, the loads of up
 // to 32 chunks issued before the first add: full batches of 32, then one batch

@@ -90,6 +90,10 @@ class _FusedOps:
             L.santa_rt_argmax.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p]
             L.santa_rt_causal_attention.argtypes = [ctypes.c_void_p] * 4 + [ctypes.c_int] * 6 + [
                 ctypes.POINTER(ctypes.c_longlong), ctypes.c_void_p]
+            L.santa_rt_exact_decode_workspace_size.restype = ctypes.c_size_t
+            L.santa_rt_exact_decode_workspace_size.argtypes = [ctypes.c_int] * 4
+            L.santa_rt_exact_decode.argtypes = [ctypes.c_void_p] * 4 + [ctypes.c_int] * 6 + [
+                ctypes.POINTER(ctypes.c_longlong), ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]
             cls._lib = L
         return cls._lib
 
@@ -201,6 +205,26 @@ class _FusedOps:
         return out
 
     @classmethod
+    def exact_decode(cls, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, L: int) -> torch.Tensor:
+        """Exact float32 attention of q [B, H, 128] over the first L positions
+        of k, v [B, T, KVH, 128]."""
+        q = q.contiguous()
+        k, v = (t if cls._attention_strides_fit(t) else t[:, :L].contiguous() for t in (k, v))
+        q, k, v = (t if t.data_ptr() % 16 == 0 else t.clone() for t in (q, k, v))
+        B, H, D = q.shape
+        KVH = k.shape[2]
+        out = torch.empty(B, H, D, dtype=q.dtype, device=q.device)
+        strides = (ctypes.c_longlong * 6)(*(s for t in (k, v) for s in t.stride()[:3]))
+        lib = cls.lib()
+        with torch.cuda.device(q.device):
+            ws = torch.empty(lib.santa_rt_exact_decode_workspace_size(B, L, H, KVH), dtype=torch.uint8,
+                             device=q.device)
+            cls._check(lib.santa_rt_exact_decode(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
+                                                 int(q.dtype == torch.float16), B, L, H, KVH, D, strides,
+                                                 ws.data_ptr(), ws.numel(), cls._stream(q)))
+        return out
+
+    @classmethod
     def silu_mul(cls, gu: torch.Tensor) -> torch.Tensor:
         assert gu.is_contiguous()
         inter = gu.shape[-1] // 2
@@ -239,13 +263,14 @@ def _plain(*ts: torch.Tensor) -> bool:
                and (fwAD._current_level < 0 or fwAD.unpack_dual(t).tangent is None) for t in ts)
 
 
-def _causal_kernel_takes(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> bool:
-    """Whether causal_attention runs as the library's kernel: bf16 or f16
-    tensors of head_dim 128 on one GPU."""
+def _attention_kernel_takes(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> bool:
+    """Whether the library's attention kernels take q [.., H, D] with k, v
+    [B, T, KVH, D]: bf16 or f16 tensors of head_dim 128 on one GPU, whole
+    groups of query heads."""
     return (q.is_cuda and q.dtype in (torch.bfloat16, torch.float16) and k.dtype == q.dtype and v.dtype == q.dtype
-            and k.device == q.device and v.device == q.device and q.dim() == 4 and q.shape[-1] == 128
-            and k.shape == v.shape and k.shape[:2] == q.shape[:2] and k.shape[-1] == 128
-            and q.numel() > 0 and k.shape[2] > 0 and q.shape[2] % k.shape[2] == 0 and _plain(q, k, v))
+            and k.device == q.device and v.device == q.device and k.dim() == 4 and k.shape == v.shape
+            and q.shape[-1] == 128 and k.shape[-1] == 128 and k.shape[0] == q.shape[0] and q.numel() > 0
+            and k.shape[2] > 0 and q.shape[-2] % k.shape[2] == 0 and _plain(q, k, v))
 
 
 def causal_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, chunk: int = 512) -> torch.Tensor:
@@ -259,7 +284,7 @@ def causal_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, chunk
     B, P, H, D = q.shape
     KVH = k.shape[2]
     GH = H // KVH
-    if chunk > 0 and _causal_kernel_takes(q, k, v):
+    if chunk > 0 and k.shape[1] == P and _attention_kernel_takes(q, k, v):
         return _FusedOps.causal_attention(q, k, v)
     scale = 1.0 / math.sqrt(D)
     kt = k.permute(0, 2, 3, 1).reshape(B * KVH, D, P).contiguous()      # [B*KVH, D, P]
@@ -283,9 +308,11 @@ def causal_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, chunk
 
 
 class ExactDecodeBackend:
-    """Exact dense decode attention in float32 with contiguous operands only
-    (the comparator of the model-level decode; same adapter contract as the
-    backends in santa_amd.attention_backends)."""
+    """Exact dense decode attention in float32 (the comparator of the
+    model-level decode; same adapter contract as the backends in
+    santa_amd.attention_backends): one kernel pass over the caches for bf16 and
+    f16 of head_dim 128 on a GPU, else torch products on contiguous float32
+    copies."""
 
     name = "exact_fp32"
     exact_attention = True
@@ -296,6 +323,8 @@ class ExactDecodeBackend:
         KVH = k_nhd.shape[2]
         GH = H // KVH
         L = int(valid_len)
+        if q_bhd.dim() == 3 and 0 < L <= k_nhd.shape[1] and _attention_kernel_takes(q_bhd, k_nhd, v_nhd):
+            return _FusedOps.exact_decode(q_bhd, k_nhd, v_nhd, L)
         k = k_nhd[:, :L].permute(0, 2, 1, 3).reshape(B * KVH, L, D).float().contiguous()    # [B*KVH, L, D]
         v = v_nhd[:, :L].permute(0, 2, 1, 3).reshape(B * KVH, L, D).float().contiguous()
         q = q_bhd.float().reshape(B * KVH, GH, D).transpose(1, 2).contiguous()              # [B*KVH, D, GH]

@@ -2,9 +2,10 @@
 PyTorch float32.
 
 Tolerance of the causal kernel: probabilities and output are rounded to the
-16-bit type (relative 2^-9 in bf16, 2^-12 in f16) and the sums are float32, so
-an element is off by at most half an ulp of itself plus the rounding of the
-probabilities, which an output of |v| <= vmax scales to 2^-9 vmax (2^-12);
+16-bit type and the sums are float32.  Rounding to a p-bit significand is off by
+at most half an ulp, 2^-p of the value (p = 8 in bf16, 11 in f16).  So an
+element is off by at most 2^-p of itself plus the rounding of the
+probabilities, which an output of |v| <= vmax scales to 2^-p vmax;
 the float32 score sums over 128 products of magnitude <= 25 add
 128 x 2^-24 x 25 = 2e-4 relative to every probability.
 
@@ -15,7 +16,7 @@ import math
 import pytest
 import torch
 
-from santa_amd.runtime import causal_attention
+from santa_amd.runtime import ExactDecodeBackend, causal_attention
 
 pytestmark = pytest.mark.gpu
 
@@ -34,7 +35,7 @@ def _ref(q, k, v):
 
 
 def _check(out, ref, v, dtype):
-    eps = 2.0 ** -9 if dtype == torch.bfloat16 else 2.0 ** -12
+    eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
     vmax = v.float().abs().max().item()
     bound = eps * ref.abs() + (eps + 2e-4) * vmax
     err = (out.float() - ref).abs()
@@ -86,7 +87,7 @@ def test_causal_attention_large_scores():
     q, k, v = (t.to("cuda", torch.bfloat16) for t in (q, k, v))
     out, ref = causal_attention(q, k, v), _ref(q, k, v)
     # scores up to 850 carry 128 x 2^-24 x 850 = 6.5e-3 of absolute rounding
-    assert ((out.float() - ref).abs() <= 2.0 ** -9 * ref.abs() + (2.0 ** -9 + 1.3e-2) * v.float().abs().max()).all()
+    assert ((out.float() - ref).abs() <= 2.0 ** -8 * ref.abs() + (2.0 ** -8 + 1.3e-2) * v.float().abs().max()).all()
 
 
 def test_causal_attention_keeps_autograd():
@@ -95,3 +96,60 @@ def test_causal_attention_keeps_autograd():
     q, k, v = (torch.randn(1, 40, h, 128, device="cuda", dtype=torch.bfloat16, requires_grad=True) for h in (4, 1, 1))
     causal_attention(q.float(), k.float(), v.float()).sum().backward()
     assert all(t.grad is not None and torch.isfinite(t.grad).all() for t in (q, k, v))
+
+
+def _ref_decode(q, k, v, L):
+    """float64 decode attention, head by head."""
+    B, H, D = q.shape
+    G = H // k.shape[2]
+    out = torch.empty(B, H, D, device=q.device, dtype=torch.float64)
+    for b in range(B):
+        for h in range(H):
+            s = k[b, :L, h // G].double().contiguous() @ q[b, h].double() / math.sqrt(D)
+            out[b, h] = torch.softmax(s, 0) @ v[b, :L, h // G].double().contiguous()
+    return out
+
+
+def _check_decode(out, ref, v, dtype):
+    # the output's own rounding (2^-p, as above), and float32 throughout: scores of magnitude
+    # <= 25 over 128 products carry 2e-4 relative into every probability
+    eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    bound = eps * ref.abs() + 2e-4 * v.double().abs().max()
+    err = (out.double() - ref).abs()
+    assert torch.isfinite(out).all() and (err <= bound).all(), (err / bound).max().item()
+
+
+# lengths around the 32-position steps and 64-position chunks, one chunk and
+# many; every group-size form, idle head slots, two head groups, item counts
+# that do not fill a workgroup
+@pytest.mark.parametrize("B,L,H,KVH,dtype", [
+    (1, 1, 8, 2, torch.bfloat16), (2, 31, 4, 4, torch.float16), (1, 32, 2, 1, torch.bfloat16),
+    (3, 33, 6, 2, torch.bfloat16), (1, 63, 8, 1, torch.float16), (1, 64, 32, 8, torch.bfloat16),
+    (2, 65, 10, 2, torch.bfloat16), (1, 97, 16, 1, torch.bfloat16), (1, 700, 24, 2, torch.float16),
+    (1, 20000, 4, 1, torch.bfloat16), (5, 2049, 7, 1, torch.bfloat16), (8, 3000, 32, 8, torch.float16),
+    (1, 40001, 4, 4, torch.bfloat16),
+])
+def test_exact_decode(B, L, H, KVH, dtype):
+    print(f"\n[case] exact decode B={B} L={L} H={H} KVH={KVH} {dtype}", flush=True)
+    g = torch.Generator().manual_seed(L)
+    q = torch.randn(B, H, 128, generator=g).mul(1.5).to("cuda", dtype)
+    k, v = (torch.randn(B, L + 5, KVH, 128, generator=g).to("cuda", dtype) for _ in range(2))
+    k[:, L:] = float("nan")  # past the valid length: never read into the result
+    v[:, L:] = float("nan")
+    _check_decode(ExactDecodeBackend().decode(q, k, v, L), _ref_decode(q, k, v, L), v[:, :L], dtype)
+
+
+def test_exact_decode_growing_scores_and_strides():
+    """Scores growing with the position (the maximum moves every step) over
+    caches that are slices of one tensor."""
+    print("\n[case] exact decode, growing scores, strided caches", flush=True)
+    g = torch.Generator().manual_seed(5)
+    L = 500
+    kv = torch.randn(2, L, 4, 128, generator=g)
+    kv[:, :, :2] = 0.1 * kv[:, :, :2] + torch.arange(L).view(1, L, 1, 1) * 0.02
+    kv = kv.to("cuda", torch.bfloat16)
+    k, v = kv[:, :, :2], kv[:, :, 2:]
+    q = torch.ones(2, 8, 128, device="cuda", dtype=torch.bfloat16)
+    ref = _ref_decode(q, k, v, L)
+    out = ExactDecodeBackend().decode(q, k, v, L)
+    assert ((out.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-3 * v.double().abs().max()).all()
