@@ -261,6 +261,9 @@ int santa_prop_decode_paged(const void* q, const void* K_pages, const void* V_pa
  * k_cache[b, pos] and v heads copied into v_cache[b, pos] of caches
  * [B, storage, KVH, D]; RoPE in the rotate-half convention with cos, sin
  * [D] and bf16 rounding of each product and of the sum.
+ * santa_rt_rope_write_rows: santa_rt_rope_write for a prefill's P positions
+ * pos .. pos + P - 1: qkv [B, P, H + 2 KVH, D], cos, sin [P, D], q_out
+ * [B, P, H, D]; D a multiple of 16, every tensor 16-byte aligned.
  * santa_rt_silu_mul: out [rows, inter] = bf16(bf16(silu(gate)) * up), gate
  * and up the two halves of gu [rows, 2 inter].
  * santa_rt_linear: the decode step's weight products (the HF layers'
@@ -270,6 +273,8 @@ int santa_prop_decode_paged(const void* q, const void* K_pages, const void* V_pa
  * aligned.  swiglu != 0: w is [2N, K] (gate rows, then up rows) and
  * y [M, N] = bf16(bf16(silu(bf16(g))) * bf16(u)), silu_mul of the product.
  * The weights are read once at the HBM bound.
+ * santa_rt_linear_f32: santa_rt_linear's product with its float32 sums as the
+ * output, y [M, N] float32 (the logits of the head).
  * santa_rt_linear_rope: the fused q/k/v projection of rows x [M, K] by
  * w [(H + 2 KVH) D, K] (head by head) with santa_rt_rope_write's epilogue
  * applied to the bf16 products: q heads rotated into q_out [M, H, D], k heads
@@ -300,8 +305,12 @@ int santa_rt_add_rms_norm(void* h, const void* a, const void* w, void* x, int ro
                           hipStream_t stream);
 int santa_rt_rope_write(const void* qkv, const void* cos_, const void* sin_, void* q_out, void* k_cache, void* v_cache,
                         int B, int H, int KVH, int D, long long storage, int pos, hipStream_t stream);
+int santa_rt_rope_write_rows(const void* qkv, const void* cos_, const void* sin_, void* q_out, void* k_cache,
+                             void* v_cache, int B, int P, int H, int KVH, int D, long long storage, int pos,
+                             hipStream_t stream);
 int santa_rt_silu_mul(const void* gu, void* out, int rows, int inter, hipStream_t stream);
 int santa_rt_linear(const void* x, const void* w, void* y, int M, int N, int K, int swiglu, hipStream_t stream);
+int santa_rt_linear_f32(const void* x, const void* w, float* y, int M, int N, int K, hipStream_t stream);
 int santa_rt_linear_rope(const void* x, const void* w, int M, int K, const void* cos_, const void* sin_, void* q_out,
                          void* k_cache, void* v_cache, int H, int KVH, int D, long long storage, int pos,
                          hipStream_t stream);

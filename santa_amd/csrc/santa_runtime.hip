@@ -167,6 +167,58 @@ __global__ __launch_bounds__(256) void rope_write_kernel(const uint16_t* __restr
   }
 }
 
+// The same for P positions from pos on (qkv [B, P, H + 2 KVH, D], cos and sin
+// [P, D], q_out [B, P, H, D]), D a multiple of 16 and every tensor 16-byte
+// aligned: a thread takes dims d .. d + 7 and d + D/2 .. d + D/2 + 7 of one
+// head, the two pieces rotate-half combines, as 16-byte vectors.  Bound by
+// reading qkv and writing q, k and v once; same roundings, same bits.
+__global__ __launch_bounds__(256) void rope_write_vec_kernel(const uint16_t* __restrict__ qkv,
+                                                             const uint16_t* __restrict__ cos_,
+                                                             const uint16_t* __restrict__ sin_,
+                                                             uint16_t* __restrict__ q_out,
+                                                             uint16_t* __restrict__ k_cache,
+                                                             uint16_t* __restrict__ v_cache, int P, int H, int KVH,
+                                                             int D, long long storage, int pos, uint32_t total) {
+  typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));
+  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+  if (i >= total) return;
+  const uint32_t per = static_cast<uint32_t>(D) / 16;  // threads per head
+  const uint32_t heads = static_cast<uint32_t>(H + 2 * KVH);
+  const int d = 8 * static_cast<int>(i % per);
+  const int hh = static_cast<int>(i / per % heads);
+  const uint32_t row = i / per / heads;  // b * P + p
+  const int b = static_cast<int>(row / static_cast<uint32_t>(P)), p = static_cast<int>(row % static_cast<uint32_t>(P));
+  const int half = D / 2;
+  const uint16_t* src = qkv + (static_cast<size_t>(row) * heads + hh) * D + d;
+  u32x4v x0 = *reinterpret_cast<const u32x4v*>(src), x1 = *reinterpret_cast<const u32x4v*>(src + half);
+  uint16_t* dst;
+  if (hh < H) {
+    dst = q_out + (static_cast<size_t>(row) * H + hh) * D + d;
+  } else {
+    const bool is_k = hh < H + KVH;
+    dst = (is_k ? k_cache : v_cache) +
+          ((static_cast<size_t>(b) * storage + pos + p) * KVH + (is_k ? hh - H : hh - H - KVH)) * D + d;
+  }
+  if (hh < H + KVH) {
+    const size_t cs = static_cast<size_t>(p) * D + d;
+    const u32x4v c0 = *reinterpret_cast<const u32x4v*>(cos_ + cs), c1 = *reinterpret_cast<const u32x4v*>(cos_ + cs + half);
+    const u32x4v s0 = *reinterpret_cast<const u32x4v*>(sin_ + cs), s1 = *reinterpret_cast<const u32x4v*>(sin_ + cs + half);
+    auto rot = [](float a, float c, float ra, float s) {
+      return static_cast<uint32_t>(to_bf(bf(to_bf(a * c)) + bf(to_bf(ra * s))));
+    };
+    auto lo = [](uint32_t w) { return __uint_as_float(w << 16); };
+    auto hi = [](uint32_t w) { return __uint_as_float(w & 0xffff0000u); };
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const uint32_t a = x0[k], e = x1[k];
+      x0[k] = rot(lo(a), lo(c0[k]), -lo(e), lo(s0[k])) | (rot(hi(a), hi(c0[k]), -hi(e), hi(s0[k])) << 16);
+      x1[k] = rot(lo(e), lo(c1[k]), lo(a), lo(s1[k])) | (rot(hi(e), hi(c1[k]), hi(a), hi(s1[k])) << 16);
+    }
+  }
+  *reinterpret_cast<u32x4v*>(dst) = x0;
+  *reinterpret_cast<u32x4v*>(dst + half) = x1;
+}
+
 // out = bf16(bf16(silu(gate)) * up), gate = gu[:, :inter], up = gu[:, inter:];
 // silu in float32, x / (1 + exp(-x)), as torch evaluates it for bf16.
 __global__ __launch_bounds__(256) void silu_mul_kernel(const uint16_t* __restrict__ gu, uint16_t* __restrict__ out,
@@ -180,6 +232,29 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const uint16_t* __restric
   const float u = bf(gu[r * 2 * inter + inter + c]);
   const float s = bf(to_bf(g / (1.0f + expf(-g))));
   out[i] = to_bf(s * u);
+}
+
+// The same for rows of 16-byte vectors (inter a multiple of 8, aligned): eight
+// values per thread and 32-bit indices, so many rows run at the memory rate
+// (the form above spends a 64-bit division per value).  Same bits.
+__global__ __launch_bounds__(256) void silu_mul_vec_kernel(const uint16_t* __restrict__ gu,
+                                                           uint16_t* __restrict__ out, uint32_t nv, uint32_t total) {
+  typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));
+  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+  if (i >= total) return;
+  const size_t r = i / nv;
+  const uint32_t c = i - static_cast<uint32_t>(r) * nv;
+  const u32x4v g = reinterpret_cast<const u32x4v*>(gu)[2 * r * nv + c];
+  const u32x4v u = reinterpret_cast<const u32x4v*>(gu)[(2 * r + 1) * nv + c];
+  auto one = [](float gf, float uf) {
+    return static_cast<uint32_t>(to_bf(bf(to_bf(gf / (1.0f + expf(-gf)))) * uf));
+  };
+  u32x4v o;
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    o[k] = one(__uint_as_float(g[k] << 16), __uint_as_float(u[k] << 16)) |
+           (one(__uint_as_float(g[k] & 0xffff0000u), __uint_as_float(u[k] & 0xffff0000u)) << 16);
+  reinterpret_cast<u32x4v*>(out)[i] = o;
 }
 
 // ------------------------------------------------------------------ linear
@@ -203,7 +278,9 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const uint16_t* __restric
 // RoPE combines, and the output goes where rope_write_kernel puts it (q
 // rotated to q_out, k rotated and v as is to the caches at pos), in its
 // roundings applied to the bf16 products; y is not written.
-constexpr int kLinPlain = 0, kLinSwiglu = 1, kLinRope = 2;
+// kLinF32: y is float32, the sums as they are (the head: its logits are wanted
+// in float32, and a bf16 y cost another pass and launch to widen it).
+constexpr int kLinPlain = 0, kLinSwiglu = 1, kLinRope = 2, kLinF32 = 3;
 struct RopeOut {
   const uint16_t* cos;
   const uint16_t* sin;
@@ -376,7 +453,13 @@ __global__ __launch_bounds__(kLinThreads, 1) void linear_kernel(const uint16_t* 
         }
       } else {
         const int r = (idx & 1) ? r1 : r0;
-        if (lead && m < M && r < N) y[static_cast<size_t>(m) * N + r] = to_bf(acc[0]);
+        if (lead && m < M && r < N) {
+          if constexpr (MODE == kLinF32) {
+            reinterpret_cast<float*>(y)[static_cast<size_t>(m) * N + r] = acc[0];
+          } else {
+            y[static_cast<size_t>(m) * N + r] = to_bf(acc[0]);
+          }
+        }
       }
       acc = accv_t{};
     }
@@ -524,6 +607,29 @@ extern "C" int santa_rt_rope_write(const void* qkv, const void* cos_, const void
   return clear_error();
 }
 
+extern "C" int santa_rt_rope_write_rows(const void* qkv, const void* cos_, const void* sin_, void* q_out,
+                                        void* k_cache, void* v_cache, int B, int P, int H, int KVH, int D,
+                                        long long storage, int pos, hipStream_t stream) {
+  if (!qkv || !cos_ || !sin_ || !q_out || !k_cache || !v_cache || B <= 0 || P <= 0 || H <= 0 || KVH <= 0 || D <= 0 ||
+      pos < 0 || static_cast<long long>(pos) + P > storage)
+    return set_error(SANTA_ERR_INVALID, "bad rope_write_rows arguments");
+  const long long total = static_cast<long long>(B) * P * (static_cast<long long>(H) + 2LL * KVH) * (D / 16);
+  if (D % 16 != 0 || total >= 0x7fffff00LL ||
+      (reinterpret_cast<uintptr_t>(qkv) | reinterpret_cast<uintptr_t>(cos_) | reinterpret_cast<uintptr_t>(sin_) |
+       reinterpret_cast<uintptr_t>(q_out) | reinterpret_cast<uintptr_t>(k_cache) |
+       reinterpret_cast<uintptr_t>(v_cache)) % 16 != 0)
+    return set_error(SANTA_ERR_UNSUPPORTED, "rope_write_rows: D must be a multiple of 16, the tensors 16-byte aligned "
+                                            "and fewer than 2^31 vectors");
+  hipLaunchKernelGGL(rt::rope_write_vec_kernel, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0, stream,
+                     static_cast<const uint16_t*>(qkv), static_cast<const uint16_t*>(cos_),
+                     static_cast<const uint16_t*>(sin_), static_cast<uint16_t*>(q_out),
+                     static_cast<uint16_t*>(k_cache), static_cast<uint16_t*>(v_cache), P, H, KVH, D, storage, pos,
+                     static_cast<uint32_t>(total));
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return set_error(SANTA_ERR_HIP, "rope_write_rows launch failed: %s", hipGetErrorString(e));
+  return clear_error();
+}
+
 namespace {
 // The shape checks and launch shared by the santa_rt_linear entry points
 // (rows: the weight's row count, N the output width the kernel indexes).
@@ -538,7 +644,7 @@ int launch_linear(int mode, const void* x, const void* w, void* y, int M, int N,
     return set_error(SANTA_ERR_INVALID, "linear: M x K too large for the staged rows (M rounded up to 1, 2, 4 or 8, "
                                         "times K rounded up to 2048, at most 65536)");
   if (static_cast<long long>(rows) * K * 2 > 0x7fffffffffffLL) return set_error(SANTA_ERR_INVALID, "linear: weight too large");
-  const int nbatch = mode == rt::kLinPlain ? (N + 1) / 2 : mode == rt::kLinSwiglu ? N : N / 2;
+  const int nbatch = mode == rt::kLinSwiglu ? N : mode == rt::kLinRope ? N / 2 : (N + 1) / 2;
   // the CU count of the current device, queried on each call (cheap next to
   // a weight-streaming kernel, and free of shared state between host threads)
   int dev = 0, cus = 256;
@@ -557,6 +663,9 @@ int launch_linear(int mode, const void* x, const void* w, void* y, int M, int N,
                        wp, yp, M, N, K, kp, nbatch, ro);                                                          \
   else if (mode == rt::kLinRope)                                                                                  \
     hipLaunchKernelGGL((rt::linear_kernel<MPV, rt::kLinRope>), dim3(grid), dim3(rt::kLinThreads), 0, stream, xp,   \
+                       wp, yp, M, N, K, kp, nbatch, ro);                                                          \
+  else if (mode == rt::kLinF32)                                                                                   \
+    hipLaunchKernelGGL((rt::linear_kernel<MPV, rt::kLinF32>), dim3(grid), dim3(rt::kLinThreads), 0, stream, xp,    \
                        wp, yp, M, N, K, kp, nbatch, ro);                                                          \
   else                                                                                                            \
     hipLaunchKernelGGL((rt::linear_kernel<MPV, rt::kLinPlain>), dim3(grid), dim3(rt::kLinThreads), 0, stream, xp,  \
@@ -579,6 +688,12 @@ extern "C" int santa_rt_linear(const void* x, const void* w, void* y, int M, int
   if (!y) return set_error(SANTA_ERR_INVALID, "bad linear arguments (null output)");
   const rt::RopeOut none{nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, 2, 0, 0};
   return launch_linear(swiglu ? rt::kLinSwiglu : rt::kLinPlain, x, w, y, M, N, K, swiglu ? 2 * N : N, none, stream);
+}
+
+extern "C" int santa_rt_linear_f32(const void* x, const void* w, float* y, int M, int N, int K, hipStream_t stream) {
+  if (!y) return set_error(SANTA_ERR_INVALID, "bad linear arguments (null output)");
+  const rt::RopeOut none{nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, 2, 0, 0};
+  return launch_linear(rt::kLinF32, x, w, y, M, N, K, N, none, stream);
 }
 
 extern "C" int santa_rt_linear_rope(const void* x, const void* w, int M, int K, const void* cos_, const void* sin_,
@@ -609,6 +724,16 @@ extern "C" int santa_rt_silu_mul(const void* gu, void* out, int rows, int inter,
   if (!gu || !out || rows < 0 || inter <= 0) return set_error(SANTA_ERR_INVALID, "bad silu_mul arguments");
   if (rows == 0) return clear_error();
   const long long total = static_cast<long long>(rows) * inter;
+  if (inter % 8 == 0 && total / 8 < 0x7fffff00LL &&
+      (reinterpret_cast<uintptr_t>(gu) | reinterpret_cast<uintptr_t>(out)) % 16 == 0) {
+    const uint32_t vecs = static_cast<uint32_t>(total / 8);
+    hipLaunchKernelGGL(rt::silu_mul_vec_kernel, dim3((vecs + 255) / 256), dim3(256), 0, stream,
+                       static_cast<const uint16_t*>(gu), static_cast<uint16_t*>(out), static_cast<uint32_t>(inter / 8),
+                       vecs);
+    const hipError_t ev = hipGetLastError();
+    if (ev != hipSuccess) return set_error(SANTA_ERR_HIP, "silu_mul launch failed: %s", hipGetErrorString(ev));
+    return clear_error();
+  }
   const unsigned grid = static_cast<unsigned>((total + 255) / 256);
   hipLaunchKernelGGL(rt::silu_mul_kernel, dim3(grid), dim3(256), 0, stream, static_cast<const uint16_t*>(gu),
                      static_cast<uint16_t*>(out), rows, inter);

@@ -82,9 +82,12 @@ class _FusedOps:
                                                                          ctypes.c_void_p]
             L.santa_rt_rope_write.argtypes = [ctypes.c_void_p] * 6 + [ctypes.c_int] * 4 + [
                 ctypes.c_longlong, ctypes.c_int, ctypes.c_void_p]
+            L.santa_rt_rope_write_rows.argtypes = [ctypes.c_void_p] * 6 + [ctypes.c_int] * 5 + [
+                ctypes.c_longlong, ctypes.c_int, ctypes.c_void_p]
             L.santa_rt_silu_mul.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_int,
                                             ctypes.c_void_p]
             L.santa_rt_linear.argtypes = [ctypes.c_void_p] * 3 + [ctypes.c_int] * 4 + [ctypes.c_void_p]
+            L.santa_rt_linear_f32.argtypes = [ctypes.c_void_p] * 3 + [ctypes.c_int] * 3 + [ctypes.c_void_p]
             L.santa_rt_linear_rope.argtypes = [ctypes.c_void_p] * 2 + [ctypes.c_int] * 2 + [ctypes.c_void_p] * 5 + [
                 ctypes.c_int] * 3 + [ctypes.c_longlong, ctypes.c_int, ctypes.c_void_p]
             L.santa_rt_argmax.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p]
@@ -129,6 +132,19 @@ class _FusedOps:
                                                  kc.shape[1], pos, cls._stream(qkv)))
         return q
 
+    @classmethod
+    def rope_write_rows(cls, qkv: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, k_cache: torch.Tensor,
+                        v_cache: torch.Tensor, heads: int, kv_heads: int, head_dim: int) -> torch.Tensor:
+        """rope_write for the positions 0 .. P-1 of a prefill: qkv [B, P, ...],
+        cos and sin [P, head_dim]; q rotated ([B, P, H, D]) returned."""
+        assert qkv.is_contiguous() and cos.is_contiguous() and sin.is_contiguous()
+        B, P = qkv.shape[:2]
+        q = torch.empty(B, P, heads, head_dim, dtype=qkv.dtype, device=qkv.device)
+        cls._check(cls.lib().santa_rt_rope_write_rows(qkv.data_ptr(), cos.data_ptr(), sin.data_ptr(), q.data_ptr(),
+                                                      k_cache.data_ptr(), v_cache.data_ptr(), B, P, heads, kv_heads,
+                                                      head_dim, k_cache.shape[1], 0, cls._stream(qkv)))
+        return q
+
     @staticmethod
     def linear_fits(rows: int, K: int) -> bool:
         """Whether santa_rt_linear takes x [rows, K]: rows <= 8, K a multiple
@@ -152,6 +168,19 @@ class _FusedOps:
         y = torch.empty(*x.shape[:-1], N, dtype=x.dtype, device=x.device)
         cls._check(cls.lib().santa_rt_linear(x.data_ptr(), w.data_ptr(), y.data_ptr(), rows, N, K, int(swiglu),
                                              cls._stream(x)))
+        return y
+
+    @classmethod
+    def logits(cls, x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+        """x @ w.T in float32 for few rows of x (santa_rt_linear_f32: the
+        float32 sums; F.linear widened where the shape does not fit it)."""
+        rows, K = x.shape
+        if not (cls.linear_fits(rows, K) and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
+                and x.is_contiguous() and w.is_contiguous() and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0):
+            return F.linear(x, w).float()
+        y = torch.empty(rows, w.shape[0], dtype=torch.float32, device=x.device)
+        cls._check(cls.lib().santa_rt_linear_f32(x.data_ptr(), w.data_ptr(), y.data_ptr(), rows, w.shape[0], K,
+                                                 cls._stream(x)))
         return y
 
     @classmethod
@@ -422,6 +451,8 @@ class RandomLlama:
         pos = torch.arange(P, device=self.device)
         cos, sin = _rope_cos_sin(pos, D, s.rope_theta, self.dtype)  # [P, D]
         h = self.embed[tokens]  # [B, P, hidden]
+        if mlp_chunk > 0 and attn_chunk > 0 and self._fused_prefill_takes(h, cache):
+            return self._prefill_fused(h, cos, sin, cache, mlp_chunk, attn_chunk)
         for li, L in enumerate(self.layers):
             x = _rms_norm(h, L["ln1"], s.rms_eps)
             q, k, v = self._qkv(L, x)
@@ -439,6 +470,46 @@ class RandomLlama:
                 hc += self._mlp(L, _rms_norm(hc, L["ln2"], s.rms_eps))
         last = _rms_norm(h[:, -1], self.norm, s.rms_eps)
         return F.linear(last, self.lm_head).float()
+
+    def _fused_prefill_takes(self, h: torch.Tensor, cache: NHDCache) -> bool:
+        """Whether the prefill of h [B, P, hidden] runs its elementwise work as
+        the library's kernels: a bf16 model and caches on one GPU, laid out as
+        the kernels address them (16-byte rows)."""
+        s = self.shape
+        B, P = h.shape[:2]
+        shape = (B, cache.storage, s.kv_heads, s.head_dim)
+        return (h.is_cuda and h.dtype == torch.bfloat16 and P <= cache.storage and B * P > 0 and s.head_dim % 16 == 0
+                and s.intermediate % 8 == 0 and s.hidden % 8 == 0
+                and B * P * (s.heads + 2 * s.kv_heads) * s.head_dim < 1 << 34
+                and all(t.shape == shape and t.dtype == h.dtype and t.device == h.device and t.is_contiguous()
+                        and t.data_ptr() % 16 == 0 for t in cache.k + cache.v)
+                and all(w.dtype == h.dtype and w.is_contiguous() for L in self.layers for w in (L["ln1"], L["ln2"]))
+                and self.norm.dtype == h.dtype and self.norm.is_contiguous() and _plain(h))
+
+    def _prefill_fused(self, h, cos, sin, cache, mlp_chunk, attn_chunk):
+        """prefill on the GPU: the torch products with the fused residual add +
+        norm, RoPE with the cache writes, and SwiGLU between them, in the torch
+        expressions' bf16 roundings."""
+        s, D = self.shape, self.shape.head_dim
+        B, P = h.shape[:2]
+        h, cos, sin = h.contiguous(), cos.contiguous(), sin.contiguous()
+        x = _FusedOps.add_rms_norm(h, None, self.layers[0]["ln1"], s.rms_eps)
+        rows = mlp_chunk * B
+        for li, L in enumerate(self.layers):
+            q = _FusedOps.rope_write_rows(F.linear(x, L["wqkv"]), cos, sin, cache.k[li], cache.v[li], s.heads,
+                                          s.kv_heads, D)
+            a = causal_attention(q, cache.k[li][:, :P], cache.v[li][:, :P], chunk=attn_chunk)
+            o = F.linear(a.reshape(B, P, s.heads * D), L["wo"])
+            del q, a
+            x = _FusedOps.add_rms_norm(h, o, L["ln2"], s.rms_eps).view(B * P, -1)  # h += o
+            m = o.view(B * P, -1)
+            for c0 in range(0, B * P, rows):
+                gu = F.linear(x[c0:c0 + rows], L["wgu"])
+                torch.mm(_FusedOps.silu_mul(gu), L["wd"].t(), out=m[c0:c0 + rows])
+                del gu
+            nxt = self.layers[li + 1]["ln1"] if li + 1 < len(self.layers) else self.norm
+            x = _FusedOps.add_rms_norm(h, o, nxt, s.rms_eps)  # h += m, then the next layer's (or final) norm
+        return _FusedOps.logits(x.view(B, P, -1)[:, -1].contiguous(), self.lm_head)
 
     # ------------------------------------------------------------ decode
     @torch.inference_mode()
@@ -484,7 +555,7 @@ class RandomLlama:
             m = lin(lin(x, L["wgu"], swiglu=True), L["wd"])
             nxt = self.layers[li + 1]["ln1"] if li + 1 < len(self.layers) else self.norm
             x = _FusedOps.add_rms_norm(h, m, nxt, s.rms_eps)  # h += m, then the next layer's (or final) norm
-        return lin(x, self.lm_head).float()
+        return _FusedOps.logits(x, self.lm_head)
 
 
 @torch.inference_mode()

@@ -41,6 +41,27 @@ def test_exact_decode_matches_recomputation():
         assert err <= 0.05 * scale, (j, err, scale)
 
 
+@pytest.mark.parametrize("B,P,mlp_chunk", [(1, 1, 8192), (2, 97, 40), (1, 300, 128)])
+def test_fused_prefill_matches_torch_expressions(B, P, mlp_chunk, monkeypatch):
+    """The prefill on the library's kernels against the torch expressions: the
+    same roundings up to the order of float32 sums, so logits and caches agree
+    to a few bf16 units (2^-8 each) of their scale through two layers."""
+    print(f"\n[case] fused prefill B={B} P={P} mlp_chunk={mlp_chunk}", flush=True)
+    dev = torch.device("cuda:0")
+    model = RandomLlama(SMALL, seed=7, std=0.05, device=dev)
+    toks = torch.randint(0, SMALL.vocab, (B, P), generator=torch.Generator().manual_seed(P)).to(dev)
+    fused, plain = (NHDCache(SMALL, B, P + 2, torch.bfloat16, dev) for _ in range(2))
+    got = model.prefill(toks, fused, mlp_chunk=mlp_chunk, attn_chunk=64)
+    monkeypatch.setattr(RandomLlama, "_fused_prefill_takes", lambda self, h, cache: False)
+    want = model.prefill(toks, plain, mlp_chunk=mlp_chunk, attn_chunk=64)
+    torch.cuda.synchronize()
+    for a, b in [(got, want)] + list(zip(fused.k + fused.v, plain.k + plain.v)):
+        a, b = a.float(), b.float()
+        assert (a - b).abs().max() <= 8 * 2.0 ** -8 * b.abs().max(), ((a - b).abs().max(), b.abs().max())
+        assert (a - b).norm() <= 2.0 ** -6 * b.norm()
+    assert not fused.k[0][:, P:].any() and not fused.v[1][:, P:].any()
+
+
 def test_santa_backends_in_the_decode_loop():
     print("\n[case] runtime santa_flash (large S) and santa_prop vs exact, P=700 B=2", flush=True)
     model, toks, cache, logits = _setup()

@@ -64,6 +64,49 @@ def test_add_rms_norm(rows, hidden):
     _ulp_close(x0, _rms_norm(h, w, 1e-5), 2)
 
 
+@pytest.mark.parametrize("B,P,H,KVH,D", [(1, 1, 32, 8, 128), (2, 33, 7, 1, 128), (3, 100, 4, 2, 64), (1, 130, 5, 5, 16)])
+def test_rope_write_rows(B, P, H, KVH, D):
+    """A prefill's positions: bit for bit the torch expressions, rows of the
+    caches past the prompt untouched."""
+    print(f"\n[case] rope_write_rows B={B} P={P} H={H} KVH={KVH} D={D}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(P)
+    qkv = torch.randn(B, P, (H + 2 * KVH) * D, device=DEV, generator=g).to(torch.bfloat16)
+    kc, vc = (torch.randn(B, P + 3, KVH, D, device=DEV, generator=g).to(torch.bfloat16) for _ in range(2))
+    want_k, want_v = kc.clone(), vc.clone()
+    cos, sin = _rope_cos_sin(torch.arange(P, device=DEV), D, 500000.0, torch.bfloat16)
+    q = _FusedOps.rope_write_rows(qkv, cos.contiguous(), sin.contiguous(), kc, vc, H, KVH, D)
+    torch.cuda.synchronize()
+    rq, rk, rv = qkv.view(B, P, -1, D).split([H, KVH, KVH], dim=2)
+    want_k[:, :P] = _apply_rope(rk, cos[:, None], sin[:, None])
+    want_v[:, :P] = rv
+    for got, want in ((q, _apply_rope(rq, cos[:, None], sin[:, None])), (kc, want_k), (vc, want_v)):
+        assert torch.equal(got.view(torch.int16), want.contiguous().view(torch.int16))
+
+
+@pytest.mark.parametrize("rows,K,N", [(1, 2048, 7), (3, 4096, 1001), (4, 72, 128), (8, 4104, 64), (9, 256, 33)])
+def test_logits(rows, K, N):
+    """The float32 product: its bf16 rounding is santa_rt_linear's output bit
+    for bit (same sums); 9 rows take F.linear."""
+    print(f"\n[case] logits rows={rows} K={K} N={N}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(K + N)
+    x = torch.randn(rows, K, device=DEV, generator=g).to(torch.bfloat16)
+    w = torch.randn(N, K, device=DEV, generator=g).to(torch.bfloat16)
+    y = _FusedOps.logits(x, w)
+    torch.cuda.synchronize()
+    assert y.dtype == torch.float32 and torch.equal(y.to(torch.bfloat16), _FusedOps.linear(x, w))
+
+
+@pytest.mark.parametrize("rows,inter", [(1, 8), (5, 1000), (3, 1001), (300, 1032)])
+def test_silu_mul_forms(rows, inter):
+    """The vector form and, for widths that are not a multiple of 8, the scalar one."""
+    print(f"\n[case] silu_mul rows={rows} inter={inter}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(rows + inter)
+    gu = (3.0 * torch.randn(rows, 2 * inter, device=DEV, generator=g)).to(torch.bfloat16)
+    out = _FusedOps.silu_mul(gu)
+    torch.cuda.synchronize()
+    _ulp_close(out, F.silu(gu[:, :inter]) * gu[:, inter:], 1)
+
+
 @pytest.mark.parametrize("B,H,KVH,pos", [(4, 32, 8, 37), (2, 64, 8, 0), (1, 16, 2, 99)])
 def test_rope_write(B, H, KVH, pos):
     D = 128
