@@ -176,12 +176,84 @@ __device__ __forceinline__ int ragged_len(const int* seq_lens, int b, int max_ro
   return min(max(seq_lens[b], 1), max_rows);
 }
 
+// Inclusive sum of v over the wave's lanes in lane order.
+__device__ __forceinline__ int wave_scan_sum(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, true);  // lane - 1, - 2, - 4, - 8 inside each 16-lane row
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);  // rows 1, 3 take lane 15 / 47
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);  // then rows 2, 3 take lane 31
+  return v;
+}
+
+// Chunks of the 64 sequences g0 + lane of a ragged grid, one per lane (0 chunks
+// past B): their tiles, tiles per chunk, chunks, and the chunks of the lanes
+// up to and including this one.  One pass of vector arithmetic for the whole
+// batch, where a walk over the sequences cost each workgroup B divisions in a
+// row before its first load.
+struct RaggedLane {
+  int len, tiles, cs, chunks, incl;
+};
+__device__ __forceinline__ RaggedLane ragged_lane(const int* seq_lens, int g0, int B, int max_rows, int BN, int cs,
+                                                  const DenseCut& dense) {
+  const int lane = static_cast<int>(threadIdx.x) & 63;
+  const bool in = g0 + lane < B;
+  RaggedLane r;
+  r.len = in ? ragged_len(seq_lens, g0 + lane, max_rows) : 0;
+  r.tiles = static_cast<int>(static_cast<uint32_t>(r.len + BN - 1) / static_cast<uint32_t>(BN));
+  r.cs = cs;
+  r.chunks = static_cast<int>(static_cast<uint32_t>(r.tiles + cs - 1) / static_cast<uint32_t>(cs));
+  // S * gh >= 64 tiles: the tiles may carry 64 samples (both sides below 2^31)
+  const bool short_seq = r.tiles > 1 && static_cast<uint32_t>(dense.S) * dense.gh >= 64u * static_cast<uint32_t>(r.tiles);
+  if (dense.limit > 0 && __ballot(short_seq) != 0) {
+    int n = r.chunks, c = cs;
+    const uint32_t w = static_cast<uint32_t>(dense.S) / static_cast<uint32_t>(max(r.tiles, 1)) * dense.gh;
+    if (short_seq && w >= 64) {
+      const float want = ceilf(static_cast<float>(r.tiles) * (170.0f + static_cast<float>(w)) /
+                               (170.0f * static_cast<float>(cs)));
+      n = min(min(r.tiles, n + kDenseChunks), max(n, static_cast<int>(fminf(want, 1048576.0f))));
+      c = static_cast<int>(static_cast<uint32_t>(r.tiles + n - 1) / static_cast<uint32_t>(n));
+      n = static_cast<int>(static_cast<uint32_t>(r.tiles + c - 1) / static_cast<uint32_t>(c));
+    }
+    const int incl = wave_scan_sum(n);
+    if (__builtin_amdgcn_readlane(incl, 63) <= dense.limit) {
+      r.cs = c;
+      r.chunks = n;
+    }
+  }
+  r.incl = wave_scan_sum(r.chunks);
+  return r;
+}
+
+// Chunks of the sequences before b, and b's tiles and tiles per chunk.
+struct RaggedSeq {
+  int first, tiles, cs;
+};
+__device__ __forceinline__ RaggedSeq ragged_seq(const int* seq_lens, int b, int B, int max_rows, int BN, int cs,
+                                                const DenseCut& dense) {
+  RaggedSeq s{0, 0, cs};
+  for (int g0 = 0; g0 <= b; g0 += 64) {
+    const RaggedLane r = ragged_lane(seq_lens, g0, B, max_rows, BN, cs, dense);
+    if (b < g0 + 64) {
+      s.first += __builtin_amdgcn_readlane(r.incl - r.chunks, b - g0);
+      s.tiles = __builtin_amdgcn_readlane(r.tiles, b - g0);
+      s.cs = __builtin_amdgcn_readlane(r.cs, b - g0);
+      break;
+    }
+    s.first += __builtin_amdgcn_readlane(r.incl, 63);
+  }
+  return s;
+}
+
 struct GridPos {
   int b, kv, chunk, len, n_tiles, wg_base;
+  int cs;  // tiles per chunk of this sequence
 };
 __device__ __forceinline__ GridPos grid_pos(int wg, const int* seq_lens, int B, int KVH, int BN, int L_valid, int T_c,
-                                            int cs, int cpg) {
+                                            int cs, int cpg, const DenseCut& dense = DenseCut{0, 0, 0}) {
   GridPos p;
+  p.cs = cs;
   if (!seq_lens) {
     p.kv = wg % KVH;
     p.chunk = (wg / KVH) % cpg;
@@ -191,28 +263,30 @@ __device__ __forceinline__ GridPos grid_pos(int wg, const int* seq_lens, int B, 
     p.wg_base = p.b * cpg * KVH;
     return p;
   }
-  int base = 0;
   p.b = -1;
   p.kv = 0;
   p.chunk = 0;
   p.len = 0;
   p.n_tiles = 0;
   p.wg_base = 0;
-  for (int bb = 0; bb < B; ++bb) {
-    const int len = ragged_len(seq_lens, bb, L_valid);
-    const int tiles = (len + BN - 1) / BN;
-    const int n = KVH * ((tiles + cs - 1) / cs);
-    if (wg < base + n) {
-      const int local = wg - base;
-      p.b = bb;
-      p.kv = local % KVH;
-      p.chunk = local / KVH;
-      p.len = len;
-      p.n_tiles = tiles;
-      p.wg_base = base;
+  const int item = wg / KVH;
+  int first = 0;
+  for (int g0 = 0; g0 < B; g0 += 64) {
+    const RaggedLane r = ragged_lane(seq_lens, g0, B, L_valid, BN, cs, dense);
+    const int total = __builtin_amdgcn_readlane(r.incl, 63);
+    if (item < first + total) {
+      const int l = __builtin_ctzll(__ballot(item < first + r.incl));
+      const int before = first + __builtin_amdgcn_readlane(r.incl - r.chunks, l);
+      p.b = g0 + l;
+      p.kv = wg - item * KVH;
+      p.chunk = item - before;
+      p.len = __builtin_amdgcn_readlane(r.len, l);
+      p.n_tiles = __builtin_amdgcn_readlane(r.tiles, l);
+      p.wg_base = before * KVH;
+      p.cs = __builtin_amdgcn_readlane(r.cs, l);
       break;
     }
-    base += n;
+    first += total;
   }
   return p;
 }

@@ -855,7 +855,7 @@ __global__ __launch_bounds__(ROWS ? 512 : kThreads, ROWS ? 1 : 2) void wave_kern
     int L_valid, int L_storage, int T_c, int cs, int cpg, float q_scale, int S_pt, uint64_t seed,
     float* __restrict__ part, int* __restrict__ part_emit, const int* __restrict__ seq_lens, int B, long long S_total,
     float* __restrict__ dbg_m, float* __restrict__ dbg_ell, int16_t* __restrict__ dbg_counts,
-    uint16_t* __restrict__ u_stash, int stash_ld, PageTable pt, int stash_nt, int kv_div) {
+    uint16_t* __restrict__ u_stash, int stash_ld, PageTable pt, int stash_nt, int kv_div, DenseCut dense) {
   constexpr int BN = 256;
   constexpr int NHB = GH / 4;
   constexpr int LCAP = kWaveListCap;
@@ -870,7 +870,7 @@ __global__ __launch_bounds__(ROWS ? 512 : kThreads, ROWS ? 1 : 2) void wave_kern
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // ROWS workgroups enumerate (sequence, chunk) items (grid_pos with one
   // "head"); the KV head is the wave
-  const GridPos gp = grid_pos(wg, seq_lens, B, ROWS ? 1 : KVH, BN, L_valid, T_c, cs, cpg);
+  const GridPos gp = grid_pos(wg, seq_lens, B, ROWS ? 1 : KVH, BN, L_valid, T_c, cs, cpg, dense);
   const int kv = ROWS ? wave : gp.kv;
   const int b = gp.b < 0 ? 0 : gp.b;
   // heads per KV head: GH, except that santa_prop's pass 1 at GH 8 also takes
@@ -879,8 +879,8 @@ __global__ __launch_bounds__(ROWS ? 512 : kThreads, ROWS ? 1 : 2) void wave_kern
   const int gsz = (P1 && GH == 8) ? H / KVH : GH;
   const int h0 = kv * gsz;
   L_valid = gp.len;
-  const int t_begin = gp.chunk * cs;
-  const int t_end = (gp.b < 0) ? t_begin : min(gp.n_tiles, t_begin + cs);
+  const int t_begin = gp.chunk * gp.cs;
+  const int t_end = (gp.b < 0) ? t_begin : min(gp.n_tiles, t_begin + gp.cs);
   if (seq_lens)  // S_per_tile from this sequence's tile count (flash/santa_cuda.cpp:204-208)
     S_pt = (S_total > 0) ? static_cast<int>(max(1LL, S_total / static_cast<long long>(max(gp.n_tiles, 1)))) : 0;
   const int t_first = ROWS ? t_begin : t_begin + wave;
@@ -1593,7 +1593,7 @@ __global__ __launch_bounds__(1024) void merge_kernel(const float* __restrict__ p
                                                      int H, int KVH, int cpg, int S_pt, uint16_t* __restrict__ out,
                                                      float* __restrict__ m_star, int* __restrict__ vrows,
                                                      const int* __restrict__ seq_lens, int BN, int cs, int max_len,
-                                                     int n_wg, long long S_total) {
+                                                     int n_wg, long long S_total, int B, DenseCut dense) {
   const int bh = static_cast<int>(blockIdx.x);
   const int b = bh / H;
   const int h = bh % H;
@@ -1606,9 +1606,10 @@ __global__ __launch_bounds__(1024) void merge_kernel(const float* __restrict__ p
   // chunk c of (b, kv) was workgroup base_b + c * KVH + kv
   int base = b * cpg * KVH;
   if (seq_lens) {
-    base = 0;
-    for (int bb = 0; bb < b; ++bb) base += KVH * (((ragged_len(seq_lens, bb, max_len) + BN - 1) / BN + cs - 1) / cs);
-    const int tiles = (ragged_len(seq_lens, b, max_len) + BN - 1) / BN;
+    const RaggedSeq rs = ragged_seq(seq_lens, b, B, max_len, BN, cs, dense);
+    base = KVH * rs.first;
+    const int tiles = rs.tiles;
+    cs = rs.cs;
     cpg = (tiles + cs - 1) / cs;
     cpg = max(0, min(cpg, (n_wg - base - kv + KVH - 1) / KVH));  // only launched workgroups wrote partials
     S_pt = (S_total > 0) ? static_cast<int>(max(1LL, S_total / static_cast<long long>(tiles))) : 0;
@@ -1704,7 +1705,7 @@ __global__ __launch_bounds__(64) void merge_wave_kernel(const float* __restrict_
                                                         int S_pt, uint16_t* __restrict__ out,
                                                         float* __restrict__ m_star, int* __restrict__ vrows,
                                                         const int* __restrict__ seq_lens, int BN, int cs,
-                                                        int max_len, int n_wg, long long S_total) {
+                                                        int max_len, int n_wg, long long S_total, int B, DenseCut dense) {
   const int bh = static_cast<int>(blockIdx.x);
   const int b = bh / H;
   const int h = bh % H;
@@ -1714,9 +1715,10 @@ __global__ __launch_bounds__(64) void merge_wave_kernel(const float* __restrict_
   // chunk c of (b, kv) was workgroup base_b + c * KVH + kv
   int base = b * cpg * KVH;
   if (seq_lens) {
-    base = 0;
-    for (int bb = 0; bb < b; ++bb) base += KVH * (((ragged_len(seq_lens, bb, max_len) + BN - 1) / BN + cs - 1) / cs);
-    const int tiles = (ragged_len(seq_lens, b, max_len) + BN - 1) / BN;
+    const RaggedSeq rs = ragged_seq(seq_lens, b, B, max_len, BN, cs, dense);
+    base = KVH * rs.first;
+    const int tiles = rs.tiles;
+    cs = rs.cs;
     cpg = (tiles + cs - 1) / cs;
     cpg = max(0, min(cpg, (n_wg - base - kv + KVH - 1) / KVH));  // only launched workgroups wrote partials
     S_pt = (S_total > 0) ? static_cast<int>(max(1LL, S_total / static_cast<long long>(tiles))) : 0;
@@ -1775,7 +1777,7 @@ __global__ __launch_bounds__(64 * NW) void merge_split_kernel(const float* __res
                                                               int cpg, int S_pt, uint16_t* __restrict__ out,
                                                               float* __restrict__ m_star, int* __restrict__ vrows,
                                                               const int* __restrict__ seq_lens, int BN, int cs,
-                                                              int max_len, int n_wg, long long S_total) {
+                                                              int max_len, int n_wg, long long S_total, int B, DenseCut dense) {
   constexpr int NB = 16;
   __shared__ float s_m[NW];
   __shared__ float s_z[NW];
@@ -1790,9 +1792,10 @@ __global__ __launch_bounds__(64 * NW) void merge_split_kernel(const float* __res
   const int wv = static_cast<int>(threadIdx.x) >> 6;
   int base = b * cpg * KVH;
   if (seq_lens) {
-    base = 0;
-    for (int bb = 0; bb < b; ++bb) base += KVH * (((ragged_len(seq_lens, bb, max_len) + BN - 1) / BN + cs - 1) / cs);
-    const int tiles = (ragged_len(seq_lens, b, max_len) + BN - 1) / BN;
+    const RaggedSeq rs = ragged_seq(seq_lens, b, B, max_len, BN, cs, dense);
+    base = KVH * rs.first;
+    const int tiles = rs.tiles;
+    cs = rs.cs;
     cpg = (tiles + cs - 1) / cs;
     cpg = max(0, min(cpg, (n_wg - base - kv + KVH - 1) / KVH));
     S_pt = (S_total > 0) ? static_cast<int>(max(1LL, S_total / static_cast<long long>(tiles))) : 0;
@@ -1880,6 +1883,7 @@ struct Args {
   int n_wg;             // grid size of the ragged form
   long long S_total;    // ragged flash: S, for each sequence's S_per_tile
   PageTable pt;         // paged K/V (pt.table set) or contiguous
+  DenseCut dense{0, 0, 0};  // ragged flash: finer chunks for densely sampled sequences
 };
 
 template <bool BF16, int GH, int BN, int MODE, bool PAGED>
@@ -1933,14 +1937,14 @@ static hipError_t launch_wave_t(const Args& a, float* dbg_m, float* dbg_ell, int
                          dim3(static_cast<unsigned>(64 * a.KVH)), 0, stream, static_cast<const uint16_t*>(a.q),
                          static_cast<const uint16_t*>(a.K), static_cast<const uint16_t*>(a.V), a.H, a.KVH, a.L_valid,
                          a.L_storage, a.T_c, a.cs, a.cpg, q_scale, a.S_pt, a.seed, a.part, a.part_emit, a.seq_lens,
-                         a.B, a.S_total, dbg_m, dbg_ell, dbg_counts, nullptr, 0, a.pt, 0, 1);
+                         a.B, a.S_total, dbg_m, dbg_ell, dbg_counts, nullptr, 0, a.pt, 0, 1, a.dense);
       return hipGetLastError();
     }
     hipLaunchKernelGGL((wave_kernel<BF16, GH, true>), dim3(grid), dim3(kThreads), 0, stream,
                        static_cast<const uint16_t*>(a.q), static_cast<const uint16_t*>(a.K),
                        static_cast<const uint16_t*>(a.V), a.H, a.KVH, a.L_valid, a.L_storage, a.T_c, a.cs, a.cpg,
                        q_scale, a.S_pt, a.seed, a.part, a.part_emit, a.seq_lens, a.B, a.S_total, dbg_m, dbg_ell,
-                       dbg_counts, nullptr, 0, a.pt, 0, 1);
+                       dbg_counts, nullptr, 0, a.pt, 0, 1, a.dense);
   } else if (rows_layout(a.KVH)) {
     // one workgroup of KVH waves per (sequence, chunk) item
     const unsigned rgrid = grid / static_cast<unsigned>(a.KVH);
@@ -1950,25 +1954,25 @@ static hipError_t launch_wave_t(const Args& a, float* dbg_m, float* dbg_ell, int
                          static_cast<const uint16_t*>(a.q), static_cast<const uint16_t*>(a.K),
                          static_cast<const uint16_t*>(a.V), a.H, a.KVH, a.L_valid, a.L_storage, a.T_c, a.cs, a.cpg,
                          q_scale, a.S_pt, a.seed, a.part, a.part_emit, a.seq_lens, a.B, a.S_total, nullptr,
-                         nullptr, nullptr, nullptr, 0, a.pt, 0, 1);
+                         nullptr, nullptr, nullptr, 0, a.pt, 0, 1, a.dense);
     else
       hipLaunchKernelGGL((wave_kernel<BF16, GH, false, false, false, true>), dim3(rgrid), block, 0, stream,
                          static_cast<const uint16_t*>(a.q), static_cast<const uint16_t*>(a.K),
                          static_cast<const uint16_t*>(a.V), a.H, a.KVH, a.L_valid, a.L_storage, a.T_c, a.cs, a.cpg,
                          q_scale, a.S_pt, a.seed, a.part, a.part_emit, a.seq_lens, a.B, a.S_total, nullptr,
-                         nullptr, nullptr, nullptr, 0, a.pt, 0, 1);
+                         nullptr, nullptr, nullptr, 0, a.pt, 0, 1, a.dense);
   } else if (a.pt.table) {
     hipLaunchKernelGGL((wave_kernel<BF16, GH, false, false, true>), dim3(grid), dim3(kThreads), 0, stream,
                        static_cast<const uint16_t*>(a.q), static_cast<const uint16_t*>(a.K),
                        static_cast<const uint16_t*>(a.V), a.H, a.KVH, a.L_valid, a.L_storage, a.T_c, a.cs, a.cpg,
                        q_scale, a.S_pt, a.seed, a.part, a.part_emit, a.seq_lens, a.B, a.S_total, nullptr,
-                       nullptr, nullptr, nullptr, 0, a.pt, 0, 1);
+                       nullptr, nullptr, nullptr, 0, a.pt, 0, 1, a.dense);
   } else {
     hipLaunchKernelGGL((wave_kernel<BF16, GH, false>), dim3(grid), dim3(kThreads), 0, stream,
                        static_cast<const uint16_t*>(a.q), static_cast<const uint16_t*>(a.K),
                        static_cast<const uint16_t*>(a.V), a.H, a.KVH, a.L_valid, a.L_storage, a.T_c, a.cs, a.cpg,
                        q_scale, a.S_pt, a.seed, a.part, a.part_emit, a.seq_lens, a.B, a.S_total, nullptr,
-                       nullptr, nullptr, nullptr, 0, a.pt, 0, 1);
+                       nullptr, nullptr, nullptr, 0, a.pt, 0, 1, a.dense);
   }
   return hipGetLastError();
 }
@@ -1985,14 +1989,23 @@ static hipError_t launch_wave(int dtype, int GH, const Args& a, float* dbg_m, fl
 }
 
 // The chunk-partial merge, one workgroup per (b, h); seq_lens selects the
-// ragged chunk layout (then bn, cs, max_len, n_wg and S_total describe it).
+// ragged chunk layout (then bn, cs, max_len, n_wg and S_total describe it, and
+// dense its finer cut sequences).
 static hipError_t launch_merge(const float* part, const int* pe, int dtype, int B, int H, int KVH, int cpg, int S_pt,
                                void* out, float* m_star, int* vrows, const int* seq_lens, int bn, int cs,
-                               int max_len, int n_wg, long long S_total, hipStream_t stream) {
+                               int max_len, int n_wg, long long S_total, hipStream_t stream,
+                               DenseCut dense = DenseCut{0, 0, 0}) {
   const int GH = H / KVH;
   const unsigned grid = static_cast<unsigned>(B) * static_cast<unsigned>(H);
   uint16_t* o = static_cast<uint16_t*>(out);
-  const int max_chunks = seq_lens ? ((max_len + bn - 1) / bn + cs - 1) / cs : cpg;
+  int max_chunks = cpg;
+  if (seq_lens) {
+    max_chunks = ((max_len + bn - 1) / bn + cs - 1) / cs;
+    if (dense.limit > 0) {  // a finer cut sequence holds at most S * gh / 64 tiles
+      const int widest = std::min(max_len / bn + 1, dense.S * dense.gh / 64);
+      max_chunks = std::max(max_chunks, std::min(widest, (widest + cs - 1) / cs + kDenseChunks));
+    }
+  }
   if (max_chunks <= 256) {
     // one wave per (b, h) up to 32 chunks, else 4, 8 or 16 waves of 16
     // chunks each, every load in one round trip (B = 1 at 32k, 64 chunks:
@@ -2000,10 +2013,10 @@ static hipError_t launch_merge(const float* part, const int* pe, int dtype, int 
     // took 20-26 us per call at B = 1, GH 8, 64k-96k tokens)
 #define SANTA_MERGE_WAVE(BF, G, NBC)                                                                          \
   hipLaunchKernelGGL((merge_wave_kernel<BF, G, NBC>), dim3(grid), dim3(64), 0, stream, part, pe, H, KVH, cpg, \
-                     S_pt, o, m_star, vrows, seq_lens, bn, cs, max_len, n_wg, S_total)
+                     S_pt, o, m_star, vrows, seq_lens, bn, cs, max_len, n_wg, S_total, B, dense)
 #define SANTA_MERGE_SPLIT(BF, G, NWC)                                                                       \
   hipLaunchKernelGGL((merge_split_kernel<BF, G, NWC>), dim3(grid), dim3(64 * NWC), 0, stream, part, pe, H, KVH, cpg, \
-                     S_pt, o, m_star, vrows, seq_lens, bn, cs, max_len, n_wg, S_total)
+                     S_pt, o, m_star, vrows, seq_lens, bn, cs, max_len, n_wg, S_total, B, dense)
 #define SANTA_MERGE_NB(BF, G)           \
   if (max_chunks <= 16)                 \
     SANTA_MERGE_WAVE(BF, G, 16);        \
@@ -2031,17 +2044,17 @@ static hipError_t launch_merge(const float* part, const int* pe, int dtype, int 
   if (dtype == SANTA_BF16) {
     if (GH == 4)
       hipLaunchKernelGGL((merge_kernel<true, 4>), dim3(grid), block, 0, stream, part, pe, H, KVH, cpg, S_pt, o,
-                         m_star, vrows, seq_lens, bn, cs, max_len, n_wg, S_total);
+                         m_star, vrows, seq_lens, bn, cs, max_len, n_wg, S_total, B, dense);
     else
       hipLaunchKernelGGL((merge_kernel<true, 8>), dim3(grid), block, 0, stream, part, pe, H, KVH, cpg, S_pt, o,
-                         m_star, vrows, seq_lens, bn, cs, max_len, n_wg, S_total);
+                         m_star, vrows, seq_lens, bn, cs, max_len, n_wg, S_total, B, dense);
   } else {
     if (GH == 4)
       hipLaunchKernelGGL((merge_kernel<false, 4>), dim3(grid), block, 0, stream, part, pe, H, KVH, cpg, S_pt, o,
-                         m_star, vrows, seq_lens, bn, cs, max_len, n_wg, S_total);
+                         m_star, vrows, seq_lens, bn, cs, max_len, n_wg, S_total, B, dense);
     else
       hipLaunchKernelGGL((merge_kernel<false, 8>), dim3(grid), block, 0, stream, part, pe, H, KVH, cpg, S_pt, o,
-                         m_star, vrows, seq_lens, bn, cs, max_len, n_wg, S_total);
+                         m_star, vrows, seq_lens, bn, cs, max_len, n_wg, S_total, B, dense);
   }
   return hipGetLastError();
 }
@@ -2229,7 +2242,8 @@ hipError_t launch_prop_pass1(const void* q, const void* K, int dtype, int B, int
   hipLaunchKernelGGL((wave_kernel<BF, G, false, true, PG, RW>), dim3(grid), block, 0, stream,                     \
                      static_cast<const uint16_t*>(a.q), static_cast<const uint16_t*>(a.K), nullptr, a.H, a.KVH,     \
                      a.L_valid, a.L_storage, a.T_c, a.cs, a.cpg, q_scale, 0, 0ULL, nullptr, nullptr, a.seq_lens,   \
-                     a.B, 0LL, m_tiles, ell_tiles, nullptr, u_stash, stash_ld, a.pt, stash_nt, kv_div)
+                     a.B, 0LL, m_tiles, ell_tiles, nullptr, u_stash, stash_ld, a.pt, stash_nt, kv_div, \
+                     DenseCut{0, 0, 0})
 #define SANTA_P1_GH(BF, PG, RW)    \
   do {                             \
     if (GH == 4)                   \
@@ -2595,6 +2609,7 @@ namespace {
 struct RaggedWs {
   size_t part, emit, total;
   int cs, n_wg;
+  bool dense;  // densely sampled sequences may get finer chunks (DenseCut)
 };
 // small: the tile kernel takes the pass (flash::small_pass), with the
 // four-wave plan
@@ -2611,16 +2626,16 @@ RaggedWs ragged_ws_layout(int B, int H, int KVH, long long total_tiles, int max_
   // 240.4 -> 131.8, B = 2 at 64k-128k 173.7 -> 89.4, B = 32 at 8k-32k 285.3
   // -> 247.4; but B = 12 at 1k-128k 325.2 -> 353.6, and at B = 40, 48 and 64
   // (a quarter of the round and more in partial chunks) 3-10 % slower.  The
-  // loss at B = 12 (GH 8: 450.1 -> 589.6 us) is a sequence shorter than one
-  // chunk (4 tiles against 12): it is one chunk, and S_per_tile = S / 4 puts
-  // all its S samples per head, S * GH row gathers per wave in dependent
-  // batches of 16, on one CU, where eight rounds split it in two.  The host
-  // does not know the shortest length (the call carries total_tiles and
-  // max_len), so the rule stands on the batches measured above.
+  // loss at B = 12 was a sequence shorter than one chunk (4 tiles against 12),
+  // all its samples on one CU; the rows layout now cuts such sequences finer
+  // (DenseCut), unless every sequence has the same tile count and
+  // the grid is the uniform one.
   const int rounds = (rows && 8LL * B * KVH <= flash::rows_per_round()) ? 1 : 8;
   flash::plan_ragged(B, KVH, total_tiles, max_tiles, &w.cs, &w.n_wg, rows ? flash::rows_per_round() : 0,
                      rows ? 1 : 4, rounds);
-  const size_t chunks = static_cast<size_t>(w.n_wg);
+  // densely sampled sequences are cut finer where the plan is one round
+  w.dense = rows && rounds == 1 && total_tiles != static_cast<long long>(B) * max_tiles;
+  const size_t chunks = w.dense ? std::max<size_t>(w.n_wg, KVH * (flash::rows_per_round() / KVH)) : w.n_wg;
   size_t off = 0;
   w.part = off;
   off = santa::align_up(off + chunks * (H / KVH) * flash::kPartStride * sizeof(float));
@@ -2666,11 +2681,18 @@ static int flash_decode_ragged(const void* q, const void* K, const void* V, int 
   int* pe = reinterpret_cast<int*>(base + w.emit);
   flash::Args a{q, K, V, B, H, KVH, max_len, L_storage, T_c, 0, seed, nullptr, nullptr, nullptr, nullptr, nullptr,
                 part, pe, w.cs, 0, nullptr, seq_lens, w.n_wg, static_cast<long long>(S), pt};
+  if (w.dense && block_n == 256 && S > 0) {
+    // the finer chunks all fit one round or are not cut, so the grid needs no
+    // more than the plan's workgroups or a round of them
+    const int round = flash::rows_per_round() / KVH;
+    a.dense = DenseCut{H / KVH, round, static_cast<int>(std::min<int64_t>(S, 1 << 20))};
+    a.n_wg = KVH * std::max(w.n_wg / KVH, round);
+  }
   hipError_t e = (block_n == 256 && !small) ? flash::launch_wave(dtype, H / KVH, a, nullptr, nullptr, nullptr, stream)
                                             : flash::launch_tiles<flash::kOnline>(dtype, H / KVH, block_n, a, stream);
   if (e != hipSuccess) return set_error(SANTA_ERR_HIP, "tile launch failed: %s", hipGetErrorString(e));
   e = flash::launch_merge(part, pe, dtype, B, H, KVH, 0, 0, out, m_star, vrows, seq_lens, block_n, w.cs, max_len,
-                          w.n_wg, static_cast<long long>(S), stream);
+                          a.n_wg, static_cast<long long>(S), stream, a.dense);
   if (e != hipSuccess) return set_error(SANTA_ERR_HIP, "merge launch failed: %s", hipGetErrorString(e));
   return clear_error();
 }

@@ -28,6 +28,28 @@ int clear_error();
 // num_pages > 0, table_stride >= ceil(max_len / page_size)) and fills pt.
 int check_page_table(const int* table, int num_pages, int page_size, int table_stride, int max_len, PageTable* pt);
 
+// Finer chunks for the densely sampled sequences of a ragged santa_flash grid
+// of cs tiles per chunk.  S_per_tile = S / tiles makes a short sequence's tiles
+// carry many samples, and its chunk's waves gather them (S * GH rows) in
+// dependent batches of 16, about 0.12 us a row against about 20 us for a tile
+// of keys: a tile weighs as much as (170 + GH * S_per_tile) / 170 sparse ones.
+// A sequence whose tiles carry at least 64 samples per KV head is cut into as
+// many more chunks (at most kDenseChunks more), each about as long a run as the
+// others' chunks.  limit: the (sequence, chunk) items of one resident round,
+// 0 for grids that are never cut this way; a batch whose finer chunks would
+// not all fit it keeps cs everywhere (where most sequences are dense the
+// gathers are spread evenly already, and chunks of a second round cost a start
+// and an end each: B = 32 at 2k-8k, S = 512, 117 us per step against 155).
+// 16 sequences of 1k-40k tokens at 32q/8kv, us per step: S = 256 186 -> 135,
+// S = 512 252 -> 137 (nothing to gather, S = 0: 128); at 64q/8kv 320 -> 199 and
+// 433 -> 207.
+struct DenseCut {
+  int gh;     // query heads per KV head
+  int limit;
+  int S;      // samples per sequence and head, at most 2^20 (beyond that every tile is dense anyway)
+};
+constexpr int kDenseChunks = 7;
+
 constexpr size_t kWsAlign = 256;
 inline size_t align_up(size_t x) { return (x + kWsAlign - 1) & ~(kWsAlign - 1); }
 

@@ -644,9 +644,9 @@ __global__ __launch_bounds__(kD) void finalize_kernel(const float* __restrict__ 
   int base = b * cpg * KVH;
   int nch = cpg;
   if (seq_lens) {
-    base = 0;
-    for (int bb = 0; bb < b; ++bb) base += KVH * (((ragged_len(seq_lens, bb, max_rows) + BN - 1) / BN + cs - 1) / cs);
-    nch = ((ragged_len(seq_lens, b, max_rows) + BN - 1) / BN + cs - 1) / cs;
+    const RaggedSeq rs = ragged_seq(seq_lens, b, b + 1, max_rows, BN, cs, DenseCut{0, 0, 0});
+    base = KVH * rs.first;
+    nch = (rs.tiles + cs - 1) / cs;
     // only the n_wg launched workgroups wrote partials
     nch = max(0, min(nch, (n_wg - base - kv + KVH - 1) / KVH));
   }

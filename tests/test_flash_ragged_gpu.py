@@ -96,6 +96,25 @@ def test_flash_ragged_wave_kernel_against_oracle(H, S):
     _run(H, 8, lens, S, 0, oracle_check=True)
 
 
+@pytest.mark.parametrize("H,S", [(32, 512), (64, 300), (32, 1)])
+def test_flash_ragged_dense_sequences(H, S):
+    """Short sequences beside long ones in the rows layout's one-round plan:
+    the densely sampled ones (down to one tile, and one with no dense tile at
+    S = 1) are cut into finer chunks that fit the round."""
+    lens = [30000, 300, 28000, 1000, 4097, 1, 9000, 2049]
+    assert sum((l + 255) // 256 for l in lens) * 8 > 2048
+    _run(H, 8, lens, S, 256, oracle_check=True)
+
+
+@pytest.mark.parametrize("B,lo,hi,S", [(32, 300, 4600, 512), (70, 700, 1500, 64)])
+def test_flash_ragged_many_sequences(B, lo, hi, S):
+    """Finer chunks that would not fit one round (32 sequences, all dense: the
+    plan's own chunks), and more sequences than lanes (70)."""
+    lens = seeded_lens(B, lo, hi, SEED + B)
+    assert sum((l + 255) // 256 for l in lens) * 8 > 2048
+    _run(32, 8, lens, S, 256)
+
+
 def test_flash_ragged_f16():
     _run(32, 8, [6000, 2500, 4100], 256, 0, dtype=torch.float16)
 
