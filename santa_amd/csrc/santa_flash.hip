@@ -849,7 +849,9 @@ __device__ __forceinline__ void slab_ell4(const float (&u)[4][2][2], float* fa01
 // read together, row by row, by one CU; each wave writes its own chunk
 // partial.  Otherwise four waves share one KV head, taking every fourth
 // tile, and merge their partials at the end of the chunk.
-template <bool BF16, int GH, bool DBG, bool P1 = false, bool PAGED = false, bool ROWS = false>
+// ROWS 2 (pass 1 only): the rows form for four KV heads, waves 0-3 and 4-7
+// taking KV heads 0-3 of the chunk's even and odd tiles.
+template <bool BF16, int GH, bool DBG, bool P1 = false, bool PAGED = false, int ROWS = 0>
 __global__ __launch_bounds__(ROWS ? 512 : kThreads, ROWS ? 1 : 2) void wave_kernel(
     const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K, const uint16_t* __restrict__ V, int H, int KVH,
     int L_valid, int L_storage, int T_c, int cs, int cpg, float q_scale, int S_pt, uint64_t seed,
@@ -864,14 +866,15 @@ __global__ __launch_bounds__(ROWS ? 512 : kThreads, ROWS ? 1 : 2) void wave_kern
   // the longest; workgroups past the last sequence only write an empty
   // partial)
   constexpr int NWV = ROWS ? 8 : 4;  // waves per workgroup (at most)
-  constexpr int TS = ROWS ? 1 : 4;    // tile stride of a wave
+  static_assert(ROWS < 2 || P1, "four KV heads in the rows form: no chunk partials to merge");
+  constexpr int TS = ROWS == 2 ? 2 : ROWS ? 1 : 4;  // tile stride of a wave
   const int tid = static_cast<int>(threadIdx.x);
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // ROWS workgroups enumerate (sequence, chunk) items (grid_pos with one
   // "head"); the KV head is the wave
   const GridPos gp = grid_pos(wg, seq_lens, B, ROWS ? 1 : KVH, BN, L_valid, T_c, cs, cpg, dense);
-  const int kv = ROWS ? wave : gp.kv;
+  const int kv = ROWS == 2 ? (wave & 3) : ROWS ? wave : gp.kv;
   const int b = gp.b < 0 ? 0 : gp.b;
   // heads per KV head: GH, except that santa_prop's pass 1 at GH 8 also takes
   // groups of 5-7 heads (santa_prop's generic shapes at D = 128), the second
@@ -883,7 +886,7 @@ __global__ __launch_bounds__(ROWS ? 512 : kThreads, ROWS ? 1 : 2) void wave_kern
   const int t_end = (gp.b < 0) ? t_begin : min(gp.n_tiles, t_begin + gp.cs);
   if (seq_lens)  // S_per_tile from this sequence's tile count (flash/santa_cuda.cpp:204-208)
     S_pt = (S_total > 0) ? static_cast<int>(max(1LL, S_total / static_cast<long long>(max(gp.n_tiles, 1)))) : 0;
-  const int t_first = ROWS ? t_begin : t_begin + wave;
+  const int t_first = ROWS == 2 ? t_begin + (wave >> 2) : ROWS ? t_begin : t_begin + wave;
 
   __shared__ u32x4 s_k[NWV * 64 * 16];  // per wave: 64 rows x 256 B staging; the chunk merge reuses it
   __shared__ int2 s_list[NWV * GH * LCAP];  // (row, coefficient bits) per listed row
@@ -1079,7 +1082,7 @@ __global__ __launch_bounds__(ROWS ? 512 : kThreads, ROWS ? 1 : 2) void wave_kern
       // no LDS for the checkpoint counts: the favour alternates by tile
       // parity instead (waves 4-7 on even tiles, 0-3 on odd ones), so that
       // neither SIMD partner keeps the lead the issue order gives it
-      if ((t + (wave >> 2)) & 1) {
+      if (((ROWS == 2 ? (t - t_first) >> 1 : t) + (wave >> 2)) & 1) {
         __builtin_amdgcn_s_setprio(1);
       } else {
         __builtin_amdgcn_s_setprio(0);
@@ -1933,7 +1936,7 @@ static hipError_t launch_wave_t(const Args& a, float* dbg_m, float* dbg_ell, int
   if (dbg_counts) {
     if (a.pt.table) return hipErrorInvalidValue;  // the statistics check reads contiguous caches
     if (rows_layout(a.KVH)) {  // the production layout, with the statistics written out
-      hipLaunchKernelGGL((wave_kernel<BF16, GH, true, false, false, true>), dim3(grid / static_cast<unsigned>(a.KVH)),
+      hipLaunchKernelGGL((wave_kernel<BF16, GH, true, false, false, 1>), dim3(grid / static_cast<unsigned>(a.KVH)),
                          dim3(static_cast<unsigned>(64 * a.KVH)), 0, stream, static_cast<const uint16_t*>(a.q),
                          static_cast<const uint16_t*>(a.K), static_cast<const uint16_t*>(a.V), a.H, a.KVH, a.L_valid,
                          a.L_storage, a.T_c, a.cs, a.cpg, q_scale, a.S_pt, a.seed, a.part, a.part_emit, a.seq_lens,
@@ -1950,13 +1953,13 @@ static hipError_t launch_wave_t(const Args& a, float* dbg_m, float* dbg_ell, int
     const unsigned rgrid = grid / static_cast<unsigned>(a.KVH);
     const dim3 block(static_cast<unsigned>(64 * a.KVH));
     if (a.pt.table)
-      hipLaunchKernelGGL((wave_kernel<BF16, GH, false, false, true, true>), dim3(rgrid), block, 0, stream,
+      hipLaunchKernelGGL((wave_kernel<BF16, GH, false, false, true, 1>), dim3(rgrid), block, 0, stream,
                          static_cast<const uint16_t*>(a.q), static_cast<const uint16_t*>(a.K),
                          static_cast<const uint16_t*>(a.V), a.H, a.KVH, a.L_valid, a.L_storage, a.T_c, a.cs, a.cpg,
                          q_scale, a.S_pt, a.seed, a.part, a.part_emit, a.seq_lens, a.B, a.S_total, nullptr,
                          nullptr, nullptr, nullptr, 0, a.pt, 0, 1, a.dense);
     else
-      hipLaunchKernelGGL((wave_kernel<BF16, GH, false, false, false, true>), dim3(rgrid), block, 0, stream,
+      hipLaunchKernelGGL((wave_kernel<BF16, GH, false, false, false, 1>), dim3(rgrid), block, 0, stream,
                          static_cast<const uint16_t*>(a.q), static_cast<const uint16_t*>(a.K),
                          static_cast<const uint16_t*>(a.V), a.H, a.KVH, a.L_valid, a.L_storage, a.T_c, a.cs, a.cpg,
                          q_scale, a.S_pt, a.seed, a.part, a.part_emit, a.seq_lens, a.B, a.S_total, nullptr,
@@ -2207,6 +2210,21 @@ hipError_t launch_prop_pass1(const void* q, const void* K, int dtype, int B, int
                                    : launch_bn<false, 8, kPass1Gen>(256, a, stream);
     }
     const bool rows = rows_layout(a.KVH) && (!a.seq_lens || total_tiles >= 0);
+    // Four KV heads (28q/4kv, 32q/4kv, 16q/4kv): the rows form with two tiles of
+    // a chunk at a time, whose four 256-B pieces of a token row one CU reads
+    // together, against four workgroups that read one piece each (28q/4kv, B =
+    // 8 at 32k, pass 1 69.5 -> 65.8 us; 16 sequences of 5k-70k at 16q/4kv 190 ->
+    // 176 us per step).  From one resident round of (kv, tile) items: fewer
+    // leave its second waves without a tile (16q/4kv, B = 1 at 32k 34.5 against
+    // 35.2 us per step).
+    const bool rows4 = a.KVH == 4 && kv_tiles >= rows_per_round();
+    if (rows4) {
+      if (a.seq_lens)
+        plan_ragged(a.B, a.KVH, total_tiles, a.T_c, &a.cs, &a.n_wg, rows_per_round() / 2, 2,
+                    (16LL * a.B * a.KVH <= rows_per_round()) ? 1 : 8);
+      else
+        chunk_plan(a.B, a.KVH, a.T_c, &a.cs, &a.cpg, rows_per_round() / 2);
+    }
     if (rows) {
       if (a.seq_lens) {
         // one round of chunks up to 32 sequences (B * KVH at most an eighth
@@ -2223,7 +2241,7 @@ hipError_t launch_prop_pass1(const void* q, const void* K, int dtype, int B, int
     }
     unsigned grid = a.seq_lens ? static_cast<unsigned>(a.n_wg)
                                : static_cast<unsigned>(a.B) * static_cast<unsigned>(a.KVH) * static_cast<unsigned>(a.cpg);
-    if (rows) grid /= static_cast<unsigned>(a.KVH);
+    if (rows || rows4) grid /= static_cast<unsigned>(a.KVH);
     // A tile-major stash larger than half the 256 MiB last-level cache is
     // written with non-temporal stores: cached, it would only evict itself
     // before pass 2 reads it (cfg5-shaped prop step, a 1 GiB stash: 1961 ->
@@ -2237,7 +2255,7 @@ hipError_t launch_prop_pass1(const void* q, const void* K, int dtype, int B, int
                              ? 1
                              : 0;
     if (grid == 0) return hipSuccess;
-    const dim3 block(rows ? static_cast<unsigned>(64 * a.KVH) : static_cast<unsigned>(kThreads));
+    const dim3 block(rows || rows4 ? 512u : static_cast<unsigned>(kThreads));
 #define SANTA_P1_LAUNCH(BF, G, PG, RW)                                                                            \
   hipLaunchKernelGGL((wave_kernel<BF, G, false, true, PG, RW>), dim3(grid), block, 0, stream,                     \
                      static_cast<const uint16_t*>(a.q), static_cast<const uint16_t*>(a.K), nullptr, a.H, a.KVH,     \
@@ -2253,15 +2271,19 @@ hipError_t launch_prop_pass1(const void* q, const void* K, int dtype, int B, int
   } while (0)
     if (dtype == SANTA_BF16) {
       if (rows) {
-        if (a.pt.table) SANTA_P1_GH(true, true, true); else SANTA_P1_GH(true, false, true);
+        if (a.pt.table) SANTA_P1_GH(true, true, 1); else SANTA_P1_GH(true, false, 1);
+      } else if (rows4) {
+        if (a.pt.table) SANTA_P1_GH(true, true, 2); else SANTA_P1_GH(true, false, 2);
       } else {
-        if (a.pt.table) SANTA_P1_GH(true, true, false); else SANTA_P1_GH(true, false, false);
+        if (a.pt.table) SANTA_P1_GH(true, true, 0); else SANTA_P1_GH(true, false, 0);
       }
     } else {
       if (rows) {
-        if (a.pt.table) SANTA_P1_GH(false, true, true); else SANTA_P1_GH(false, false, true);
+        if (a.pt.table) SANTA_P1_GH(false, true, 1); else SANTA_P1_GH(false, false, 1);
+      } else if (rows4) {
+        if (a.pt.table) SANTA_P1_GH(false, true, 2); else SANTA_P1_GH(false, false, 2);
       } else {
-        if (a.pt.table) SANTA_P1_GH(false, true, false); else SANTA_P1_GH(false, false, false);
+        if (a.pt.table) SANTA_P1_GH(false, true, 0); else SANTA_P1_GH(false, false, 0);
       }
     }
 #undef SANTA_P1_GH

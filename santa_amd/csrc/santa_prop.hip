@@ -374,7 +374,10 @@ __global__ __launch_bounds__(kThreads, (GH == 4 && BN == 256 && !PAGED) ? 6 : 4)
   const int kv = gp.kv;
   const int chunk = gp.chunk;
   const int b = gp.b < 0 ? 0 : gp.b;
-  const int h0 = kv * GH;
+  // heads per KV head: GH, except that GH 8 also takes groups of 5-7 heads, the
+  // missing ones with a zero budget everywhere and no partial
+  const int gsz = (GH == 8) ? H / KVH : GH;
+  const int h0 = kv * gsz;
   L = gp.len;  // this sequence's length from here on
   const int t_begin = chunk * cs;
   const int t_end = (gp.b < 0) ? t_begin : min(gp.n_tiles, t_begin + cs);
@@ -474,8 +477,9 @@ __global__ __launch_bounds__(kThreads, (GH == 4 && BN == 256 && !PAGED) ? 6 : 4)
     const int tt = min(t0 + lane, t_end - 1);
 #pragma unroll
     for (int k = 0; k < HPW; ++k) {
-      const size_t ht = (static_cast<size_t>(b) * H + h0 + wave + 4 * k) * T_c + tt;
-      inv_l[k] = invdelta[ht];
+      const bool real = GH != 8 || wave + 4 * k < gsz;
+      const size_t ht = (static_cast<size_t>(b) * H + h0 + (real ? wave + 4 * k : 0)) * T_c + tt;
+      inv_l[k] = real ? invdelta[ht] : 0.0f;
       a0_l[k] = a0_tile[ht];
     }
   };
@@ -499,7 +503,8 @@ __global__ __launch_bounds__(kThreads, (GH == 4 && BN == 256 && !PAGED) ? 6 : 4)
     if (act && !dbg_counts) {
       bool any = false;
 #pragma unroll
-      for (int g = 0; g < GH; ++g) any = any || invdelta[(static_cast<size_t>(b) * H + h0 + g) * T_c + tt] > 0.0f;
+      for (int g = 0; g < GH; ++g)
+        any = any || ((GH != 8 || g < gsz) && invdelta[(static_cast<size_t>(b) * H + h0 + g) * T_c + tt] > 0.0f);
       act = any;
     }
     return __ballot(act);
@@ -616,8 +621,8 @@ __global__ __launch_bounds__(kThreads, (GH == 4 && BN == 256 && !PAGED) ? 6 : 4)
 #pragma unroll
   for (int k = 0; k < HPW; ++k) {
     flush(k, wave + 4 * k);
-    float* pp = part + (static_cast<size_t>(wg) * GH + wave + 4 * k) * kD;
-    reinterpret_cast<float2*>(pp)[lane] = make_float2(acc0[k], acc1[k]);
+    float* pp = part + (static_cast<size_t>(wg) * gsz + wave + 4 * k) * kD;
+    if (GH != 8 || wave + 4 * k < gsz) reinterpret_cast<float2*>(pp)[lane] = make_float2(acc0[k], acc1[k]);
   }
   if (tid == 0) part_emit[wg] = emit_total;
 }
@@ -721,8 +726,26 @@ static int stash_ld(int L_storage) { return (L_storage + 255) / 256 * 256; }
 struct PropWs {
   size_t m, ell, st, inv, a0, stash, part, emit, total;
   int cs, cpg, n_wg;
+  bool pad8;  // groups of 5-7 heads on the tuned pass 2
 };
-static PropWs prop_ws_layout(int B, int H, int KVH, int D, int L_storage, int T_c, long long total_tiles = -1) {
+// Groups of 5-7 heads at D = 128 and block_n 256 run the tuned GH 8 pass 2 over
+// the tile-major stash (per-tile work of two waves' heads interleaved and the
+// stash two tiles ahead, where the generic form walks a head at a time): 28q/4kv,
+// B = 8 at 32k, pass 2 28.4 -> 23.2 us.  The debug form (counts) stays generic.
+// From half a resident round of (kv, tile) items; below it the generic form's plan
+// is level or ahead (40q/8kv, B = 3 at 5k: 32.8 against 34.6 us per step).
+static bool pass2_pad8(int GH, int D, int block_n, long long kv_tiles) {
+  return D == 128 && block_n == 256 && GH >= 5 && GH <= 7 && kv_tiles >= flash::rows_per_round() / 2;
+}
+// block_n 0: the larger of the plans a call of this shape may take.
+static PropWs prop_ws_layout(int B, int H, int KVH, int D, int L_storage, int T_c, long long total_tiles = -1,
+                             int block_n = 0) {
+  const long long kv_tiles = (total_tiles >= 0 ? total_tiles : static_cast<long long>(B) * T_c) * KVH;
+  if (block_n == 0 && pass2_pad8(H / KVH, D, 256, kv_tiles)) {
+    const PropWs a = prop_ws_layout(B, H, KVH, D, L_storage, T_c, total_tiles, 256);
+    const PropWs g = prop_ws_layout(B, H, KVH, D, L_storage, T_c, total_tiles, 32);
+    return a.total > g.total ? a : g;
+  }
   PropWs w{};
   size_t chunks;
   // Shapes that only the generic pass 2 takes: chunks for one round of as many
@@ -740,7 +763,8 @@ static PropWs prop_ws_layout(int B, int H, int KVH, int D, int L_storage, int T_
   // CU (four per CU measured 531.9 against 515.8 us on cfg3).
   const int GH = H / KVH;
   const int nw = propgen::pass2_waves(GH);
-  const bool tuned = D == 128 && (GH == 4 || GH == 8);
+  w.pad8 = pass2_pad8(GH, D, block_n, kv_tiles);
+  const bool tuned = (D == 128 && (GH == 4 || GH == 8)) || w.pad8;
   const bool uniform = total_tiles < 0 || total_tiles == static_cast<long long>(B) * T_c;
   int per_round = (!tuned && nw < 4) ? flash::rows_per_round() / nw : 0;
   if (tuned && uniform && static_cast<long long>(B) * KVH >= 32) per_round = flash::rows_per_round() / 4 * 2;
@@ -926,7 +950,8 @@ static int prop_pass2_launch(const void* V, const uint16_t* u_stash, int dtype, 
   const int want_emit = vrows ? 1 : 0;
   const float scale_out = (S > 0) ? (1.0f / static_cast<float>(S)) : 0.0f;
   hipError_t e;
-  if (propgen::generic_shape(GH, D, block_n)) {
+  const bool gen = propgen::generic_shape(GH, D, block_n);
+  if (gen && !(w.pad8 && stash_ld > 0 && !counts)) {
     e = propgen::launch_pass2(V, u_stash, dtype, B, H, KVH, D, L, L_storage, block_n, T_c, w.cs, w.cpg, w.n_wg,
                               invdelta, a0, counts, part, pe, want_emit, seq_lens, pt, stream, stash_ld);
     if (e != hipSuccess) return set_error(SANTA_ERR_HIP, "pass-2 launch failed: %s", hipGetErrorString(e));
@@ -948,6 +973,12 @@ static int prop_pass2_launch(const void* V, const uint16_t* u_stash, int dtype, 
                   : prop::launch_pass2_bn<false, 8>(block_n, Vh, u_stash, B, H, KVH, L, L_storage, T_c, w.cs, w.cpg,
                                                     invdelta, a0, counts, part, pe, want_emit, rg, stream);
   if (e != hipSuccess) return set_error(SANTA_ERR_HIP, "pass-2 launch failed: %s", hipGetErrorString(e));
+  if (gen) {  // groups of 5-7 heads: partials [chunk, GH, D], as the generic pass 2 leaves them
+    e = propgen::launch_finalize(part, pe, dtype, B, H, KVH, D, w.cpg, scale_out, out, vrows, seq_lens, seq_S,
+                                 block_n, w.cs, L, w.n_wg, stream);
+    if (e != hipSuccess) return set_error(SANTA_ERR_HIP, "finalize launch failed: %s", hipGetErrorString(e));
+    return SANTA_OK;
+  }
   const unsigned grid = static_cast<unsigned>(B) * static_cast<unsigned>(H);
   uint16_t* o = static_cast<uint16_t*>(out);
   if (dtype == SANTA_BF16) {
@@ -984,7 +1015,7 @@ extern "C" int santa_prop_pass2(const void* V, const void* u_stash, int dtype, i
   const int T_c = (L + block_n - 1) / block_n;
   if ((st = prop::check_bn(block_n, H / KVH, D)) != SANTA_OK) return st;
   if (!V || !u_stash || !invdelta || !a0 || !out) return set_error(SANTA_ERR_INVALID, "null pointer argument");
-  const prop::PropWs w = prop::prop_ws_layout(1, H, KVH, D, L, T_c);
+  const prop::PropWs w = prop::prop_ws_layout(1, H, KVH, D, L, T_c, -1, block_n);
   if (!workspace || workspace_bytes < w.total)
     return set_error(SANTA_ERR_WORKSPACE, "workspace too small: need %zu bytes, got %zu", w.total, workspace_bytes);
   st = prop_pass2_launch(V, static_cast<const uint16_t*>(u_stash), dtype, 1, H, KVH, D, L, L, block_n, T_c, S,
@@ -1005,7 +1036,7 @@ extern "C" int santa_prop_decode(const void* q, const void* K, const void* V, in
     return set_error(SANTA_ERR_INVALID, "SANTA_PASS1=vec requires GH=4, D=128, block_n=256. Got GH=%d D=%d block_n=%d",
                      H / KVH, D, block_n);
   if (!q || !K || !V || !out) return set_error(SANTA_ERR_INVALID, "null pointer argument");
-  const prop::PropWs w = prop::prop_ws_layout(1, H, KVH, D, L, T_c);
+  const prop::PropWs w = prop::prop_ws_layout(1, H, KVH, D, L, T_c, -1, block_n);
   if (!workspace || workspace_bytes < w.total)
     return set_error(SANTA_ERR_WORKSPACE, "workspace too small: need %zu bytes, got %zu", w.total, workspace_bytes);
   char* base = static_cast<char*>(workspace);
@@ -1063,7 +1094,7 @@ static int prop_decode_batched(const void* q, const void* K, const void* V, int 
     return set_error(SANTA_ERR_INVALID, "SANTA_PASS1=vec requires GH=4, D=128, block_n=256. Got GH=%d D=%d block_n=%d",
                      H / KVH, D, block_n);
   if (!q || !K || !V || !out || !seq_lens || !seq_S) return set_error(SANTA_ERR_INVALID, "null pointer argument");
-  const prop::PropWs w = prop::prop_ws_layout(B, H, KVH, D, L_storage, T_c, total_tiles);
+  const prop::PropWs w = prop::prop_ws_layout(B, H, KVH, D, L_storage, T_c, total_tiles, block_n);
   if (!workspace || workspace_bytes < w.total)
     return set_error(SANTA_ERR_WORKSPACE, "workspace too small: need %zu bytes, got %zu", w.total, workspace_bytes);
   char* base = static_cast<char*>(workspace);

@@ -243,3 +243,51 @@ def test_prop_general_batched_and_paged(H, KVH, D, lens, Ss, block_n, page_size,
         np.testing.assert_array_equal(vr[b].cpu().numpy(), exp["vrows"], err_msg=f"vrows b={b}")
         ok, mabs, mrel = tol_check(h16_to_f32(bits16(out[b])), h16_to_f32(exp["out16"]))
         assert ok, (f"b={b} vs oracle", mabs, mrel)
+
+
+@pytest.mark.parametrize("H,KVH,lens", [
+    (28, 4, [24000, 18001, 30000]),   # 1132 (kv, tile) items: tuned pass 2 (GH 7), generic pass 1
+    (20, 4, [24000] * 6),             # GH 5, uniform: four-head rows pass 1 and tuned pass 2
+    (24, 4, [23001, 300, 40000, 1, 30000, 40960, 2049]),  # GH 6, ragged, one-token and one-tile sequences
+    (48, 8, [40000, 30001]),          # GH 6 at eight KV heads
+    (16, 4, [23001, 300, 40000, 30000, 40960]),  # GH 4: four-head rows pass 1 on the vec path
+    (32, 4, [24000] * 6),             # GH 8: four-head rows pass 1
+])
+def test_batched_prop_four_kv_heads_and_groups_of_five_to_seven(H, KVH, lens, monkeypatch):
+    """Batches large enough for the rows form of pass 1 at four KV heads and
+    the tuned pass 2 at 5-7 heads per KV head, against the per-sequence calls
+    (too small for either) and the debug passes."""
+    _run(H, KVH, lens, [max(32, l // 64) for l in lens], 0, None, monkeypatch, SEED + H)
+
+
+def test_paged_prop_four_kv_heads():
+    """The paged form of the same pass 1 and pass 2: bit for bit the batched call."""
+    import santa_prop_batch_cuda as m
+
+    print("\n[case] prop paged, 28q/4kv and 16q/4kv, 64-token pages", flush=True)
+    lens, page = [23001, 300, 40000, 30000, 40960], 64
+    g = torch.Generator().manual_seed(SEED)
+    pages = [-(-l // page) for l in lens]
+    order = torch.randperm(sum(pages) + 3, generator=g)
+    table = torch.zeros(len(lens), max(pages), dtype=torch.int32)
+    for H in (28, 16):
+        q = torch.randn(len(lens), H, 128, generator=g).bfloat16().cuda()
+        K, V = (torch.randn(len(lens), max(lens), 4, 128, device="cuda", dtype=torch.bfloat16) for _ in range(2))
+        kp, vp = (torch.full((len(order), page, 4, 128), float("nan"), device="cuda", dtype=torch.bfloat16)
+                  for _ in range(2))
+        at = 0
+        for b, (l, n) in enumerate(zip(lens, pages)):
+            ids = order[at:at + n]
+            at += n
+            table[b, :n] = ids.int()
+            for src, dst in ((K, kp), (V, vp)):
+                rows = torch.full((n * page, 4, 128), float("nan"), device="cuda", dtype=torch.bfloat16)
+                rows[:l] = src[b, :l]
+                dst[ids.cuda()] = rows.view(n, page, 4, 128)
+        Ss = [max(32, l // 64) for l in lens]
+        a = m.decode_systematic_batched(q, K, V, Ss, seed=SEED, want_vrows=True, valid_len=lens)
+        p = m.decode_systematic_paged(q, kp, vp, table.cuda(), lens, Ss, seed=SEED, want_vrows=True)
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(bits16(a[0]), bits16(p[0]))
+        for x, y in zip(a[1:], p[1:]):
+            np.testing.assert_array_equal(x.cpu().numpy(), y.cpu().numpy())
