@@ -261,6 +261,8 @@ int santa_prop_decode_paged(const void* q, const void* K_pages, const void* V_pa
  * k_cache[b, pos] and v heads copied into v_cache[b, pos] of caches
  * [B, storage, KVH, D]; RoPE in the rotate-half convention with cos, sin
  * [D] and bf16 rounding of each product and of the sum.
+ * santa_rt_rope_table: cos_, sin_ [D] bf16 of position pos, the angle of
+ * dims i and i + D/2 being pos / theta^(2i / D).
  * santa_rt_rope_write_rows: santa_rt_rope_write for a prefill's P positions
  * pos .. pos + P - 1: qkv [B, P, H + 2 KVH, D], cos, sin [P, D], q_out
  * [B, P, H, D]; D a multiple of 16, every tensor 16-byte aligned.
@@ -305,6 +307,7 @@ int santa_rt_add_rms_norm(void* h, const void* a, const void* w, void* x, int ro
                           hipStream_t stream);
 int santa_rt_rope_write(const void* qkv, const void* cos_, const void* sin_, void* q_out, void* k_cache, void* v_cache,
                         int B, int H, int KVH, int D, long long storage, int pos, hipStream_t stream);
+int santa_rt_rope_table(int pos, float theta, int D, void* cos_, void* sin_, hipStream_t stream);
 int santa_rt_rope_write_rows(const void* qkv, const void* cos_, const void* sin_, void* q_out, void* k_cache,
                              void* v_cache, int B, int P, int H, int KVH, int D, long long storage, int pos,
                              hipStream_t stream);

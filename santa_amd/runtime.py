@@ -82,6 +82,7 @@ class _FusedOps:
                                                                          ctypes.c_void_p]
             L.santa_rt_rope_write.argtypes = [ctypes.c_void_p] * 6 + [ctypes.c_int] * 4 + [
                 ctypes.c_longlong, ctypes.c_int, ctypes.c_void_p]
+            L.santa_rt_rope_table.argtypes = [ctypes.c_int, ctypes.c_float, ctypes.c_int] + [ctypes.c_void_p] * 3
             L.santa_rt_rope_write_rows.argtypes = [ctypes.c_void_p] * 6 + [ctypes.c_int] * 5 + [
                 ctypes.c_longlong, ctypes.c_int, ctypes.c_void_p]
             L.santa_rt_silu_mul.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_int,
@@ -131,6 +132,15 @@ class _FusedOps:
                                                  kc.data_ptr(), vc.data_ptr(), B, heads, kv_heads, head_dim,
                                                  kc.shape[1], pos, cls._stream(qkv)))
         return q
+
+    @classmethod
+    def rope_table(cls, pos: int, head_dim: int, theta: float, like: torch.Tensor):
+        """_rope_cos_sin of one position in bf16, cos and sin [head_dim] on
+        like's device."""
+        t = torch.empty(2, head_dim, dtype=torch.bfloat16, device=like.device)
+        cls._check(cls.lib().santa_rt_rope_table(pos, theta, head_dim, t[0].data_ptr(), t[1].data_ptr(),
+                                                 cls._stream(t)))
+        return t[0], t[1]
 
     @classmethod
     def rope_write_rows(cls, qkv: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, k_cache: torch.Tensor,
@@ -519,11 +529,11 @@ class RandomLlama:
         (float32) -- tutorial_code/runtime_common.py:501-571."""
         s, D = self.shape, self.shape.head_dim
         B = token.shape[0]
-        cos, sin = _rope_cos_sin(torch.tensor([pos], device=self.device), D, s.rope_theta, self.dtype)
         h = self.embed[token]  # [B, hidden]
         if self.device.type == "cuda" and self.dtype == torch.bfloat16:
-            return self._decode_step_fused(h, cos.reshape(D).contiguous(), sin.reshape(D).contiguous(), pos, cache,
-                                           backend)
+            cos, sin = _FusedOps.rope_table(pos, D, s.rope_theta, h)
+            return self._decode_step_fused(h, cos, sin, pos, cache, backend)
+        cos, sin = _rope_cos_sin(torch.tensor([pos], device=self.device), D, s.rope_theta, self.dtype)
         for li, L in enumerate(self.layers):
             x = _rms_norm(h, L["ln1"], s.rms_eps)
             q, k, v = self._qkv(L, x)

@@ -96,6 +96,18 @@ def test_logits(rows, K, N):
     assert y.dtype == torch.float32 and torch.equal(y.to(torch.bfloat16), _FusedOps.linear(x, w))
 
 
+@pytest.mark.parametrize("D,theta", [(128, 500000.0), (64, 10000.0), (2, 500000.0), (96, 500000.0)])
+def test_rope_table(D, theta):
+    """cos and sin of single positions, bit for bit the torch expressions'."""
+    print(f"\n[case] rope_table D={D} theta={theta}", flush=True)
+    pos = list(range(0, 300)) + [1000, 4095, 8191, 32768, 40001, 131071]
+    got = [_FusedOps.rope_table(p, D, theta, torch.empty(0, device=DEV)) for p in pos]
+    cos, sin = _rope_cos_sin(torch.tensor(pos, device=DEV), D, theta, torch.bfloat16)
+    torch.cuda.synchronize()
+    for i, (c, s) in enumerate(got):
+        assert torch.equal(c, cos[i]) and torch.equal(s, sin[i]), pos[i]
+
+
 @pytest.mark.parametrize("rows,inter", [(1, 8), (5, 1000), (3, 1001), (300, 1032)])
 def test_silu_mul_forms(rows, inter):
     """The vector form and, for widths that are not a multiple of 8, the scalar one."""
