@@ -295,27 +295,41 @@ __device__ __forceinline__ GridPos grid_pos(int wg, const int* seq_lens, int B, 
 // Paged caches (PageTable): page ids are clamped to [0, num_pages), so a
 // malformed table gives wrong numbers, never an access outside the pool.
 
-// The pages of rows [n0, n0 + rows) of sequence b that lie below len, one per
-// lane: lane i holds the page of row block (n0 >> shift) + i; lanes past the
-// last such page (all lanes when n0 >= len) hold page 0.
-__device__ __forceinline__ int pages_of_rows(const PageTable& pt, int b, int n0, int rows, int len, int lane) {
-  const int last = min(n0 + rows, len) - 1;
-  const int p0 = n0 >> pt.shift;
-  const int np = (last >= n0) ? (last >> pt.shift) - p0 + 1 : 0;
-  int v = 0;
-  if (lane < np) v = pt.table[static_cast<size_t>(b) * pt.stride + p0 + lane];
-  return min(max(v, 0), pt.num_pages - 1);
-}
-
 // Per lane: the page of token `row` of sequence b (page 0 where !ok).
 __device__ __forceinline__ int page_of_row(const PageTable& pt, int b, int row, bool ok) {
   const int v = ok ? pt.table[static_cast<size_t>(b) * pt.stride + (row >> pt.shift)] : 0;
   return min(max(v, 0), pt.num_pages - 1);
 }
 
+// Page ids of row groups of G rows (G at most 8, so a group lies in one page),
+// one group per lane: rows n0 + G (lane mod N); page 0 where the group starts at
+// or past len.
+template <int G, int N>
+__device__ __forceinline__ int pages_of_groups(const PageTable& pt, int b, int n0, int len, int lane) {
+  const int n = n0 + G * (lane & (N - 1));
+  return page_of_row(pt, b, n, n < len);
+}
+
 // Byte offset from the pool base of token n, which lies in page `page`.
 __device__ __forceinline__ size_t paged_row(const PageTable& pt, int page, int n, uint32_t row_bytes) {
   return ((static_cast<size_t>(page) << pt.shift) + static_cast<size_t>(n & ((1 << pt.shift) - 1))) * row_bytes;
+}
+
+// A wave's row-group addresses, one group per lane (the two halves of a 64-bit
+// address), and group i's as a scalar: one vector pass of address arithmetic a
+// tile and two readlanes a load, where a page id read back per load cost it
+// about a dozen scalar instructions of 64-bit shifts and products (8 sequences
+// of 8k-48k over 16-token pages 109.0 -> 105.0 us per step).
+struct LaneAddr {
+  uint32_t lo, hi;
+};
+__device__ __forceinline__ LaneAddr lane_addr(const char* p) {
+  const uint64_t a = reinterpret_cast<uint64_t>(p);
+  return LaneAddr{static_cast<uint32_t>(a), static_cast<uint32_t>(a >> 32)};
+}
+__device__ __forceinline__ const char* addr_of_lane(const LaneAddr& a, int i) {
+  const uint32_t lo = __builtin_amdgcn_readlane(a.lo, i), hi = __builtin_amdgcn_readlane(a.hi, i);
+  return reinterpret_cast<const char*>((static_cast<uint64_t>(hi) << 32) | lo);
 }
 
 // ---------------------------------------------------------------- DPP

@@ -368,7 +368,7 @@ __global__ __launch_bounds__(kThreads, 2) void tile_kernel(
   // so one unconditional call site covers short tiles, waves without rows and
   // the missing successor of a chunk's last tile (no branches, so the loaded
   // registers are never copied and no wait lands before the scores).
-  // Paged: pv holds the pages of the wave's 64 rows of the tile (one per
+  // Paged: pv holds the pages of the wave's 16 row groups of the tile (one per
   // lane), loaded a tile ahead; a 4-row group never straddles two pages.
   u32x4 kw[16];
   const int k_lane_off = static_cast<int>((lane >> 4) * row_bytes + 16u * (lane & 15));
@@ -376,15 +376,15 @@ __global__ __launch_bounds__(kThreads, 2) void tile_kernel(
     const int n0 = t * BN;
     const int len = (t < t_end) ? min(BN, L_valid - n0) : 0;
     const char* kt = Kg + static_cast<size_t>(n0 + 64 * wave) * row_bytes;
+    LaneAddr av{0u, 0u};
+    if constexpr (PAGED) av = lane_addr(Kg + paged_row(pt, pv, n0 + 64 * wave + 4 * (lane & 15), row_bytes));
 #pragma unroll
     for (int c = 0; c < 16; ++c) {
       // wave-uniform; readfirstlane keeps the descriptor in SGPRs
       const int nvalid = __builtin_amdgcn_readfirstlane(min(max(len - 64 * wave - 4 * c, 0), 4));
       const char* gb;
       if constexpr (PAGED) {
-        const int n = n0 + 64 * wave + 4 * c;
-        const int page = __builtin_amdgcn_readlane(pv, (n >> pt.shift) - ((n0 + 64 * wave) >> pt.shift));
-        gb = Kg + paged_row(pt, page, n, row_bytes);
+        gb = addr_of_lane(av, c);
       } else {
         gb = kt + static_cast<size_t>(4 * c) * row_bytes;
       }
@@ -394,7 +394,7 @@ __global__ __launch_bounds__(kThreads, 2) void tile_kernel(
     }
   };
   auto wave_pages = [&](int t) -> int {
-    return PAGED ? pages_of_rows(pt, b, t * BN + 64 * wave, 64, L_valid, lane) : 0;
+    return PAGED ? pages_of_groups<4, 16>(pt, b, t * BN + 64 * wave, L_valid, lane) : 0;
   };
   load_k(t_begin, wave_pages(t_begin));
   int pv_next = wave_pages(t_begin + 1);
@@ -983,23 +983,18 @@ __global__ __launch_bounds__(ROWS ? 512 : kThreads, ROWS ? 1 : 2) void wave_kern
   // Sub-block sb = 2 hh + e of tile t: 16 loads of 4 rows (stride 2), one
   // descriptor each; rows at or past the tile's end (and every row of a tile
   // at or past t_end) read as zero and cost no traffic.  A load's rows lie in
-  // one 8-row aligned block, so in a paged cache in one page: pv holds the
-  // tile's pages, one per lane.
+  // one 8-row aligned block, so in a paged cache in one page: av holds the
+  // addresses of the tile's 8-row groups, one per lane.
   u32x4 kw[16];
   const int k_lane_off = static_cast<int>((lane >> 4) * 2u * row_bytes + 16u * (lane & 15));
-  auto group_base = [&](int t, int r, int pv) -> const char* {  // row t*BN + r, first of its load group
-    const int n = t * BN + r;
-    if constexpr (PAGED) {
-      const int page = __builtin_amdgcn_readlane(pv, (n >> pt.shift) - ((t * BN) >> pt.shift));
-      return Kg + paged_row(pt, page, n, row_bytes);
-    } else {
-      return Kg + static_cast<size_t>(n) * row_bytes;
-    }
-  };
   auto tile_pages = [&](int t) -> int {
-    return PAGED ? pages_of_rows(pt, b, t * BN, BN, L_valid, lane) : 0;
+    return PAGED ? pages_of_groups<8, 32>(pt, b, t * BN, L_valid, lane) : 0;
   };
-  auto load_k = [&](int t, int sb, int pv) {
+  auto tile_addr = [&](int t, int pv) -> LaneAddr {
+    if constexpr (PAGED) return lane_addr(Kg + paged_row(pt, pv, t * BN + 8 * (lane & 31), row_bytes));
+    return LaneAddr{0u, 0u};
+  };
+  auto load_k = [&](int t, int sb, const LaneAddr& av) {
     const uint32_t rb = row_bytes;
     const int len = (t < t_end) ? min(BN, L_valid - t * BN) : 0;
     const int r0 = 128 * (sb >> 1) + (sb & 1);
@@ -1010,7 +1005,7 @@ __global__ __launch_bounds__(ROWS ? 512 : kThreads, ROWS ? 1 : 2) void wave_kern
 #pragma unroll
     for (int c = 0; c < 16; ++c) {
       const int nvalid = min(max(rem - 8 * c, 0), 8);
-      const char* gb = PAGED ? group_base(t, r0 + 8 * c, pv) : kt + static_cast<size_t>(8 * c) * rb;
+      const char* gb = PAGED ? addr_of_lane(av, 16 * (sb >> 1) + c) + (sb & 1) * rb : kt + static_cast<size_t>(8 * c) * rb;
       const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
           const_cast<char*>(gb), static_cast<short>(0), nvalid * static_cast<int>(rb), kBufferWord3);
       kw[c] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, k_lane_off, 0, kBufferNontemporal));
@@ -1026,7 +1021,7 @@ __global__ __launch_bounds__(ROWS ? 512 : kThreads, ROWS ? 1 : 2) void wave_kern
 #pragma unroll
   for (int m = 0; m < 4; ++m)
     k_dma_off[m] = (lane >> 4) * 2u * row_bytes + 16u * static_cast<uint32_t>((lane & 15) ^ (4 * m + (lane >> 4)));
-  auto dma_k = [&](int t, int pv) {
+  auto dma_k = [&](int t, const LaneAddr& av) {
     const uint32_t rb = row_bytes;
     const int len = min(BN, L_valid - t * BN);
     const char* kt = Kg + static_cast<size_t>(t * BN) * rb;
@@ -1034,19 +1029,20 @@ __global__ __launch_bounds__(ROWS ? 512 : kThreads, ROWS ? 1 : 2) void wave_kern
 #pragma unroll
     for (int c = 0; c < 16; ++c) {
       const int nvalid = min(max(rem - 8 * c, 0), 8);
-      const char* gb = PAGED ? group_base(t, 8 * c, pv) : kt + static_cast<size_t>(8 * c) * rb;
+      const char* gb = PAGED ? addr_of_lane(av, c) : kt + static_cast<size_t>(8 * c) * rb;
       const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
           const_cast<char*>(gb), static_cast<short>(0), nvalid * static_cast<int>(rb), kBufferWord3);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)(wk + 64 * c), 16,
                                                k_dma_off[c & 3], 0, 0, kBufferNontemporal);
     }
   };
-  // pv: pages of the current tile; pv_next: of the wave's next tile (loaded
-  // while the current one is scored)
-  int pv = tile_pages(t_first);
+  // av: row-group addresses of the current tile; pv_next, av_next: pages and
+  // addresses of the wave's next tile (the pages loaded while the current one
+  // is scored)
+  LaneAddr av = tile_addr(t_first, tile_pages(t_first)), av_next{0u, 0u};
   int pv_next = 0;
-  if (t_first < t_end) dma_k(t_first, pv);
-  load_k(t_first, 1, pv);
+  if (t_first < t_end) dma_k(t_first, av);
+  load_k(t_first, 1, av);
 
   const int jrow = lane >> 4;
   const int qq = lane & 15;
@@ -1112,9 +1108,10 @@ __global__ __launch_bounds__(ROWS ? 512 : kThreads, ROWS ? 1 : 2) void wave_kern
         // sub-blocks 2, 3, then the next tile's sub-block 1 (GH 4; GH 8 loads
         // it after the next tile's DMA, below)
         if (sb < 3) {
-          load_k(t, sb + 1, pv);
-        } else if constexpr (GH == 4) {
-          load_k(t + TS, 1, pv_next);
+          load_k(t, sb + 1, av);
+        } else {
+          av_next = tile_addr(t + TS, pv_next);
+          if constexpr (GH == 4) load_k(t + TS, 1, av_next);
         }
         if (sb == 2) balance(3 * (t - t_first) + 1);
       }
@@ -1148,10 +1145,10 @@ __global__ __launch_bounds__(ROWS ? 512 : kThreads, ROWS ? 1 : 2) void wave_kern
 
     // every row of the staging area has been read: the next tile's sub-block 0
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    if (t + TS < t_end) dma_k(t + TS, pv_next);
+    if (t + TS < t_end) dma_k(t + TS, av_next);
     // GH 8: the next tile's sub-block 1 too, so that 32 KiB per wave are in
     // flight during the tail as for GH 4 (its registers fit beside the tail's)
-    if constexpr (GH == 8) load_k(t + TS, 1, pv_next);
+    if constexpr (GH == 8) load_k(t + TS, 1, av_next);
     balance(3 * (t - t_first) + 2);
 
     // ---- tile max per head (exact in any order) --------------------------------
@@ -1363,7 +1360,7 @@ __global__ __launch_bounds__(ROWS ? 512 : kThreads, ROWS ? 1 : 2) void wave_kern
         }
     }
     emit_total += __popcll(uni[0][0]) + __popcll(uni[0][1]) + __popcll(uni[1][0]) + __popcll(uni[1][1]);
-    pv = pv_next;
+    av = av_next;
   }
   // no load to LDS outstanding past here (the staging area is reused below)
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
