@@ -445,6 +445,9 @@ std::string tile_pass_kernel(int64_t B, int64_t H, int64_t KVH, int64_t T_c, int
                                                          static_cast<int>(T_c), static_cast<int>(H / KVH)))
     return "santa::flash::wave_kernel (block_n 256, " + gh +
            (santa::flash::rows_layout(static_cast<int>(KVH)) ? ", rows layout)" : ", four-wave layout)");
+  if (santa::flash::uniform_strips(static_cast<int>(B), static_cast<int>(KVH), static_cast<int>(T_c),
+                                   static_cast<int>(H / KVH), static_cast<int>(block_n)))
+    return "santa::flash::strip_kernel (block_n " + std::to_string(block_n) + ", " + gh + ", online)";
   return "santa::flash::tile_kernel (block_n " + std::to_string(block_n) + ", " + gh + ", online)";
 }
 

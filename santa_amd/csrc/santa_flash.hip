@@ -839,6 +839,56 @@ __device__ __forceinline__ void slab_ell4(const float (&u)[4][2][2], float* fa01
   __builtin_amdgcn_wave_barrier();
 }
 
+// The four waves' partials of a chunk (running max, mass, this lane's two
+// numerator dims and the emitted rows of each wave), merged in wave order into
+// pp [GH, kPartStride] and *emit.  sp: LDS that no wave uses any more, 4 * GH *
+// kPartStride floats and 4 counts.
+template <int GH>
+__device__ __forceinline__ void merge_waves(float* sp, const float (&runM)[GH], const float (&runZ)[GH],
+                                            const float (&num0)[GH], const float (&num1)[GH], int emit_total, int wave,
+                                            int lane, float* __restrict__ out, int* __restrict__ emit) {
+  __syncthreads();  // every wave is done with its staging area
+  int* s_emit = reinterpret_cast<int*>(sp + 4 * GH * kPartStride);
+#pragma unroll
+  for (int g = 0; g < GH; ++g) {
+    float* p = sp + (wave * GH + g) * kPartStride;
+    if (lane == 0) {
+      p[0] = runM[g];
+      p[1] = runZ[g];
+    }
+    p[2 + 2 * lane] = num0[g];
+    p[3 + 2 * lane] = num1[g];
+  }
+  if (lane == 0) s_emit[wave] = emit_total;
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < GH / 4; ++k) {
+    const int g = wave + 4 * k;
+    float M = -__builtin_inff();
+#pragma unroll
+    for (int w = 0; w < 4; ++w) M = fmaxf(M, sp[(w * GH + g) * kPartStride]);
+    float Z = 0.0f, n0v = 0.0f, n1v = 0.0f;
+    if (M != -__builtin_inff()) {
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        const float* p = sp + (w * GH + g) * kPartStride;
+        const float r = santa_expf(p[0] - M);
+        Z = fmaf(p[1], r, Z);
+        n0v = fmaf(p[2 + 2 * lane], r, n0v);
+        n1v = fmaf(p[3 + 2 * lane], r, n1v);
+      }
+    }
+    float* pp = out + g * kPartStride;
+    if (lane == 0) {
+      pp[0] = M;
+      pp[1] = Z;
+    }
+    pp[2 + 2 * lane] = n0v;
+    pp[3 + 2 * lane] = n1v;
+  }
+  if (wave == 0 && lane == 0) *emit = (s_emit[0] + s_emit[1]) + (s_emit[2] + s_emit[3]);
+}
+
 // P1: santa_prop pass 1 -- for GH 4 with the vec path's numerics (the flash
 // tile statistics), for GH 8 with the general path's (q rounded after
 // scaling, ell per 16-row slab): per tile and head m and ell into dbg_m /
@@ -1468,48 +1518,424 @@ __global__ __launch_bounds__(ROWS ? 512 : kThreads, ROWS ? 1 : 2) void wave_kern
     return;
   }
 
-  // ---- the four waves' partials, merged in wave order -----------------------------
-  __syncthreads();  // every wave is done with its staging area
-  float* sp = reinterpret_cast<float*>(s_k);  // [wave][g][kPartStride], then the wave emit counts
-  int* s_emit = reinterpret_cast<int*>(sp + 4 * GH * kPartStride);
+  merge_waves<GH>(reinterpret_cast<float*>(s_k), runM, runZ, num0, num1, emit_total, wave, lane,
+                  part + static_cast<size_t>(wg) * GH * kPartStride, part_emit + wg);
+}
+
+// ------------------------------------------------------------ strip kernel
+// santa_flash tiles of block_n = 32 or 64, online mode: a wave64 walks its chunk's
+// tiles (a quarter of them where the chunk is planned for a workgroup) in strips
+// of 128 consecutive rows, four tiles of 32 or two of 64.  The strip is scored in two
+// 64-row sub-blocks as wave_kernel scores a tile's half (lane 16j + q of
+// sub-block e owns row 32j + 2q + e), so a 16-lane DPP row holds one 32-row
+// block: the tiles' maxima, masses, scans and counts are the same vector
+// instructions for all tiles of the strip, with per-lane instead of
+// wave-uniform tile terms.  tile_kernel spends a workgroup, two barriers and a
+// whole latency chain on one such tile, and one wave of four has rows to score.
+// Statistics and counts are bit-identical to tile_kernel's; the output merge
+// differs in rounding (a strip's tiles share one running maximum).
+//
+// Bound by each wave's chain (scores, tail, gathers) at two waves per SIMD.  A
+// chunk planned for a single wave goes to one: four waves per such chunk of three
+// tiles leave most of their lanes without rows (B = 16: 61 us).  us per step at S =
+// 128 and 1,500 tokens, tile_kernel -> strip_kernel: B = 8 29.0 -> 20.1, B = 16
+// 63.1 -> 23.8, B = 32 105.6 -> 35.4; GH 8, B = 2 40.2 -> 27.0, B = 4 62.2 -> 35.2,
+// B = 16 153.2 -> 38.6, B = 32 253.4 -> 59.2; 16 ragged sequences of 300-1,500 (S =
+// 256) 57.0 -> 28.4, GH 8 127.7 -> 48.1.
+constexpr int kStripRows = 128;
+
+// Sum of the four (or eight) warps' sums held at lanes N * w of each 16-lane row,
+// in warp order, in every lane of the row.
+template <int N>
+__device__ __forceinline__ float row_sum4(float w) {
+  auto bc = [](float v, auto n) {
+    return __int_as_float(
+        __builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + decltype(n)::value, 0xF, 0xF, true));
+  };
+  float s = bc(w, std::integral_constant<int, 0>{});
+  s = s + bc(w, std::integral_constant<int, N>{});
+  s = s + bc(w, std::integral_constant<int, 2 * N>{});
+  return s + bc(w, std::integral_constant<int, 3 * N>{});
+}
+
+// ell of one head for the tile each lane's row lies in, from u of its two rows (0
+// past the tile's end): the reference's association for 128 threads, thread
+// GH * rho + g summing rows rho + (128 / GH) k in order k, then a tree of row
+// distances 64 / GH / 2 .. 1 per 32-thread warp, then the four warps in order.
+template <int GH, int BN>
+__device__ __forceinline__ float strip_ell(float u0, float u1, int lane) {
+  float A[2] = {u0, u1};
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    const float v = A[e];
+    if constexpr (GH == 4) {
+      if constexpr (BN == 64) A[e] = v + xrow16<0>(v);
+      A[e] = A[e] + dpp_shl_zero<2>(A[e]);
+      A[e] = A[e] + dpp_shl_zero<1>(A[e]);
+    } else {
+      float a = v + dpp_shl_zero<8>(v);
+      if constexpr (BN == 64) {
+        const float o = xrow16<0>(v);
+        a = a + o;
+        a = a + dpp_shl_zero<8>(o);
+      }
+      A[e] = a + dpp_shl_zero<1>(a);
+    }
+  }
+  float ell = row_sum4<GH == 4 ? 4 : 2>(A[0] + A[1]);
+  if constexpr (BN == 64) {  // formed in the even rows: a tile is two rows
+    const float o = __int_as_float(lane_xor<16>(__float_as_int(ell), lane));
+    ell = (lane & 16) ? o : ell;
+  }
+  return ell;
+}
+
+template <bool BF16, int GH, int BN, bool PAGED>
+__global__ __launch_bounds__(kThreads, 2) void strip_kernel(
+    const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K, const uint16_t* __restrict__ V, int H, int KVH,
+    int L_valid, int L_storage, int T_c, int cs, int cpg, float q_scale, int S_pt, uint64_t seed,
+    float* __restrict__ part, int* __restrict__ part_emit, const int* __restrict__ seq_lens, int B, long long S_total,
+    int wave_items, PageTable pt) {
+  static_assert(BN == 32 || BN == 64, "block_n");
+  constexpr int NHB = GH / 4;
+  constexpr int LCAP = kWaveListCap;
+  const int tid = static_cast<int>(threadIdx.x);
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // wave_items: each wave has a (b, kv, chunk) item of its own, the four waves
+  // four adjacent KV heads of a chunk (the grid's items are a multiple of KVH = 8)
+  const int wg = wave_items ? 4 * static_cast<int>(blockIdx.x) + wave : static_cast<int>(blockIdx.x);
+  const GridPos gp = grid_pos(wg, seq_lens, B, KVH, BN, L_valid, T_c, cs, cpg);
+  const int kv = gp.kv;
+  const int b = gp.b < 0 ? 0 : gp.b;
+  const int h0 = kv * GH;
+  L_valid = gp.len;
+  const int t_begin = gp.chunk * cs;
+  const int t_end = (gp.b < 0) ? t_begin : min(gp.n_tiles, t_begin + cs);
+  // the chunk's tiles, whole or in four near-equal runs, one per wave
+  const int run = wave_items ? t_end - t_begin : (t_end - t_begin + 3) / 4;
+  const int w_begin = wave_items ? t_begin : t_begin + run * wave;
+  const int row_end = min(L_valid, min(t_end, w_begin + run) * BN);  // of this wave's rows
+  if (seq_lens)  // S_per_tile from this sequence's tile count (flash/santa_cuda.cpp:204-208)
+    S_pt = (S_total > 0) ? static_cast<int>(max(1LL, S_total / static_cast<long long>(max(gp.n_tiles, 1)))) : 0;
+
+  __shared__ u32x4 s_k[4 * 64 * 16];        // per wave: 64 rows x 256 B staging; the chunk merge reuses it
+  __shared__ int2 s_list[4 * GH * LCAP];    // (row, coefficient bits) per listed row
+  u32x4* const wk = s_k + wave * 64 * 16;
+  int2* const list = s_list + wave * GH * LCAP;
+
+  const uint32_t row_bytes = static_cast<uint32_t>(KVH) * kD * 2u;
+  const size_t seq_off = PAGED ? 0 : static_cast<size_t>(b) * L_storage * KVH * kD;
+  const char* Kg = reinterpret_cast<const char*>(K + seq_off + static_cast<size_t>(kv) * kD);
+  const char* Vg = reinterpret_cast<const char*>(V + seq_off + static_cast<size_t>(kv) * kD);
+  const uint32_t v_lane_off = 4u * static_cast<uint32_t>(lane);
+
+  float qa[NHB][8];
+#pragma unroll
+  for (int hb = 0; hb < NHB; ++hb) {
+    const uint16_t* qh = Q + (static_cast<size_t>(b) * H + h0 + 4 * hb + (lane & 3)) * kD + (lane >> 2);
+#pragma unroll
+    for (int m = 0; m < 8; ++m) qa[hb][m] = h16_to_f32<BF16>(qh[16 * m]) * q_scale;
+  }
+
+  float runM[GH], runZ[GH], num0[GH], num1[GH];
+  int lcnt[GH];
 #pragma unroll
   for (int g = 0; g < GH; ++g) {
-    float* p = sp + (wave * GH + g) * kPartStride;
-    if (lane == 0) {
-      p[0] = runM[g];
-      p[1] = runZ[g];
-    }
-    p[2 + 2 * lane] = num0[g];
-    p[3 + 2 * lane] = num1[g];
+    runM[g] = -__builtin_inff();
+    runZ[g] = 0.0f;
+    num0[g] = 0.0f;
+    num1[g] = 0.0f;
+    lcnt[g] = 0;
   }
-  if (lane == 0) s_emit[wave] = emit_total;
-  __syncthreads();
+  int emit_total = 0;
+
+  // Listed rows' loads and sums, as in wave_kernel: entry j's V row through the
+  // address lane j holds, the lane's 4 B at v_lane_off.
+  auto v_addr = [&](int rowv, bool ok) -> LaneAddr {
+    if constexpr (PAGED) {
+      return lane_addr(Vg + paged_row(pt, page_of_row(pt, b, rowv, ok), rowv, row_bytes));
+    } else {
+      return lane_addr(Vg + static_cast<size_t>(rowv) * row_bytes);
+    }
+  };
+  auto v_load = [&](const LaneAddr& av, int j) -> uint32_t {
+    typedef const __attribute__((address_space(1))) char* gbytes;
+    const gbytes row = reinterpret_cast<gbytes>(reinterpret_cast<uint64_t>(addr_of_lane(av, j)));
+    return *reinterpret_cast<const __attribute__((address_space(1))) uint32_t*>(row + v_lane_off);
+  };
+  auto accumulate = [&](int g, float coefv, const uint32_t (&vw)[16], int q0, int n) {
 #pragma unroll
-  for (int k = 0; k < NHB; ++k) {
-    const int g = wave + 4 * k;
-    float M = -__builtin_inff();
+    for (int q = 0; q < 16; ++q) {
+      const float c = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(coefv), min(q0 + q, n - 1)));
+      const float a0 = fmaf(c, lo16_to_f32<BF16>(vw[q]), num0[g]);
+      const float a1 = fmaf(c, hi16_to_f32<BF16>(vw[q]), num1[g]);
+      const bool ok = q0 + q < n;
+      num0[g] = ok ? a0 : num0[g];
+      num1[g] = ok ? a1 : num1[g];
+    }
+  };
+  auto flush = [&](int g) {
+    const int n = lcnt[g];
+    if (n <= 0) return;
+    const int2 ent = (lane < n) ? list[g * LCAP + lane] : make_int2(0, 0);
+    const LaneAddr av = v_addr(ent.x, lane < n);
+    const float coefv = __int_as_float(ent.y);
+    int q0 = 0;
+    do {
+      uint32_t vw[16];
 #pragma unroll
-    for (int w = 0; w < 4; ++w) M = fmaxf(M, sp[(w * GH + g) * kPartStride]);
-    float Z = 0.0f, n0v = 0.0f, n1v = 0.0f;
-    if (M != -__builtin_inff()) {
+      for (int q = 0; q < 16; ++q) vw[q] = v_load(av, min(q0 + q, n - 1));
+      accumulate(g, coefv, vw, q0, n);
+      q0 += 16;
+    } while (q0 < n);
+    lcnt[g] = 0;
+  };
+
+  // Sub-block e of the strip from row n0: 16 loads of 4 rows (stride 2), as
+  // wave_kernel's; rows at or past row_end read as zero.  Sub-block 0 goes
+  // straight into the staging area, sub-block 1 through registers.
+  u32x4 kw[16];
+  const int k_lane_off = static_cast<int>((lane >> 4) * 2u * row_bytes + 16u * (lane & 15));
+  uint32_t k_dma_off[4];
 #pragma unroll
-      for (int w = 0; w < 4; ++w) {
-        const float* p = sp + (w * GH + g) * kPartStride;
-        const float r = santa_expf(p[0] - M);
-        Z = fmaf(p[1], r, Z);
-        n0v = fmaf(p[2 + 2 * lane], r, n0v);
-        n1v = fmaf(p[3 + 2 * lane], r, n1v);
+  for (int m = 0; m < 4; ++m)
+    k_dma_off[m] = (lane >> 4) * 2u * row_bytes + 16u * static_cast<uint32_t>((lane & 15) ^ (4 * m + (lane >> 4)));
+  auto strip_pages = [&](int n0) -> int {
+    return PAGED ? pages_of_groups<8, 16>(pt, b, n0, row_end, lane) : 0;
+  };
+  auto load_strip = [&](int n0, int pv) {
+    const char* kt = Kg + static_cast<size_t>(n0) * row_bytes;
+    LaneAddr av{0u, 0u};
+    if constexpr (PAGED) av = lane_addr(Kg + paged_row(pt, pv, n0 + 8 * (lane & 15), row_bytes));
+    const int rem = __builtin_amdgcn_readfirstlane(row_end - n0);
+#pragma unroll
+    for (int c = 0; c < 16; ++c) {
+      // wave-uniform; readfirstlane keeps the descriptor in SGPRs
+      const int nvalid = __builtin_amdgcn_readfirstlane(min(max(rem - 8 * c, 0), 8));
+      const char* gb = PAGED ? addr_of_lane(av, c) : kt + static_cast<size_t>(8 * c) * row_bytes;
+      const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+          const_cast<char*>(gb), static_cast<short>(0), nvalid * static_cast<int>(row_bytes), kBufferWord3);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)(wk + 64 * c), 16,
+                                               k_dma_off[c & 3], 0, 0, kBufferNontemporal);
+    }
+    // the wait for sub-block 0 counts on this order of the loads
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int c = 0; c < 16; ++c) {
+      const int nvalid = __builtin_amdgcn_readfirstlane(min(max(rem - 1 - 8 * c, 0), 8));
+      const char* gb = (PAGED ? addr_of_lane(av, c) : kt + static_cast<size_t>(8 * c) * row_bytes) + row_bytes;
+      const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+          const_cast<char*>(gb), static_cast<short>(0), nvalid * static_cast<int>(row_bytes), kBufferWord3);
+      kw[c] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, k_lane_off, 0, kBufferNontemporal));
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  const int jrow = lane >> 4;
+  const int qq = lane & 15;
+  const int first = w_begin * BN;
+  if (first < row_end) load_strip(first, strip_pages(first));
+  for (int n0 = first; n0 < row_end; n0 += kStripRows) {
+    const int len = min(kStripRows, row_end - n0);
+    const int next = n0 + kStripRows;
+
+    // ---- scores ------------------------------------------------------------
+    f32x4 sc[2][NHB];
+    int pv_next = 0;
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      if (e == 0) {
+        // sub-block 0 came by DMA; the 16 register loads of sub-block 1 were
+        // issued after it and may still be in flight
+        asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+        if constexpr (PAGED) pv_next = strip_pages(next);
+      } else {
+#pragma unroll
+        for (int c = 0; c < 16; ++c) {
+          const int r = 4 * c + (lane >> 4);
+          wk[r * 16 + ((lane & 15) ^ (r & 15))] = kw[c];
+        }
+      }
+      __builtin_amdgcn_wave_barrier();
+      if constexpr (NHB == 1) {
+        f32x4 be0[1], bo0[1], be2[1], bo2[1], be1[1], bo1[1], be3[1], bo3[1];
+        score_group<BF16, 1, 0>(wk, lane, qa, be0, bo0);
+        score_group<BF16, 1, 2>(wk, lane, qa, be2, bo2);
+        score_group<BF16, 1, 1>(wk, lane, qa, be1, bo1);
+        score_group<BF16, 1, 3>(wk, lane, qa, be3, bo3);
+        const f32x4 de = (be0[0] + be2[0]) + (be1[0] + be3[0]);
+        const f32x4 dd = (bo0[0] + bo2[0]) + (bo1[0] + bo3[0]);
+        sc[e][0] = de + dd;
+        pin(sc[e][0]);
+      } else {
+#pragma unroll
+        for (int hb = 0; hb < NHB; ++hb) {
+          f32x4 be0, bo0, be2, bo2, be1, bo1, be3, bo3;
+          score_group1<BF16, 0>(wk, lane, qa[hb], be0, bo0);
+          score_group1<BF16, 2>(wk, lane, qa[hb], be2, bo2);
+          score_group1<BF16, 1>(wk, lane, qa[hb], be1, bo1);
+          score_group1<BF16, 3>(wk, lane, qa[hb], be3, bo3);
+          sc[e][hb] = ((be0 + be2) + (be1 + be3)) + ((bo0 + bo2) + (bo1 + bo3));
+          pin(sc[e][hb]);
+        }
       }
     }
-    float* pp = part + (static_cast<size_t>(wg) * GH + g) * kPartStride;
-    if (lane == 0) {
-      pp[0] = M;
-      pp[1] = Z;
-    }
-    pp[2 + 2 * lane] = n0v;
-    pp[3 + 2 * lane] = n1v;
+    // every row of the staging area has been read
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (next < row_end) load_strip(next, pv_next);
+
+    // ---- per tile and head: max, u, ell, counts; per strip: running max, lists ----
+    const bool ok = (BN == 32 ? 32 * jrow : 64 * (jrow >> 1)) < len;  // this lane's tile has rows
+    const bool valid[2] = {32 * jrow + 2 * qq < len, 32 * jrow + 2 * qq + 1 < len};
+    const int t = n0 / BN + (BN == 32 ? jrow : jrow >> 1);            // this lane's tile
+    uint64_t uni[2] = {0, 0};
+    auto head_block = [&](auto hbc) {
+      constexpr int hb = decltype(hbc)::value;
+      // a0 of head 4 hb + k: drawn in the lanes k mod 4 of the tile's rows
+      const float draw = u01(seed, b * H + h0 + 4 * hb + (qq & 3), t);
+      float a0[4];
+      a0[0] = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(draw), 0x150, 0xF, 0xF, true));
+      a0[1] = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(draw), 0x151, 0xF, 0xF, true));
+      a0[2] = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(draw), 0x152, 0xF, 0xF, true));
+      a0[3] = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(draw), 0x153, 0xF, 0xF, true));
+      int cnt[4][2];
+      float mg[4], ell[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        int key = -2147483647 - 1;
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+          if (valid[e]) key = max(key, order_key(sc[e][hb][k]));
+        key = max(key, __builtin_amdgcn_update_dpp(0, key, kDppQuadXor1, 0xF, 0xF, false));
+        key = max(key, __builtin_amdgcn_update_dpp(0, key, kDppQuadXor2, 0xF, 0xF, false));
+        key = max(key, __builtin_amdgcn_update_dpp(0, key, kDppRowHalfMirror, 0xF, 0xF, false));
+        key = max(key, __builtin_amdgcn_update_dpp(0, key, kDppRowMirror, 0xF, 0xF, false));
+        if constexpr (BN == 64) key = max(key, lane_xor<16>(key, lane));
+        mg[k] = ok ? from_order_key(key) : -__builtin_inff();
+        float u[2], ub[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const float d = sc[e][hb][k] - mg[k];
+          const float ex = santa_expf_nonpos(valid[e] ? d : 0.0f);
+          u[e] = valid[e] ? ex : 0.0f;
+          ub[e] = round16_nonneg<BF16>(u[e]);
+        }
+        ell[k] = strip_ell<GH, BN>(u[0], u[1], lane);
+        const float invdel = (S_pt > 0 && ell[k] > 1e-20f) ? (static_cast<float>(S_pt) / ell[k]) : 0.0f;
+        const float x0[1] = {ub[0] * invdel}, x1[1] = {ub[1] * invdel};
+        float pre0[1], pre1[1];
+        scan_pairs<1>(x0, x1, pre0, pre1);
+        float car = 0.0f;
+        if constexpr (BN == 64)  // the second 32-row chunk carries the first one's total
+          car = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(pre1[0] + x1[0]), 0x142, 0xA, 0xF, false));
+        const float pg0 = car + pre0[0], pg1 = car + pre1[0];
+        cnt[k][0] = valid[0] ? count_from_floors(a0[k], pg0, pg0 + x0[0]) : 0;
+        cnt[k][1] = valid[1] ? count_from_floors(a0[k], pg1, pg1 + x1[0]) : 0;
+      }
+      // the strip's maximum, the running one with it, and the sampled rows'
+      // coefficients c * ell_t * exp(m_t - M) relative to it
+      float f[4], rsc[4];
+      bool grow[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int g = 4 * hb + k;
+        float mw = fmaxf(mg[k], __int_as_float(lane_xor<16>(__float_as_int(mg[k]), lane)));
+        mw = fmaxf(mw, __int_as_float(lane_xor<32>(__float_as_int(mw), lane)));
+        mw = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(mw)));
+        grow[k] = mw > runM[g];
+        const float mn = grow[k] ? mw : runM[g];
+        rsc[k] = santa_expf(runM[g] - mn);
+        f[k] = ok ? ell[k] * santa_expf(mg[k] - mn) : 0.0f;
+        float z = f[k];
+        if constexpr (BN == 32) z = z + __int_as_float(lane_xor<16>(__float_as_int(z), lane));
+        z = z + __int_as_float(lane_xor<32>(__float_as_int(z), lane));
+        runZ[g] = grow[k] ? fmaf(runZ[g], rsc[k], z) : runZ[g] + z;
+        num0[g] = grow[k] ? num0[g] * rsc[k] : num0[g];
+        num1[g] = grow[k] ? num1[g] * rsc[k] : num1[g];
+        runM[g] = mn;
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int g = 4 * hb + k;
+        if (grow[k] && lane < lcnt[g]) {
+          int* const cw = &list[g * LCAP + lane].y;
+          *cw = __float_as_int(__int_as_float(*cw) * rsc[k]);
+        }
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const int c = cnt[k][e];
+          const uint64_t nz = __ballot(c != 0);
+          uni[e] |= nz;
+          const int nn = __popcll(nz);
+          if (nn) {
+            if (lcnt[g] + nn > LCAP) flush(g);
+            if (c != 0) {
+              const int pos = lcnt[g] + static_cast<int>(__builtin_amdgcn_mbcnt_hi(
+                                            static_cast<uint32_t>(nz >> 32),
+                                            __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(nz), 0u)));
+              list[g * LCAP + pos] =
+                  make_int2(n0 + 32 * jrow + 2 * qq + e, __float_as_int(static_cast<float>(c) * f[k]));
+            }
+            lcnt[g] += nn;
+          }
+        }
+      }
+    };
+    head_block(std::integral_constant<int, 0>{});
+    if constexpr (NHB == 2) head_block(std::integral_constant<int, 1>{});
+    emit_total += __popcll(uni[0]) + __popcll(uni[1]);
   }
-  if (tid == 0) part_emit[wg] = (s_emit[0] + s_emit[1]) + (s_emit[2] + s_emit[3]);
+  // no load to LDS outstanding past here (the staging area is reused below)
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  // the remaining listed rows: up to 16 of each of four heads in one round trip
+#pragma unroll
+  for (int hb = 0; hb < NHB; ++hb) {
+    int nmax = 0;
+    LaneAddr av[4];
+    float coefv[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int g = 4 * hb + k;
+      nmax = max(nmax, lcnt[g]);
+      const int2 ent = (lane < lcnt[g]) ? list[g * LCAP + lane] : make_int2(0, 0);
+      av[k] = v_addr(ent.x, lane < lcnt[g]);
+      coefv[k] = __int_as_float(ent.y);
+    }
+    for (int q0 = 0; q0 < nmax; q0 += 16) {
+      uint32_t vw[4][16];
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (lcnt[4 * hb + k] > q0) {
+#pragma unroll
+          for (int q = 0; q < 16; ++q) vw[k][q] = v_load(av[k], min(q0 + q, lcnt[4 * hb + k] - 1));
+        }
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (lcnt[4 * hb + k] > q0) accumulate(4 * hb + k, coefv[k], vw[k], q0, lcnt[4 * hb + k]);
+    }
+  }
+
+  if (wave_items) {
+    // this wave's partial is the (b, kv, chunk) partial
+#pragma unroll
+    for (int g = 0; g < GH; ++g) {
+      float* pp = part + (static_cast<size_t>(wg) * GH + g) * kPartStride;
+      if (lane == 0) {
+        pp[0] = runM[g];
+        pp[1] = runZ[g];
+      }
+      pp[2 + 2 * lane] = num0[g];
+      pp[3 + 2 * lane] = num1[g];
+    }
+    if (lane == 0) part_emit[wg] = emit_total;
+    return;
+  }
+
+  // ---- the four waves' partials, merged in wave order -----------------------------
+  merge_waves<GH>(reinterpret_cast<float*>(s_k), runM, runZ, num0, num1, emit_total, wave, lane,
+                  part + static_cast<size_t>(wg) * GH * kPartStride, part_emit + wg);
 }
 
 // Split-KV merge of per-tile partials (flash/santa_cuda_kernel.cu:386-470):
@@ -1886,6 +2312,23 @@ struct Args {
   DenseCut dense{0, 0, 0};  // ragged flash: finer chunks for densely sampled sequences
 };
 
+// The online pass at block_n 32 / 64 runs on strip_kernel where a strip has
+// company: in single waves' chunks from a quarter of a round of items, in
+// workgroups' from four tiles.  Below, a CU holds a workgroup or two and
+// tile_kernel's shorter chain for one tile wins.  us per step, tile_kernel against
+// strip_kernel: ragged lengths of 60-300, B = 8 (416 items) 15.3 / 19.4, GH 8 24.6
+// / 32.6, B = 16 (840) 25.8 / 20.1, 48.4 / 34.1; workgroups' chunks of two tiles
+// (B = 2, 1,500 tokens) 15.8 / 19.8, three (B = 4) 18.9 / 20.1, five (B = 6)
+// 25.5 / 19.9.
+// *waves: chunks planned for single-wave items (the rows plan of flash_ws_layout and
+// ragged_ws_layout) go to single waves, others to workgroups.
+static bool strips(bool ragged, int B, int KVH, int T_c, int GH, int cs, long long items, bool* waves) {
+  const bool many = items > rows_per_round() / 4;
+  if (!many && cs < 4) return false;
+  *waves = rows_layout(KVH) && (ragged || !uniform_small_pass(B, KVH, T_c, GH));
+  return *waves ? many : cs >= 4;
+}
+
 template <bool BF16, int GH, int BN, int MODE, bool PAGED>
 static hipError_t launch_tk(const Args& a, hipStream_t stream) {
   const float q_scale = 1.0f / sqrtf(static_cast<float>(kD));
@@ -1900,10 +2343,34 @@ static hipError_t launch_tk(const Args& a, hipStream_t stream) {
   return hipGetLastError();
 }
 
+template <bool BF16, int GH, int BN>
+static hipError_t launch_strips(const Args& a, bool wave_items, hipStream_t stream) {
+  const float q_scale = 1.0f / sqrtf(static_cast<float>(kD));
+  const unsigned items = a.seq_lens ? static_cast<unsigned>(a.n_wg)
+                                    : static_cast<unsigned>(a.B) * static_cast<unsigned>(a.KVH) * static_cast<unsigned>(a.cpg);
+  const unsigned grid = wave_items ? (items + 3) / 4 : items;
+  if (grid == 0) return hipSuccess;
+#define SANTA_STRIP(PG)                                                                                             \
+  hipLaunchKernelGGL((strip_kernel<BF16, GH, BN, PG>), dim3(grid), dim3(kThreads), 0, stream,                      \
+                     static_cast<const uint16_t*>(a.q), static_cast<const uint16_t*>(a.K),                          \
+                     static_cast<const uint16_t*>(a.V), a.H, a.KVH, a.L_valid, a.L_storage, a.T_c, a.cs, a.cpg,     \
+                     q_scale, a.S_pt, a.seed, a.part, a.part_emit, a.seq_lens, a.B, a.S_total, wave_items ? 1 : 0, a.pt)
+  if (a.pt.table) SANTA_STRIP(true);
+  else SANTA_STRIP(false);
+#undef SANTA_STRIP
+  return hipGetLastError();
+}
+
 // Paged caches go through the online mode at block_n 32/64 (block_n 256 is
 // the wave kernel's) and the general pass 1.
 template <bool BF16, int GH, int BN, int MODE>
 static hipError_t launch_t(const Args& a, hipStream_t stream) {
+  if constexpr (MODE == kOnline && BN != 256) {
+    const long long items = a.seq_lens ? a.n_wg : static_cast<long long>(a.B) * a.KVH * a.cpg;
+    bool waves;
+    if (strips(a.seq_lens != nullptr, a.B, a.KVH, a.T_c, GH, a.cs, items, &waves))
+      return launch_strips<BF16, GH, BN>(a, waves, stream);
+  }
   if (a.pt.table) {
     if constexpr (MODE == kOnline || MODE == kPass1Gen) return launch_tk<BF16, GH, BN, MODE, true>(a, stream);
     return hipErrorInvalidValue;
@@ -2483,6 +2950,11 @@ FlashWs flash_ws_layout(int B, int H, int KVH, int T_c) {
 namespace santa {
 namespace flash {
 // Declared in santa_internal.h.
+bool uniform_strips(int B, int KVH, int T_c, int GH, int block_n) {
+  const FlashWs w = flash_ws_layout(B, GH * KVH, KVH, T_c);
+  bool waves;
+  return block_n != 256 && strips(false, B, KVH, T_c, GH, w.cs, static_cast<long long>(B) * KVH * w.cpg, &waves);
+}
 hipError_t launch_wave_debug(const void* q, const void* K, const void* V, int dtype, int B, int H, int KVH,
                              int L_valid, int L_storage, int S_pt, uint64_t seed, void* workspace, float* m_tiles,
                              float* ell_tiles, int16_t* counts, hipStream_t stream) {

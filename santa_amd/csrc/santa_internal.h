@@ -89,6 +89,8 @@ bool small_pass(long long kv_tiles, int GH);
 // resident rounds (a quarter of one at GH 8); the launch, the workspace plan and
 // the bench label all decide with this one function.
 bool uniform_small_pass(int B, int KVH, int T_c, int GH);
+// Whether a uniform flash call at block_n 32 / 64 runs the strip kernel.
+bool uniform_strips(int B, int KVH, int T_c, int GH, int block_n);
 bool small_prop_pass(long long kv_tiles);
 // santa_prop's pass 1 on the wave kernel (block_n 256: the vec path at GH 4,
 // the general path at GH 8); it writes the tile-major stash when given a
