@@ -106,9 +106,13 @@ class _FusedOps:
         if rc != 0:
             raise RuntimeError(cls.lib().santa_last_error().decode())
 
-    @staticmethod
-    def _stream(t: torch.Tensor):
-        return torch.cuda.current_stream(t.device).cuda_stream
+    @classmethod
+    def _launch(cls, t: torch.Tensor, fn: str, *args):
+        """santa_rt_<fn>(*args, stream) on t's device and its current stream,
+        with that device current: a default stream is 0, which the runtime
+        takes as the current device's."""
+        with torch.cuda.device(t.device):
+            cls._check(getattr(cls.lib(), "santa_rt_" + fn)(*args, torch.cuda.current_stream(t.device).cuda_stream))
 
     @classmethod
     def add_rms_norm(cls, h: torch.Tensor, a: Optional[torch.Tensor], w: torch.Tensor, eps: float) -> torch.Tensor:
@@ -116,8 +120,8 @@ class _FusedOps:
         assert h.is_contiguous() and h.dtype == torch.bfloat16 and (a is None or a.is_contiguous())
         x = torch.empty_like(h)
         rows, hidden = h.numel() // h.shape[-1], h.shape[-1]
-        cls._check(cls.lib().santa_rt_add_rms_norm(h.data_ptr(), a.data_ptr() if a is not None else None,
-                                                   w.data_ptr(), x.data_ptr(), rows, hidden, eps, cls._stream(h)))
+        cls._launch(h, "add_rms_norm", h.data_ptr(), a.data_ptr() if a is not None else None, w.data_ptr(),
+                    x.data_ptr(), rows, hidden, eps)
         return x
 
     @classmethod
@@ -128,9 +132,8 @@ class _FusedOps:
         B = qkv.shape[0]
         q = torch.empty(B, heads, head_dim, dtype=qkv.dtype, device=qkv.device)
         kc, vc = cache.k[layer], cache.v[layer]
-        cls._check(cls.lib().santa_rt_rope_write(qkv.data_ptr(), cos.data_ptr(), sin.data_ptr(), q.data_ptr(),
-                                                 kc.data_ptr(), vc.data_ptr(), B, heads, kv_heads, head_dim,
-                                                 kc.shape[1], pos, cls._stream(qkv)))
+        cls._launch(qkv, "rope_write", qkv.data_ptr(), cos.data_ptr(), sin.data_ptr(), q.data_ptr(), kc.data_ptr(),
+                    vc.data_ptr(), B, heads, kv_heads, head_dim, kc.shape[1], pos)
         return q
 
     @classmethod
@@ -138,8 +141,7 @@ class _FusedOps:
         """_rope_cos_sin of one position in bf16, cos and sin [head_dim] on
         like's device."""
         t = torch.empty(2, head_dim, dtype=torch.bfloat16, device=like.device)
-        cls._check(cls.lib().santa_rt_rope_table(pos, theta, head_dim, t[0].data_ptr(), t[1].data_ptr(),
-                                                 cls._stream(t)))
+        cls._launch(t, "rope_table", pos, theta, head_dim, t[0].data_ptr(), t[1].data_ptr())
         return t[0], t[1]
 
     @classmethod
@@ -150,9 +152,8 @@ class _FusedOps:
         assert qkv.is_contiguous() and cos.is_contiguous() and sin.is_contiguous()
         B, P = qkv.shape[:2]
         q = torch.empty(B, P, heads, head_dim, dtype=qkv.dtype, device=qkv.device)
-        cls._check(cls.lib().santa_rt_rope_write_rows(qkv.data_ptr(), cos.data_ptr(), sin.data_ptr(), q.data_ptr(),
-                                                      k_cache.data_ptr(), v_cache.data_ptr(), B, P, heads, kv_heads,
-                                                      head_dim, k_cache.shape[1], 0, cls._stream(qkv)))
+        cls._launch(qkv, "rope_write_rows", qkv.data_ptr(), cos.data_ptr(), sin.data_ptr(), q.data_ptr(),
+                    k_cache.data_ptr(), v_cache.data_ptr(), B, P, heads, kv_heads, head_dim, k_cache.shape[1], 0)
         return q
 
     @staticmethod
@@ -176,8 +177,7 @@ class _FusedOps:
             return cls.silu_mul(y) if swiglu else y
         N = w.shape[0] // 2 if swiglu else w.shape[0]
         y = torch.empty(*x.shape[:-1], N, dtype=x.dtype, device=x.device)
-        cls._check(cls.lib().santa_rt_linear(x.data_ptr(), w.data_ptr(), y.data_ptr(), rows, N, K, int(swiglu),
-                                             cls._stream(x)))
+        cls._launch(x, "linear", x.data_ptr(), w.data_ptr(), y.data_ptr(), rows, N, K, int(swiglu))
         return y
 
     @classmethod
@@ -189,8 +189,7 @@ class _FusedOps:
                 and x.is_contiguous() and w.is_contiguous() and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0):
             return F.linear(x, w).float()
         y = torch.empty(rows, w.shape[0], dtype=torch.float32, device=x.device)
-        cls._check(cls.lib().santa_rt_linear_f32(x.data_ptr(), w.data_ptr(), y.data_ptr(), rows, w.shape[0], K,
-                                                 cls._stream(x)))
+        cls._launch(x, "linear_f32", x.data_ptr(), w.data_ptr(), y.data_ptr(), rows, w.shape[0], K)
         return y
 
     @classmethod
@@ -206,9 +205,8 @@ class _FusedOps:
             return cls.rope_write(cls.linear(x, w), cos, sin, cache, layer, pos, heads, kv_heads, head_dim)
         q = torch.empty(B, heads, head_dim, dtype=x.dtype, device=x.device)
         kc, vc = cache.k[layer], cache.v[layer]
-        cls._check(cls.lib().santa_rt_linear_rope(x.data_ptr(), w.data_ptr(), B, K, cos.data_ptr(), sin.data_ptr(),
-                                                  q.data_ptr(), kc.data_ptr(), vc.data_ptr(), heads, kv_heads,
-                                                  head_dim, kc.shape[1], pos, cls._stream(x)))
+        cls._launch(x, "linear_rope", x.data_ptr(), w.data_ptr(), B, K, cos.data_ptr(), sin.data_ptr(), q.data_ptr(),
+                    kc.data_ptr(), vc.data_ptr(), heads, kv_heads, head_dim, kc.shape[1], pos)
         return q
 
     @classmethod
@@ -218,7 +216,7 @@ class _FusedOps:
         n = logits.shape[-1]
         rows = logits.numel() // n
         out = torch.empty(logits.shape[:-1], dtype=torch.int64, device=logits.device)
-        cls._check(cls.lib().santa_rt_argmax(logits.data_ptr(), rows, n, out.data_ptr(), cls._stream(logits)))
+        cls._launch(logits, "argmax", logits.data_ptr(), rows, n, out.data_ptr())
         return out
 
     @staticmethod
@@ -237,10 +235,8 @@ class _FusedOps:
         B, P, H, D = q.shape
         out = torch.empty(B, P, H, D, dtype=q.dtype, device=q.device)
         strides = (ctypes.c_longlong * 12)(*(s for t in (q, k, v, out) for s in t.stride()[:3]))
-        with torch.cuda.device(q.device):
-            cls._check(cls.lib().santa_rt_causal_attention(
-                q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), int(q.dtype == torch.float16), B, P, H,
-                k.shape[2], D, strides, cls._stream(q)))
+        cls._launch(q, "causal_attention", q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
+                    int(q.dtype == torch.float16), B, P, H, k.shape[2], D, strides)
         return out
 
     @classmethod
@@ -254,13 +250,11 @@ class _FusedOps:
         KVH = k.shape[2]
         out = torch.empty(B, H, D, dtype=q.dtype, device=q.device)
         strides = (ctypes.c_longlong * 6)(*(s for t in (k, v) for s in t.stride()[:3]))
-        lib = cls.lib()
-        with torch.cuda.device(q.device):
-            ws = torch.empty(lib.santa_rt_exact_decode_workspace_size(B, L, H, KVH), dtype=torch.uint8,
+        with torch.cuda.device(q.device):  # the plan asks for the device's CUs
+            ws = torch.empty(cls.lib().santa_rt_exact_decode_workspace_size(B, L, H, KVH), dtype=torch.uint8,
                              device=q.device)
-            cls._check(lib.santa_rt_exact_decode(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
-                                                 int(q.dtype == torch.float16), B, L, H, KVH, D, strides,
-                                                 ws.data_ptr(), ws.numel(), cls._stream(q)))
+        cls._launch(q, "exact_decode", q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
+                    int(q.dtype == torch.float16), B, L, H, KVH, D, strides, ws.data_ptr(), ws.numel())
         return out
 
     @classmethod
@@ -269,7 +263,7 @@ class _FusedOps:
         inter = gu.shape[-1] // 2
         rows = gu.numel() // gu.shape[-1]
         out = torch.empty(*gu.shape[:-1], inter, dtype=gu.dtype, device=gu.device)
-        cls._check(cls.lib().santa_rt_silu_mul(gu.data_ptr(), out.data_ptr(), rows, inter, cls._stream(gu)))
+        cls._launch(gu, "silu_mul", gu.data_ptr(), out.data_ptr(), rows, inter)
         return out
 
 
