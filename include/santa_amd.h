@@ -289,14 +289,15 @@ int santa_prop_decode_paged(const void* q, const void* K_pages, const void* V_pa
  * tutorial_code/runtime_common.py:501-571): q [B, P, H, D], k, v [B, P, KVH,
  * D], out [B, P, H, D] of one 16-bit type (enum santa_dtype); strides: 12 host
  * values, the batch, position and head strides in elements of q, k, v, out
- * (multiples of 8, the last dimension contiguous, the tensors 16-byte
- * aligned).  Scores, softmax and sums in float32, the probabilities rounded
+ * (multiples of 8, positions at least D apart, the last dimension contiguous,
+ * the tensors 16-byte aligned).  Scores, softmax and sums in float32, the probabilities rounded
  * to the 16-bit type for the second product.
  * santa_rt_exact_decode: exact decode attention in float32, D = 128: q, out
  * [B, H, D] contiguous, k, v [B, L.., KVH, D] of which the first L positions
  * count, one 16-bit type (enum santa_dtype); strides: 6 host values, the
- * batch, position and head strides in elements of k and v (multiples of 8, the
- * last dimension contiguous, the tensors 16-byte aligned).  workspace:
+ * batch, position and head strides in elements of k and v (multiples of 8,
+ * positions at least D apart, the last dimension contiguous, the tensors
+ * 16-byte aligned).  workspace:
  * santa_rt_exact_decode_workspace_size bytes, 16-byte aligned, needing no
  * initialization.
  * santa_rt_argmax: out[r] (int64) = the index of the maximum of row r of

@@ -220,21 +220,31 @@ class _FusedOps:
         return out
 
     @staticmethod
-    def _attention_strides_fit(t: torch.Tensor) -> bool:
-        """Whether the attention kernels can address t [..., heads, 128]:
-        last dimension contiguous, the other strides multiples of 8 elements,
-        16-byte aligned storage."""
-        return (t.stride(-1) == 1 and all(s % 8 == 0 and s < 1 << 24 for s in t.stride()[1:-1])
-                and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0)
+    def _attention_operand(t: torch.Tensor):
+        """t [B, P, heads, 128] as the attention kernels address it, with its
+        batch, position and head strides: last dimension contiguous, strides
+        of whole 16-byte pieces, positions at least a row apart (the kernels
+        tell rows past the end by their offset) and less than 2^24 elements,
+        16-byte aligned; a packed copy where t is laid out otherwise.  A
+        dimension of size 1 counts as packed: its stride is never used and
+        can be any number, also in a tensor that is_contiguous."""
+        def strides(x):
+            packed = (x.shape[1] * x.shape[2] * 128, x.shape[2] * 128, 128)
+            return [d if n == 1 else s for n, s, d in zip(x.shape, x.stride(), packed)]
+
+        st = strides(t)
+        if t.stride(3) != 1 or any(s % 8 for s in st) or not 128 <= st[1] < 1 << 24 or t.data_ptr() % 16:
+            t = torch.empty(t.shape, dtype=t.dtype, device=t.device).copy_(t)
+            st = strides(t)
+        return t, st
 
     @classmethod
     def causal_attention(cls, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> torch.Tensor:
         """causal_attention of [B, P, heads, 128] tensors as one kernel."""
-        q, k, v = (t if cls._attention_strides_fit(t) else t.contiguous() for t in (q, k, v))
-        q, k, v = (t if t.data_ptr() % 16 == 0 else t.clone() for t in (q, k, v))
         B, P, H, D = q.shape
         out = torch.empty(B, P, H, D, dtype=q.dtype, device=q.device)
-        strides = (ctypes.c_longlong * 12)(*(s for t in (q, k, v, out) for s in t.stride()[:3]))
+        (q, sq), (k, sk), (v, sv) = (cls._attention_operand(t) for t in (q, k, v))
+        strides = (ctypes.c_longlong * 12)(*sq, *sk, *sv, *out.stride()[:3])
         cls._launch(q, "causal_attention", q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
                     int(q.dtype == torch.float16), B, P, H, k.shape[2], D, strides)
         return out
@@ -244,12 +254,12 @@ class _FusedOps:
         """Exact float32 attention of q [B, H, 128] over the first L positions
         of k, v [B, T, KVH, 128]."""
         q = q.contiguous()
-        k, v = (t if cls._attention_strides_fit(t) else t[:, :L].contiguous() for t in (k, v))
-        q, k, v = (t if t.data_ptr() % 16 == 0 else t.clone() for t in (q, k, v))
+        q = q if q.data_ptr() % 16 == 0 else q.clone()
+        (k, sk), (v, sv) = (cls._attention_operand(t[:, :L]) for t in (k, v))
         B, H, D = q.shape
         KVH = k.shape[2]
         out = torch.empty(B, H, D, dtype=q.dtype, device=q.device)
-        strides = (ctypes.c_longlong * 6)(*(s for t in (k, v) for s in t.stride()[:3]))
+        strides = (ctypes.c_longlong * 6)(*sk, *sv)
         with torch.cuda.device(q.device):  # the plan asks for the device's CUs
             ws = torch.empty(cls.lib().santa_rt_exact_decode_workspace_size(B, L, H, KVH), dtype=torch.uint8,
                              device=q.device)
@@ -299,11 +309,12 @@ def _plain(*ts: torch.Tensor) -> bool:
 def _attention_kernel_takes(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> bool:
     """Whether the library's attention kernels take q [.., H, D] with k, v
     [B, T, KVH, D]: bf16 or f16 tensors of head_dim 128 on one GPU, whole
-    groups of query heads."""
+    groups of query heads (fewer than 2^17, so that a packed position's
+    stride is one the kernels take)."""
     return (q.is_cuda and q.dtype in (torch.bfloat16, torch.float16) and k.dtype == q.dtype and v.dtype == q.dtype
             and k.device == q.device and v.device == q.device and k.dim() == 4 and k.shape == v.shape
             and q.shape[-1] == 128 and k.shape[-1] == 128 and k.shape[0] == q.shape[0] and q.numel() > 0
-            and k.shape[2] > 0 and q.shape[-2] % k.shape[2] == 0 and _plain(q, k, v))
+            and k.shape[2] > 0 and q.shape[-2] % k.shape[2] == 0 and q.shape[-2] < 1 << 17 and _plain(q, k, v))
 
 
 def causal_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, chunk: int = 512) -> torch.Tensor:

@@ -75,6 +75,28 @@ def test_causal_attention_strided():
     _check(causal_attention(q.transpose(2, 3).contiguous().transpose(2, 3), k, v), want, v, torch.bfloat16)
 
 
+def test_attention_size_one_dimensions():
+    """Strides of size-1 dimensions that are no multiple of 8, which torch
+    leaves as they are in a tensor that counts as contiguous: one KV head with
+    head stride 1, a batch of one cut from wider rows, a single position; and
+    one position repeated, whose infinite values must not reach the rows past
+    the end."""
+    print("\n[case] attention on size-1 dimensions of odd strides", flush=True)
+    g = torch.Generator().manual_seed(6)
+    P, bf = 70, torch.bfloat16
+    one_head = torch.randn(1, P, 128, 1, generator=g).to("cuda", bf).transpose(2, 3)
+    packed = torch.randn(2, P * 256 + 4, generator=g).to("cuda", bf)[:, :P * 256].view(2, P, 2, 128)[:1]
+    for k in (one_head, packed, packed[:, :1]):
+        n, KVH = k.shape[1:3]
+        q = torch.randn(1, n, 4 * KVH, 128, generator=g).to("cuda", bf)
+        _check(causal_attention(q, k, k), _ref(q, k, k), k, bf)
+        _check_decode(ExactDecodeBackend().decode(q[:, -1], k, k, n), _ref_decode(q[:, -1], k, k, n), k, bf)
+    same = torch.randn(1, 1, 1, 128, generator=g).to("cuda", bf)
+    same[..., 7] = math.inf
+    k, v = torch.zeros(1, 9, 1, 128, device="cuda", dtype=bf), same.expand(1, 9, 1, 128)
+    assert torch.equal(ExactDecodeBackend().decode(k[:, 0], k, v, 9)[0, 0].isinf(), same[0, 0, 0].isinf())
+
+
 def test_causal_attention_large_scores():
     """Scores of several hundred, growing with the position: the running
     maximum moves in every tile and the early sums are rescaled to nothing."""

@@ -3,6 +3,7 @@ launched, on the CPU: the library is replaced by a recorder, so nothing here
 needs a GPU.
 """
 import contextlib
+import ctypes
 
 import pytest
 import torch
@@ -14,14 +15,14 @@ BF = torch.bfloat16
 
 
 class _Recorder:
-    """A library whose functions only note the device that is current."""
+    """A library whose functions only note their arguments and the device that is current."""
 
     def __init__(self, current):
         self.current, self.calls = current, []
 
     def __getattr__(self, name):
         def fn(*args):
-            self.calls.append((name, self.current[-1]))
+            self.calls.append((name, self.current[-1], args))
             return 0
 
         return fn
@@ -75,5 +76,50 @@ def test_launches_on_the_tensors_device(op, recorder):
     stream is 0, which the runtime takes as the current device's."""
     _ops()[op]()
     launches = [c for c in recorder.calls if not c[0].endswith("workspace_size")]
-    assert [name for name, _ in launches] == ["santa_rt_" + op]
+    assert [c[0] for c in launches] == ["santa_rt_" + op]
     assert launches[0][1] == torch.device("cpu")
+
+
+def _operands():
+    """(name, k of shape [B, P, heads, 128]): layouts the kernels cannot address
+    as they are, or only because a stride belongs to a dimension of size 1."""
+    one_head = torch.randn(1, 5, 128, 1, dtype=BF).transpose(2, 3)  # head stride 1
+    packed = torch.randn(3, 5 * 2 * 128 + 4, dtype=BF)[:, :5 * 2 * 128].view(3, 5, 2, 128)[:1]  # batch stride 1284
+    row = torch.randn(2, 3, 2 * 128 + 4, dtype=BF)[..., :256].view(2, 3, 2, 128)[:1, :1]  # 780, 260
+    far = torch.randn(128, dtype=BF).as_strided((1, 1, 1, 128), (3, 1 << 25, 5, 1))  # a position stride above the limit
+    swapped = torch.randn(2, 5, 128, 2, dtype=BF).transpose(2, 3)  # last dimension not contiguous
+    ragged = torch.randn(2, 5 * 2 * 128 + 4, dtype=BF)[:, :5 * 2 * 128].view(2, 5, 2, 128)  # batch stride 1284, B 2
+    odd = torch.randn(5 * 2 * 128 + 1, dtype=BF)[1:].view(1, 5, 2, 128)  # 2 bytes off
+    expanded = torch.randn(1, 5, 1, 128, dtype=BF).expand(2, 5, 3, 128)
+    same = torch.randn(2, 1, 3, 128, dtype=BF).expand(2, 5, 3, 128)  # one position for all
+    return {"one head": one_head, "packed batch of one": packed, "single row": row, "far position": far,
+            "swapped": swapped, "ragged batch": ragged, "odd address": odd, "expanded": expanded,
+            "same positions": same}
+
+
+def _rows(ptr, shape, strides):
+    """The 256-byte rows [B, P, heads] of a 16-bit tensor at ptr."""
+    return [ctypes.string_at(ptr + 2 * (b * strides[0] + p * strides[1] + h * strides[2]), 256)
+            for b in range(shape[0]) for p in range(shape[1]) for h in range(shape[2])]
+
+
+@pytest.mark.parametrize("name", sorted(_operands()))
+def test_attention_operands_fit_the_kernels(name, recorder):
+    """Whatever the layout, the strides and the address passed on are ones the
+    kernels take (multiples of 8 elements, positions at least a row apart and
+    below 2^24, 16-byte aligned) and lead to the same values."""
+    k = _operands()[name]
+    B, P, KVH, D = k.shape
+    q = torch.randn(B, P, 2 * KVH, D, dtype=BF)
+    dense = torch.empty(k.shape, dtype=BF).copy_(k)
+    want = _rows(dense.data_ptr(), k.shape, (P * KVH * D, KVH * D, D))
+
+    def check(ptr, strides):
+        assert ptr % 16 == 0 and all(s >= 0 and s % 8 == 0 for s in strides) and 128 <= strides[1] < 1 << 24
+        assert _rows(ptr, k.shape, strides) == want
+        return 0
+
+    recorder.santa_rt_causal_attention = lambda *a: check(a[1], a[10][3:6]) or check(a[2], a[10][6:9])
+    recorder.santa_rt_exact_decode = lambda *a: check(a[1], a[10][:3]) or check(a[2], a[10][3:6])
+    _FusedOps.causal_attention(q, k, k)
+    _FusedOps.exact_decode(q[:, 0], k, k, P)
