@@ -117,7 +117,8 @@ class _FusedOps:
     @classmethod
     def add_rms_norm(cls, h: torch.Tensor, a: Optional[torch.Tensor], w: torch.Tensor, eps: float) -> torch.Tensor:
         """h += a (in place, bf16) when a is given; returns rms_norm(h) * w."""
-        assert h.is_contiguous() and h.dtype == torch.bfloat16 and (a is None or a.is_contiguous())
+        assert h.is_contiguous() and (a is None or a.is_contiguous())
+        assert all(t is None or t.dtype == torch.bfloat16 for t in (h, a, w))
         x = torch.empty_like(h)
         rows, hidden = h.numel() // h.shape[-1], h.shape[-1]
         cls._launch(h, "add_rms_norm", h.data_ptr(), a.data_ptr() if a is not None else None, w.data_ptr(),
@@ -129,9 +130,10 @@ class _FusedOps:
                    pos: int, heads: int, kv_heads: int, head_dim: int) -> torch.Tensor:
         """q rotated ([B, H, D]); k rotated and v written to the caches at pos."""
         assert qkv.is_contiguous() and cos.is_contiguous() and sin.is_contiguous()
+        kc, vc = cache.k[layer], cache.v[layer]
+        assert all(t.dtype == torch.bfloat16 for t in (qkv, cos, sin, kc, vc))
         B = qkv.shape[0]
         q = torch.empty(B, heads, head_dim, dtype=qkv.dtype, device=qkv.device)
-        kc, vc = cache.k[layer], cache.v[layer]
         cls._launch(qkv, "rope_write", qkv.data_ptr(), cos.data_ptr(), sin.data_ptr(), q.data_ptr(), kc.data_ptr(),
                     vc.data_ptr(), B, heads, kv_heads, head_dim, kc.shape[1], pos)
         return q
@@ -150,6 +152,7 @@ class _FusedOps:
         """rope_write for the positions 0 .. P-1 of a prefill: qkv [B, P, ...],
         cos and sin [P, head_dim]; q rotated ([B, P, H, D]) returned."""
         assert qkv.is_contiguous() and cos.is_contiguous() and sin.is_contiguous()
+        assert all(t.dtype == torch.bfloat16 for t in (qkv, cos, sin, k_cache, v_cache))
         B, P = qkv.shape[:2]
         q = torch.empty(B, P, heads, head_dim, dtype=qkv.dtype, device=qkv.device)
         cls._launch(qkv, "rope_write_rows", qkv.data_ptr(), cos.data_ptr(), sin.data_ptr(), q.data_ptr(),
@@ -164,6 +167,12 @@ class _FusedOps:
         mp = 1 if rows <= 1 else 2 if rows <= 2 else 4 if rows <= 4 else 8
         return 1 <= rows <= 8 and K % 8 == 0 and mp * (-(-K // 2048) * 2048) <= 65536
 
+    @staticmethod
+    def _product(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+        """F.linear in x's type, also under autocast (as the kernel it stands in for)."""
+        with torch.autocast(x.device.type, enabled=False):
+            return F.linear(x, w)
+
     @classmethod
     def linear(cls, x: torch.Tensor, w: torch.Tensor, *, swiglu: bool = False) -> torch.Tensor:
         """bf16(x @ w.T) for few rows of x (santa_rt_linear; F.linear where
@@ -173,7 +182,7 @@ class _FusedOps:
         rows, K = x.numel() // x.shape[-1], x.shape[-1]
         if not (cls.linear_fits(rows, K) and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
                 and x.is_contiguous() and w.is_contiguous() and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0):
-            y = F.linear(x, w)
+            y = cls._product(x, w)
             return cls.silu_mul(y) if swiglu else y
         N = w.shape[0] // 2 if swiglu else w.shape[0]
         y = torch.empty(*x.shape[:-1], N, dtype=x.dtype, device=x.device)
@@ -187,7 +196,7 @@ class _FusedOps:
         rows, K = x.shape
         if not (cls.linear_fits(rows, K) and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
                 and x.is_contiguous() and w.is_contiguous() and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0):
-            return F.linear(x, w).float()
+            return cls._product(x, w).float()
         y = torch.empty(rows, w.shape[0], dtype=torch.float32, device=x.device)
         cls._launch(x, "linear_f32", x.data_ptr(), w.data_ptr(), y.data_ptr(), rows, w.shape[0], K)
         return y
@@ -203,8 +212,9 @@ class _FusedOps:
                 and x.is_contiguous() and w.is_contiguous() and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
                 and cos.is_contiguous() and sin.is_contiguous() and head_dim % 2 == 0):
             return cls.rope_write(cls.linear(x, w), cos, sin, cache, layer, pos, heads, kv_heads, head_dim)
-        q = torch.empty(B, heads, head_dim, dtype=x.dtype, device=x.device)
         kc, vc = cache.k[layer], cache.v[layer]
+        assert all(t.dtype == torch.bfloat16 for t in (cos, sin, kc, vc))
+        q = torch.empty(B, heads, head_dim, dtype=x.dtype, device=x.device)
         cls._launch(x, "linear_rope", x.data_ptr(), w.data_ptr(), B, K, cos.data_ptr(), sin.data_ptr(), q.data_ptr(),
                     kc.data_ptr(), vc.data_ptr(), heads, kv_heads, head_dim, kc.shape[1], pos)
         return q
@@ -269,7 +279,7 @@ class _FusedOps:
 
     @classmethod
     def silu_mul(cls, gu: torch.Tensor) -> torch.Tensor:
-        assert gu.is_contiguous()
+        assert gu.is_contiguous() and gu.dtype == torch.bfloat16
         inter = gu.shape[-1] // 2
         rows = gu.numel() // gu.shape[-1]
         out = torch.empty(*gu.shape[:-1], inter, dtype=gu.dtype, device=gu.device)
@@ -296,11 +306,13 @@ def _apply_rope(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.
 
 def _plain(*ts: torch.Tensor) -> bool:
     """Ordinary tensors outside autograd, forward-mode differentiation,
-    functorch transforms and tracing: what a kernel behind raw pointers may
-    take in place of torch operations."""
+    functorch transforms, tracing and autocast to another type: what a kernel
+    behind raw pointers may take in place of torch operations."""
     if torch.is_grad_enabled() and any(t.requires_grad for t in ts):
         return False
     if torch.compiler.is_compiling() or torch.jit.is_tracing():
+        return False
+    if torch.is_autocast_enabled("cuda") and any(t.dtype != torch.get_autocast_dtype("cuda") for t in ts):
         return False
     return all(type(t) is torch.Tensor and not torch._C._functorch.is_functorch_wrapped_tensor(t)
                and (fwAD._current_level < 0 or fwAD.unpack_dual(t).tangent is None) for t in ts)

@@ -9,7 +9,7 @@ import pytest
 import torch
 
 from santa_amd import runtime
-from santa_amd.runtime import LlamaShape, NHDCache, _FusedOps
+from santa_amd.runtime import LlamaShape, NHDCache, _FusedOps, _plain
 
 BF = torch.bfloat16
 
@@ -123,3 +123,43 @@ def test_attention_operands_fit_the_kernels(name, recorder):
     recorder.santa_rt_exact_decode = lambda *a: check(a[1], a[10][:3]) or check(a[2], a[10][3:6])
     _FusedOps.causal_attention(q, k, k)
     _FusedOps.exact_decode(q[:, 0], k, k, P)
+
+
+@contextlib.contextmanager
+def _autocast(dtype):
+    """torch.autocast("cuda", dtype) without a GPU, where it switches itself off."""
+    kept = torch.is_autocast_enabled("cuda"), torch.get_autocast_dtype("cuda")
+    torch.set_autocast_enabled("cuda", True)
+    torch.set_autocast_dtype("cuda", dtype)
+    try:
+        yield
+    finally:
+        torch.set_autocast_enabled("cuda", kept[0])
+        torch.set_autocast_dtype("cuda", kept[1])
+
+
+def test_autocast_to_another_type_is_not_plain():
+    """Under autocast the torch products change type; a kernel's operands would not."""
+    t = torch.ones(2, dtype=BF)
+    assert _plain(t)
+    with _autocast(torch.float16):
+        assert not _plain(t) and _plain(t.half()) and not _plain(t.half(), t)
+    with _autocast(BF):
+        assert _plain(t) and not _plain(t.half())
+
+
+@pytest.mark.parametrize("op", ["add_rms_norm", "rope_write", "rope_write_rows", "silu_mul"])
+def test_kernels_refuse_another_type(op, recorder):
+    """float16 bits are never read as bf16."""
+    x, cs = torch.ones(2, 64, dtype=BF), torch.ones(2, 16, dtype=BF)
+    cache = NHDCache(LlamaShape(hidden=32, intermediate=8, heads=2, kv_heads=1, layers=1, vocab=8), 1, 4, BF, "cpu")
+    with pytest.raises(AssertionError):
+        if op == "add_rms_norm":
+            _FusedOps.add_rms_norm(x, x.half(), x[0], 1e-5)
+        elif op == "rope_write":
+            _FusedOps.rope_write(x[:1].half(), cs[0], cs[0], cache, 0, 1, 2, 1, 16)
+        elif op == "rope_write_rows":
+            _FusedOps.rope_write_rows(x[None].half(), cs, cs, cache.k[0], cache.v[0], 2, 1, 16)
+        else:
+            _FusedOps.silu_mul(x.half())
+    assert not recorder.calls

@@ -62,6 +62,45 @@ def test_fused_prefill_matches_torch_expressions(B, P, mlp_chunk, monkeypatch):
     assert not fused.k[0][:, P:].any() and not fused.v[1][:, P:].any()
 
 
+def test_prefill_and_step_under_autocast():
+    """Autocast to float16, torch's default on a GPU: the prefill is the torch
+    expressions under the same autocast, and a step of more sequences than the
+    few-row product takes stays the step without autocast (its products beside
+    that kernel are torch's)."""
+    print("\n[case] prefill and a step of nine sequences under autocast", flush=True)
+    dev = torch.device("cuda:0")
+    model = RandomLlama(SMALL, seed=7, std=0.05, device=dev)
+    toks = torch.randint(0, SMALL.vocab, (9, 20), generator=torch.Generator().manual_seed(8)).to(dev)
+    cast, want, plain = (NHDCache(SMALL, 9, 22, torch.bfloat16, dev) for _ in range(3))
+    ref = model.prefill(toks, plain)
+    with torch.autocast("cuda"):
+        got = model.prefill(toks, cast)
+        with pytest.MonkeyPatch.context() as mp:
+            mp.setattr(RandomLlama, "_fused_prefill_takes", lambda self, h, cache: False)
+            torch_path = model.prefill(toks, want)
+    torch.cuda.synchronize()
+    for a, b, c in [(got, torch_path, ref)] + list(zip(cast.k + cast.v, want.k + want.v, plain.k + plain.v)):
+        assert torch.equal(a, b)
+        a, c = a.float(), c.float()
+        # float16 products keep three bits more than bf16's: a few bf16 units apart through two layers
+        assert (a - c).abs().max() <= 8 * 2.0 ** -8 * c.abs().max()
+    nxt = torch.argmax(ref, -1)
+    other = plain.clone()
+    step = model.decode_step(nxt, 20, plain, ExactDecodeBackend())
+    with torch.autocast("cuda"):
+        same = model.decode_step(nxt, 20, other, _NoAutocast())
+    torch.cuda.synchronize()
+    assert torch.equal(step, same) and all(torch.equal(a, b) for a, b in zip(plain.k + plain.v, other.k + other.v))
+
+
+class _NoAutocast(ExactDecodeBackend):
+    """The exact backend outside the step's autocast (its torch form would be cast)."""
+
+    def decode(self, *args):
+        with torch.autocast("cuda", enabled=False):
+            return super().decode(*args)
+
+
 def test_santa_backends_in_the_decode_loop():
     print("\n[case] runtime santa_flash (large S) and santa_prop vs exact, P=700 B=2", flush=True)
     model, toks, cache, logits = _setup()
