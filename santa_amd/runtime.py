@@ -306,11 +306,12 @@ def _apply_rope(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.
 
 def _plain(*ts: torch.Tensor) -> bool:
     """Ordinary tensors outside autograd, forward-mode differentiation,
-    functorch transforms, tracing and autocast to another type: what a kernel
-    behind raw pointers may take in place of torch operations."""
+    functorch transforms, tracing, dispatch modes (which see every torch
+    operation) and autocast to another type: what a kernel behind raw pointers
+    may take in place of torch operations."""
     if torch.is_grad_enabled() and any(t.requires_grad for t in ts):
         return False
-    if torch.compiler.is_compiling() or torch.jit.is_tracing():
+    if torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() > 0:
         return False
     if torch.is_autocast_enabled("cuda") and any(t.dtype != torch.get_autocast_dtype("cuda") for t in ts):
         return False

@@ -7,6 +7,10 @@ import ctypes
 
 import pytest
 import torch
+import torch.autograd.forward_ad as fwAD
+from torch._subclasses.fake_tensor import FakeTensorMode
+from torch.fx.experimental.proxy_tensor import make_fx
+from torch.utils.flop_counter import FlopCounterMode
 
 from santa_amd import runtime
 from santa_amd.runtime import LlamaShape, NHDCache, _FusedOps, _plain
@@ -163,3 +167,25 @@ def test_kernels_refuse_another_type(op, recorder):
         else:
             _FusedOps.silu_mul(x.half())
     assert not recorder.calls
+
+
+def test_only_ordinary_calls_are_plain():
+    """What a kernel behind raw pointers would drop or hide: gradients, tangents,
+    transforms, and operations recorded by a dispatch mode."""
+    t = torch.ones(2, 3, dtype=BF)
+    leaf = t.clone().requires_grad_()
+    assert _plain(t) and not _plain(t, leaf)
+    with torch.no_grad():
+        assert _plain(leaf)
+    with fwAD.dual_level():
+        dual = fwAD.make_dual(t, t)
+        assert _plain(t) and not _plain(dual)
+    seen = []
+    torch.vmap(lambda x: seen.append(_plain(x)) or x)(t)
+    torch.func.jvp(lambda x: seen.append(_plain(x)) or x, (t,), (t,))
+    make_fx(lambda x: seen.append(_plain(x)) or x * 2)(t)  # records what is run on ordinary tensors
+    with FakeTensorMode():
+        seen.append(_plain(torch.empty(2, dtype=BF)))
+    with FlopCounterMode(display=False):
+        seen.append(_plain(t))
+    assert seen == [False] * 5 and _plain(t)
