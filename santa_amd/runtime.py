@@ -521,7 +521,7 @@ class RandomLlama:
         s, D = self.shape, self.shape.head_dim
         B, P = h.shape[:2]
         h, cos, sin = h.contiguous(), cos.contiguous(), sin.contiguous()
-        x = _FusedOps.add_rms_norm(h, None, self.layers[0]["ln1"], s.rms_eps)
+        x = _FusedOps.add_rms_norm(h, None, self.layers[0]["ln1"] if self.layers else self.norm, s.rms_eps)
         rows = mlp_chunk * B
         for li, L in enumerate(self.layers):
             q = _FusedOps.rope_write_rows(F.linear(x, L["wqkv"]), cos, sin, cache.k[li], cache.v[li], s.heads,
@@ -573,7 +573,7 @@ class RandomLlama:
         s, D = self.shape, self.shape.head_dim
         B = h.shape[0]
         h = h.contiguous()
-        x = _FusedOps.add_rms_norm(h, None, self.layers[0]["ln1"], s.rms_eps)
+        x = _FusedOps.add_rms_norm(h, None, self.layers[0]["ln1"] if self.layers else self.norm, s.rms_eps)
         lin = _FusedOps.linear
         for li, L in enumerate(self.layers):
             q = _FusedOps.linear_rope(x, L["wqkv"], cos, sin, cache, li, pos, s.heads, s.kv_heads, D)

@@ -9,8 +9,11 @@ head_dim 128 and 4 query heads per KV head).
 
 Every case prints its name before touching the GPU.
 """
+from dataclasses import replace
+
 import pytest
 import torch
+import torch.nn.functional as F
 
 from santa_amd import attention_backends as ab
 from santa_amd.runtime import ExactDecodeBackend, LlamaShape, NHDCache, RandomLlama, decode_deviation, greedy_decode
@@ -60,6 +63,23 @@ def test_fused_prefill_matches_torch_expressions(B, P, mlp_chunk, monkeypatch):
         assert (a - b).abs().max() <= 8 * 2.0 ** -8 * b.abs().max(), ((a - b).abs().max(), b.abs().max())
         assert (a - b).norm() <= 2.0 ** -6 * b.norm()
     assert not fused.k[0][:, P:].any() and not fused.v[1][:, P:].any()
+
+
+def test_model_without_layers():
+    """Embedding, final norm and head: the prefill's logits are the step's."""
+    print("\n[case] prefill and step of a model without layers", flush=True)
+    dev, shape = torch.device("cuda:0"), replace(SMALL, layers=0)
+    model = RandomLlama(shape, seed=7, std=0.05, device=dev)
+    toks = torch.randint(0, shape.vocab, (2, 5), generator=torch.Generator().manual_seed(9)).to(dev)
+    cache = NHDCache(shape, 2, 8, torch.bfloat16, dev)
+    got = model.prefill(toks, cache)
+    torch.cuda.synchronize()
+    h = model.embed[toks[:, -1]].float()
+    want = F.linear((h * torch.rsqrt(h.pow(2).mean(-1, keepdim=True) + shape.rms_eps)).bfloat16().float(),
+                    model.lm_head.float())
+    assert torch.equal(got, model.decode_step(toks[:, -1], 5, cache, ExactDecodeBackend()))
+    # the norm's sum in another order can move its rounding by one bf16 unit
+    assert (got - want).abs().max() <= 2.0 ** -7 * want.abs().max()
 
 
 def test_prefill_and_step_under_autocast():
