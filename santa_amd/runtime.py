@@ -510,7 +510,7 @@ class RandomLlama:
                 and s.intermediate % 8 == 0 and s.hidden % 8 == 0
                 and B * P * (s.heads + 2 * s.kv_heads) * s.head_dim < 1 << 34
                 and all(t.shape == shape and t.dtype == h.dtype and t.device == h.device and t.is_contiguous()
-                        and t.data_ptr() % 16 == 0 for t in cache.k + cache.v)
+                        and t.data_ptr() % 16 == 0 for t in (*cache.k, *cache.v))
                 and all(w.dtype == h.dtype and w.is_contiguous() for L in self.layers for w in (L["ln1"], L["ln2"]))
                 and self.norm.dtype == h.dtype and self.norm.is_contiguous() and _plain(h))
 

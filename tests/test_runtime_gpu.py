@@ -82,6 +82,25 @@ def test_model_without_layers():
     assert (got - want).abs().max() <= 2.0 ** -7 * want.abs().max()
 
 
+def test_prefill_into_stacked_caches():
+    """Caches that are one tensor over the layers, cut from a wider one (rows
+    not packed): the same K and V in their places, nothing beside them."""
+    print("\n[case] prefill into stacked caches", flush=True)
+    dev = torch.device("cuda:0")
+    model = RandomLlama(SMALL, seed=7, std=0.05, device=dev)
+    toks = torch.randint(0, SMALL.vocab, (2, 33), generator=torch.Generator().manual_seed(10)).to(dev)
+    plain, stacked = (NHDCache(SMALL, 2, 40, torch.bfloat16, dev) for _ in range(2))
+    want = model.prefill(toks, plain)
+    wide = [torch.zeros(SMALL.layers, 2, 40, 3, 128, device=dev, dtype=torch.bfloat16) for _ in range(2)]
+    stacked.k, stacked.v = wide[0][:, :, :, 1:2], wide[1][:, :, :, 1:2]
+    got = model.prefill(toks, stacked)
+    torch.cuda.synchronize()
+    for a, b in [(got, want)] + list(zip([*stacked.k, *stacked.v], plain.k + plain.v)):
+        a, b = a.float(), b.float()
+        assert (a - b).abs().max() <= 8 * 2.0 ** -8 * b.abs().max()  # the torch expressions' roundings, two layers
+    assert not any(w[:, :, :, i].any() for w in wide for i in (0, 2))
+
+
 def test_prefill_and_step_under_autocast():
     """Autocast to float16, torch's default on a GPU: the prefill is the torch
     expressions under the same autocast, and a step of more sequences than the
