@@ -77,6 +77,11 @@ __device__ __forceinline__ void load_lds16(__amdgpu_buffer_rsrc_t rs, u32x4* dst
   __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)(dst), 16, off, 0, 0, 0);
 }
 
+// Where running maxima start: below every finite score, so that scores of -inf
+// (masked through K) weigh nothing as long as one key of the query is finite;
+// relative to a maximum of -inf they would be NaN.
+constexpr float kLowest = -3.402823466e38f;
+
 constexpr int kTileKeys = 64;
 constexpr int kTileVecs = kTileKeys * kD * 2 / 16;  // 16-byte LDS slots of one K or V tile
 
@@ -191,7 +196,7 @@ __global__ __launch_bounds__(64 * NW, 2) void causal_attention_kernel(
   for (int mb = 0; mb < 4; ++mb)
 #pragma unroll
     for (int i = 0; i < 16; ++i) o[mb][i] = 0.0f;
-  float m = -__builtin_inff(), l = 0.0f;  // running max (of the raw scores) and this half's sum
+  float m = kLowest, l = 0.0f;  // running max (of the raw scores) and this half's sum
 
   for (int t = 0; t < nt; ++t) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -379,7 +384,7 @@ __global__ __launch_bounds__(64 * kDecWaves) void exact_decode_kernel(
     for (int d = 0; d < 8; ++d) o[g][d] = 0.0f;
   // of the head whose scores end in this lane: running max (raw scores) and
   // the mass of this row's positions
-  float m = -__builtin_inff(), l = 0.0f;
+  float m = kLowest, l = 0.0f;
 
   for (int n = n_begin; n < n_end; n += kDecStep) {
     float s[8];

@@ -112,6 +112,24 @@ def test_causal_attention_large_scores():
     assert ((out.float() - ref).abs() <= 2.0 ** -8 * ref.abs() + (2.0 ** -8 + 1.3e-2) * v.float().abs().max()).all()
 
 
+def test_attention_minus_infinite_scores():
+    """Keys masked through K, more of them than a tile, a step and a chunk
+    hold, before the first one that counts: they weigh nothing, and a query
+    with no other key is NaN, as in torch's softmax."""
+    print("\n[case] attention, the first 100 keys at -inf", flush=True)
+    g = torch.Generator().manual_seed(7)
+    P, n, bf = 300, 100, torch.bfloat16
+    q, k, v = (torch.randn(1, P, h, 128, generator=g) for h in (4, 1, 1))
+    q[..., 5], k[:, :n, :, 5] = 1.0, -math.inf
+    q, k, v = (t.to("cuda", bf) for t in (q, k, v))
+    out = causal_attention(q, k, v)
+    assert out[:, :n].isnan().all()
+    _check(out[:, n:], _ref(q, k, v)[:, n:], v, bf)
+    for L in (n + 1, P):
+        _check_decode(ExactDecodeBackend().decode(q[:, -1], k, v, L), _ref_decode(q[:, -1], k, v, L), v, bf)
+    assert ExactDecodeBackend().decode(q[:, -1], k, v, n).isnan().all()
+
+
 def test_causal_attention_keeps_autograd():
     """With gradients asked for, the torch expressions run and differentiate."""
     print("\n[case] causal attention under autograd", flush=True)
