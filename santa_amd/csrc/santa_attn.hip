@@ -82,6 +82,12 @@ __device__ __forceinline__ void load_lds16(__amdgpu_buffer_rsrc_t rs, u32x4* dst
 // relative to a maximum of -inf they would be NaN.
 constexpr float kLowest = -3.402823466e38f;
 
+// Above this a maximum in log2 units is subtracted from the scores before they
+// are scaled: fma(score, scale, -round(max * scale)) is off by half an ulp of
+// the product, up to a factor 2^(1/4) common to a query's probabilities here but
+// an overflow from 2^31 on (scores from about 2e10).
+constexpr float kHugeMax = 4194304.0f;
+
 constexpr int kTileKeys = 64;
 constexpr int kTileVecs = kTileKeys * kD * 2 / 16;  // 16-byte LDS slots of one K or V tile
 
@@ -197,6 +203,9 @@ __global__ __launch_bounds__(64 * NW, 2) void causal_attention_kernel(
 #pragma unroll
     for (int i = 0; i < 16; ++i) o[mb][i] = 0.0f;
   float m = kLowest, l = 0.0f;  // running max (of the raw scores) and this half's sum
+  // mc: m in log2 units, or 0 where the scores have m subtracted (kHugeMax);
+  // grows: m, or -inf there, so that every tile's scores pass that way
+  float mc = 0.0f, grows = -__builtin_inff();
 
   for (int t = 0; t < nt; ++t) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -233,16 +242,24 @@ __global__ __launch_bounds__(64 * NW, 2) void causal_attention_kernel(
     // factor (273 us at the size above), keeps the largest probability exactly
     // 1: rounded relative to an older maximum it would be off by up to an ulp,
     // and with it the whole output of a query that attends to one key.
-    if (__any(m_new > m)) {
+    if (__any(m_new > grows)) {
       const float a = __builtin_amdgcn_exp2f((m - m_new) * scale_log2);
       l *= a;
 #pragma unroll
       for (int mb = 0; mb < 4; ++mb)
 #pragma unroll
         for (int i = 0; i < 16; ++i) o[mb][i] *= a;
-      m = m_new;
+      grows = m = m_new;
+      mc = m * scale_log2;
+      if (__any(fabsf(mc) > kHugeMax)) {
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) s[kb][i] -= m;
+        mc = 0.0f;
+        grows = -__builtin_inff();
+      }
     }
-    const float mc = m * scale_log2;
     u32x4 p[4];
 #pragma unroll
     for (int kc = 0; kc < 4; ++kc) {
@@ -385,6 +402,7 @@ __global__ __launch_bounds__(64 * kDecWaves) void exact_decode_kernel(
   // of the head whose scores end in this lane: running max (raw scores) and
   // the mass of this row's positions
   float m = kLowest, l = 0.0f;
+  float mc = 0.0f, grows = -__builtin_inff();  // as in causal_attention_kernel
 
   for (int n = n_begin; n < n_end; n += kDecStep) {
     float s[8];
@@ -404,7 +422,7 @@ __global__ __launch_bounds__(64 * kDecWaves) void exact_decode_kernel(
     mx = fmaxf(mx, fxor<16>(mx, lane));
     mx = fmaxf(mx, fxor<32>(mx, lane));
     const float m_new = fmaxf(m, mx);
-    if (__any(m_new > m)) {
+    if (__any(m_new > grows)) {
       const float a = __builtin_amdgcn_exp2f((m - m_new) * scale_log2);
       l *= a;
       static_for<GHP>([&](auto gc) {
@@ -413,9 +431,15 @@ __global__ __launch_bounds__(64 * kDecWaves) void exact_decode_kernel(
 #pragma unroll
         for (int d = 0; d < 8; ++d) o[g][d] *= ag;
       });
-      m = m_new;
+      grows = m = m_new;
+      mc = m * scale_log2;
+      if (__any(fabsf(mc) > kHugeMax)) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) s[i] -= m;
+        mc = 0.0f;
+        grows = -__builtin_inff();
+      }
     }
-    const float mc = m * scale_log2;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       s[i] = __builtin_amdgcn_exp2f(fmaf(s[i], scale_log2, -mc));

@@ -130,6 +130,28 @@ def test_attention_minus_infinite_scores():
     assert ExactDecodeBackend().decode(q[:, -1], k, v, n).isnan().all()
 
 
+def test_attention_huge_scores():
+    """Scores of 1e12 to 1e16 (finite in float32), 1e13 and more apart: every
+    query attends to its best key alone."""
+    print("\n[case] attention, scores up to 1e16", flush=True)
+    g = torch.Generator().manual_seed(8)
+    P, bf = 300, torch.bfloat16
+    # float32 products of integers below 2^8 and 2^20 sum to the same value for equal keys only
+    level = torch.randperm(P, generator=g).float() + 1.0
+    q = torch.full((1, P, 4, 128), 2.0 ** 20)
+    k = (level * 2.0 ** 18).view(1, P, 1, 1).expand(1, P, 1, 128).contiguous()
+    v = torch.randn(1, P, 1, 128, generator=g)
+    q, k, v = (t.to("cuda", bf) for t in (q, k, v))
+    best = torch.cummax(k[0, :, 0, 0].float(), 0)
+    keep = (k[0, :, 0, 0][None, :] == best.values[:, None]).sum(1)  # bf16 rounds some levels together
+    out = causal_attention(q, k, v)
+    _check(out, _ref(q, k, v), v, bf)
+    one = keep == 1
+    assert one.sum() > 0 and torch.equal(out[0, one], v[0, best.indices[one]].expand(-1, 4, 128))
+    for L in (40, 65, P):
+        _check_decode(ExactDecodeBackend().decode(q[:, -1], k, v, L), _ref_decode(q[:, -1], k, v, L), v, bf)
+
+
 def test_causal_attention_keeps_autograd():
     """With gradients asked for, the torch expressions run and differentiate."""
     print("\n[case] causal attention under autograd", flush=True)
