@@ -111,14 +111,18 @@ class _FusedOps:
         """santa_rt_<fn>(*args, stream) on t's device and its current stream,
         with that device current: a default stream is 0, which the runtime
         takes as the current device's."""
+        fn = getattr(cls.lib(), "santa_rt_" + fn)
+        if torch.cuda.current_device() == t.get_device():
+            cls._check(fn(*args, torch.cuda.current_stream(t.device).cuda_stream))
+            return
         with torch.cuda.device(t.device):
-            cls._check(getattr(cls.lib(), "santa_rt_" + fn)(*args, torch.cuda.current_stream(t.device).cuda_stream))
+            cls._check(fn(*args, torch.cuda.current_stream(t.device).cuda_stream))
 
     @classmethod
     def add_rms_norm(cls, h: torch.Tensor, a: Optional[torch.Tensor], w: torch.Tensor, eps: float) -> torch.Tensor:
         """h += a (in place, bf16) when a is given; returns rms_norm(h) * w."""
-        assert h.is_contiguous() and (a is None or a.is_contiguous())
-        assert all(t is None or t.dtype == torch.bfloat16 for t in (h, a, w))
+        assert h.is_contiguous() and h.dtype == w.dtype == torch.bfloat16
+        assert a is None or (a.is_contiguous() and a.dtype == h.dtype)
         x = torch.empty_like(h)
         rows, hidden = h.numel() // h.shape[-1], h.shape[-1]
         cls._launch(h, "add_rms_norm", h.data_ptr(), a.data_ptr() if a is not None else None, w.data_ptr(),
@@ -131,7 +135,7 @@ class _FusedOps:
         """q rotated ([B, H, D]); k rotated and v written to the caches at pos."""
         assert qkv.is_contiguous() and cos.is_contiguous() and sin.is_contiguous()
         kc, vc = cache.k[layer], cache.v[layer]
-        assert all(t.dtype == torch.bfloat16 for t in (qkv, cos, sin, kc, vc))
+        assert torch.bfloat16 == qkv.dtype == cos.dtype == sin.dtype == kc.dtype == vc.dtype
         B = qkv.shape[0]
         q = torch.empty(B, heads, head_dim, dtype=qkv.dtype, device=qkv.device)
         cls._launch(qkv, "rope_write", qkv.data_ptr(), cos.data_ptr(), sin.data_ptr(), q.data_ptr(), kc.data_ptr(),
@@ -152,7 +156,7 @@ class _FusedOps:
         """rope_write for the positions 0 .. P-1 of a prefill: qkv [B, P, ...],
         cos and sin [P, head_dim]; q rotated ([B, P, H, D]) returned."""
         assert qkv.is_contiguous() and cos.is_contiguous() and sin.is_contiguous()
-        assert all(t.dtype == torch.bfloat16 for t in (qkv, cos, sin, k_cache, v_cache))
+        assert torch.bfloat16 == qkv.dtype == cos.dtype == sin.dtype == k_cache.dtype == v_cache.dtype
         B, P = qkv.shape[:2]
         q = torch.empty(B, P, heads, head_dim, dtype=qkv.dtype, device=qkv.device)
         cls._launch(qkv, "rope_write_rows", qkv.data_ptr(), cos.data_ptr(), sin.data_ptr(), q.data_ptr(),
@@ -213,7 +217,7 @@ class _FusedOps:
                 and cos.is_contiguous() and sin.is_contiguous() and head_dim % 2 == 0):
             return cls.rope_write(cls.linear(x, w), cos, sin, cache, layer, pos, heads, kv_heads, head_dim)
         kc, vc = cache.k[layer], cache.v[layer]
-        assert all(t.dtype == torch.bfloat16 for t in (cos, sin, kc, vc))
+        assert torch.bfloat16 == cos.dtype == sin.dtype == kc.dtype == vc.dtype
         q = torch.empty(B, heads, head_dim, dtype=x.dtype, device=x.device)
         cls._launch(x, "linear_rope", x.data_ptr(), w.data_ptr(), B, K, cos.data_ptr(), sin.data_ptr(), q.data_ptr(),
                     kc.data_ptr(), vc.data_ptr(), heads, kv_heads, head_dim, kc.shape[1], pos)
@@ -230,31 +234,33 @@ class _FusedOps:
         return out
 
     @staticmethod
-    def _attention_operand(t: torch.Tensor):
-        """t [B, P, heads, 128] as the attention kernels address it, with its
-        batch, position and head strides: last dimension contiguous, strides
-        of whole 16-byte pieces, positions at least a row apart (the kernels
-        tell rows past the end by their offset) and less than 2^24 elements,
-        16-byte aligned; a packed copy where t is laid out otherwise.  A
-        dimension of size 1 counts as packed: its stride is never used and
-        can be any number, also in a tensor that is_contiguous."""
-        def strides(x):
-            packed = (x.shape[1] * x.shape[2] * 128, x.shape[2] * 128, 128)
-            return [d if n == 1 else s for n, s, d in zip(x.shape, x.stride(), packed)]
-
-        st = strides(t)
-        if t.stride(3) != 1 or any(s % 8 for s in st) or not 128 <= st[1] < 1 << 24 or t.data_ptr() % 16:
-            t = torch.empty(t.shape, dtype=t.dtype, device=t.device).copy_(t)
-            st = strides(t)
-        return t, st
+    def _attention_operand(t: torch.Tensor, rows: int):
+        """t [B, P, heads, 128], of which the first rows positions count, as
+        the attention kernels address it, with its batch, position and head
+        strides: last dimension contiguous, strides of whole 16-byte pieces,
+        positions at least a row apart (the kernels tell rows past the end by
+        their offset) and less than 2^24 elements, 16-byte aligned; a packed
+        copy where t is laid out otherwise.  A dimension of size 1 counts as
+        packed: its stride is never used and can be any number, also in a
+        tensor that is_contiguous."""
+        B, P, heads, _ = t.shape
+        sb, sp, sh, sd = t.stride()
+        sb = P * heads * 128 if B == 1 else sb
+        sp = heads * 128 if P == 1 else sp
+        sh = 128 if heads == 1 else sh
+        if sd == 1 and not (sb | sp | sh) & 7 and 128 <= sp < 1 << 24 and not t.data_ptr() & 15:
+            return t, (sb, sp, sh)
+        t = t[:, :rows]
+        t = torch.empty(t.shape, dtype=t.dtype, device=t.device).copy_(t)
+        return t, (rows * heads * 128, heads * 128, 128)
 
     @classmethod
     def causal_attention(cls, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> torch.Tensor:
         """causal_attention of [B, P, heads, 128] tensors as one kernel."""
         B, P, H, D = q.shape
         out = torch.empty(B, P, H, D, dtype=q.dtype, device=q.device)
-        (q, sq), (k, sk), (v, sv) = (cls._attention_operand(t) for t in (q, k, v))
-        strides = (ctypes.c_longlong * 12)(*sq, *sk, *sv, *out.stride()[:3])
+        (q, sq), (k, sk), (v, sv) = (cls._attention_operand(t, P) for t in (q, k, v))
+        strides = (ctypes.c_longlong * 12)(*sq, *sk, *sv, P * H * D, H * D, D)
         cls._launch(q, "causal_attention", q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
                     int(q.dtype == torch.float16), B, P, H, k.shape[2], D, strides)
         return out
@@ -265,16 +271,19 @@ class _FusedOps:
         of k, v [B, T, KVH, 128]."""
         q = q.contiguous()
         q = q if q.data_ptr() % 16 == 0 else q.clone()
-        (k, sk), (v, sv) = (cls._attention_operand(t[:, :L]) for t in (k, v))
+        (k, sk), (v, sv) = cls._attention_operand(k, L), cls._attention_operand(v, L)
         B, H, D = q.shape
         KVH = k.shape[2]
         out = torch.empty(B, H, D, dtype=q.dtype, device=q.device)
         strides = (ctypes.c_longlong * 6)(*sk, *sv)
-        with torch.cuda.device(q.device):  # the plan asks for the device's CUs
-            ws = torch.empty(cls.lib().santa_rt_exact_decode_workspace_size(B, L, H, KVH), dtype=torch.uint8,
+        lib = cls.lib()
+        with torch.cuda.device(q.device):
+            ws = torch.empty(lib.santa_rt_exact_decode_workspace_size(B, L, H, KVH), dtype=torch.uint8,
                              device=q.device)
-        cls._launch(q, "exact_decode", q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
-                    int(q.dtype == torch.float16), B, L, H, KVH, D, strides, ws.data_ptr(), ws.numel())
+            cls._check(lib.santa_rt_exact_decode(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
+                                                 int(q.dtype == torch.float16), B, L, H, KVH, D, strides,
+                                                 ws.data_ptr(), ws.numel(),
+                                                 torch.cuda.current_stream(q.device).cuda_stream))
         return out
 
     @classmethod

@@ -47,6 +47,7 @@ def recorder(monkeypatch):
 
     rec = _Recorder(current)
     monkeypatch.setattr(torch.cuda, "device", device)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)  # a CPU tensor's get_device() is -1
     monkeypatch.setattr(torch.cuda, "current_stream", lambda d=None: stream)
     monkeypatch.setattr(_FusedOps, "_lib", rec)
     return rec
