@@ -352,7 +352,7 @@ __device__ __forceinline__ int union_rows(const uint64_t* s_mask, int lane) {
 // as many resident waves as fit without spilling: six per SIMD (80 VGPRs)
 // for one head per wave at block_n 256, four (128) otherwise; the V gathers
 // go out 16 rows at a time (cfg3 step 542 -> 518 us).
-template <bool BF16, int GH, int BN, bool HM, bool PAGED = false>
+template <bool BF16, int GH, int BN, bool HM, bool PAGED = false, bool PAD = false>
 __global__ __launch_bounds__(kThreads, (GH == 4 && BN == 256 && !PAGED) ? 6 : 4) void pass2_kernel(const uint16_t* __restrict__ V,
                                                          const uint16_t* __restrict__ u_stash, int H, int KVH,
                                                          int L, int L_storage, int T_c, int cs, int cpg,
@@ -374,9 +374,11 @@ __global__ __launch_bounds__(kThreads, (GH == 4 && BN == 256 && !PAGED) ? 6 : 4)
   const int kv = gp.kv;
   const int chunk = gp.chunk;
   const int b = gp.b < 0 ? 0 : gp.b;
-  // heads per KV head: GH, except that GH 8 also takes groups of 5-7 heads, the
-  // missing ones with a zero budget everywhere and no partial
-  const int gsz = (GH == 8) ? H / KVH : GH;
+  // heads per KV head: GH, except that the PAD form takes groups of fewer (5-7
+  // for GH 8), the missing ones with a zero budget everywhere and no partial.
+  // A form of its own: carried through the GH 8 kernel, the group size cost it
+  // 15-18 more SGPR spills (64q/8kv, one sequence of 16k: 41.4 -> 42.1 us).
+  const int gsz = PAD ? H / KVH : GH;
   const int h0 = kv * gsz;
   L = gp.len;  // this sequence's length from here on
   const int t_begin = chunk * cs;
@@ -477,7 +479,7 @@ __global__ __launch_bounds__(kThreads, (GH == 4 && BN == 256 && !PAGED) ? 6 : 4)
     const int tt = min(t0 + lane, t_end - 1);
 #pragma unroll
     for (int k = 0; k < HPW; ++k) {
-      const bool real = GH != 8 || wave + 4 * k < gsz;
+      const bool real = !PAD || wave + 4 * k < gsz;
       const size_t ht = (static_cast<size_t>(b) * H + h0 + (real ? wave + 4 * k : 0)) * T_c + tt;
       inv_l[k] = real ? invdelta[ht] : 0.0f;
       a0_l[k] = a0_tile[ht];
@@ -504,7 +506,7 @@ __global__ __launch_bounds__(kThreads, (GH == 4 && BN == 256 && !PAGED) ? 6 : 4)
       bool any = false;
 #pragma unroll
       for (int g = 0; g < GH; ++g)
-        any = any || ((GH != 8 || g < gsz) && invdelta[(static_cast<size_t>(b) * H + h0 + g) * T_c + tt] > 0.0f);
+        any = any || ((!PAD || g < gsz) && invdelta[(static_cast<size_t>(b) * H + h0 + g) * T_c + tt] > 0.0f);
       act = any;
     }
     return __ballot(act);
@@ -622,7 +624,7 @@ __global__ __launch_bounds__(kThreads, (GH == 4 && BN == 256 && !PAGED) ? 6 : 4)
   for (int k = 0; k < HPW; ++k) {
     flush(k, wave + 4 * k);
     float* pp = part + (static_cast<size_t>(wg) * gsz + wave + 4 * k) * kD;
-    if (GH != 8 || wave + 4 * k < gsz) reinterpret_cast<float2*>(pp)[lane] = make_float2(acc0[k], acc1[k]);
+    if (!PAD || wave + 4 * k < gsz) reinterpret_cast<float2*>(pp)[lane] = make_float2(acc0[k], acc1[k]);
   }
   if (tid == 0) part_emit[wg] = emit_total;
 }
@@ -685,15 +687,23 @@ static hipError_t launch_pass2_t(const uint16_t* V, const uint16_t* u_stash, int
   const unsigned grid = rg.seq_lens ? static_cast<unsigned>(rg.n_wg)
                                     : static_cast<unsigned>(B) * static_cast<unsigned>(KVH) * static_cast<unsigned>(cpg);
   if (grid == 0) return hipSuccess;
-#define SANTA_P2_LAUNCH(HM, PG, SLD)                                                                               \
-  hipLaunchKernelGGL((pass2_kernel<BF16, GH, BN, HM, PG>), dim3(grid), dim3(kThreads), 0, stream, V, u_stash, H, KVH, \
-                     L, L_storage, T_c, cs, cpg, invdelta, a0, counts, part, part_emit, want_emit, rg.seq_lens, B,    \
+#define SANTA_P2_LAUNCH(HM, PG, PAD, SLD)                                                                          \
+  hipLaunchKernelGGL((pass2_kernel<BF16, GH, BN, HM, PG, PAD>), dim3(grid), dim3(kThreads), 0, stream, V, u_stash, H, \
+                     KVH, L, L_storage, T_c, cs, cpg, invdelta, a0, counts, part, part_emit, want_emit, rg.seq_lens, B,    \
                      SLD, rg.pt)
   const bool hm = BN == 256 && rg.stash_ld > 0;
+  if constexpr (GH == 8 && BN == 256) {
+    if (H != KVH * GH) {  // groups of 5-7 heads (pass2_pad8), always over a tile-major stash
+      if (!hm) return hipErrorInvalidValue;
+      if (rg.pt.table) SANTA_P2_LAUNCH(true, true, true, rg.stash_ld);
+      else SANTA_P2_LAUNCH(true, false, true, rg.stash_ld);
+      return hipGetLastError();
+    }
+  }
   if (rg.pt.table) {
-    if (hm) SANTA_P2_LAUNCH(true, true, rg.stash_ld); else SANTA_P2_LAUNCH(false, true, 0);
+    if (hm) SANTA_P2_LAUNCH(true, true, false, rg.stash_ld); else SANTA_P2_LAUNCH(false, true, false, 0);
   } else {
-    if (hm) SANTA_P2_LAUNCH(true, false, rg.stash_ld); else SANTA_P2_LAUNCH(false, false, 0);
+    if (hm) SANTA_P2_LAUNCH(true, false, false, rg.stash_ld); else SANTA_P2_LAUNCH(false, false, false, 0);
   }
 #undef SANTA_P2_LAUNCH
   return hipGetLastError();
