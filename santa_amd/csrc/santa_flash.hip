@@ -369,7 +369,12 @@ __global__ __launch_bounds__(kThreads, 2) void tile_kernel(
   // the missing successor of a chunk's last tile (no branches, so the loaded
   // registers are never copied and no wait lands before the scores).
   // Paged: pv holds the pages of the wave's 16 row groups of the tile (one per
-  // lane), loaded a tile ahead; a 4-row group never straddles two pages.
+  // lane), loaded a tile ahead; a 4-row group never straddles two pages.  The
+  // general pass 1 at GH 8, which spills registers, holds the tile's pages
+  // instead and forms each load's address from one (8 sequences of 800-3,000
+  // over 16-token pages, 64q/8kv: 331.3 us with the groups' addresses, 325.9
+  // so; at GH 4 the addresses win, 32q/8kv 400-1,500 42.8 against 44.4).
+  constexpr bool LANE_ADDR = !(MODE == kPass1Gen && GH == 8);
   u32x4 kw[16];
   const int k_lane_off = static_cast<int>((lane >> 4) * row_bytes + 16u * (lane & 15));
   auto load_k = [&](int t, int pv) {
@@ -377,14 +382,19 @@ __global__ __launch_bounds__(kThreads, 2) void tile_kernel(
     const int len = (t < t_end) ? min(BN, L_valid - n0) : 0;
     const char* kt = Kg + static_cast<size_t>(n0 + 64 * wave) * row_bytes;
     LaneAddr av{0u, 0u};
-    if constexpr (PAGED) av = lane_addr(Kg + paged_row(pt, pv, n0 + 64 * wave + 4 * (lane & 15), row_bytes));
+    if constexpr (PAGED && LANE_ADDR)
+      av = lane_addr(Kg + paged_row(pt, pv, n0 + 64 * wave + 4 * (lane & 15), row_bytes));
 #pragma unroll
     for (int c = 0; c < 16; ++c) {
       // wave-uniform; readfirstlane keeps the descriptor in SGPRs
       const int nvalid = __builtin_amdgcn_readfirstlane(min(max(len - 64 * wave - 4 * c, 0), 4));
       const char* gb;
-      if constexpr (PAGED) {
+      if constexpr (PAGED && LANE_ADDR) {
         gb = addr_of_lane(av, c);
+      } else if constexpr (PAGED) {
+        const int n = n0 + 64 * wave + 4 * c;
+        const int page = __builtin_amdgcn_readlane(pv, (n >> pt.shift) - ((n0 + 64 * wave) >> pt.shift));
+        gb = Kg + paged_row(pt, page, n, row_bytes);
       } else {
         gb = kt + static_cast<size_t>(4 * c) * row_bytes;
       }
@@ -394,6 +404,7 @@ __global__ __launch_bounds__(kThreads, 2) void tile_kernel(
     }
   };
   auto wave_pages = [&](int t) -> int {
+    if constexpr (PAGED && !LANE_ADDR) return pages_of_rows(pt, b, t * BN + 64 * wave, 64, L_valid, lane);
     return PAGED ? pages_of_groups<4, 16>(pt, b, t * BN + 64 * wave, L_valid, lane) : 0;
   };
   load_k(t_begin, wave_pages(t_begin));
