@@ -233,6 +233,10 @@ struct RaggedSeq {
 __device__ __forceinline__ RaggedSeq ragged_seq(const int* seq_lens, int b, int B, int max_rows, int BN, int cs,
                                                 const DenseCut& dense) {
   RaggedSeq s{0, 0, cs};
+  if (B == 1 && dense.limit == 0) {  // one sequence: nothing to scan
+    s.tiles = (ragged_len(seq_lens, 0, max_rows) + BN - 1) / BN;
+    return s;
+  }
   for (int g0 = 0; g0 <= b; g0 += 64) {
     const RaggedLane r = ragged_lane(seq_lens, g0, B, max_rows, BN, cs, dense);
     if (b < g0 + 64) {
@@ -270,6 +274,18 @@ __device__ __forceinline__ GridPos grid_pos(int wg, const int* seq_lens, int B, 
   p.n_tiles = 0;
   p.wg_base = 0;
   const int item = wg / KVH;
+  if (B == 1 && dense.limit == 0) {  // one sequence: no scan before the first load
+    const int len = ragged_len(seq_lens, 0, L_valid);
+    const int tiles = (len + BN - 1) / BN;
+    if (item * cs < tiles) {
+      p.b = 0;
+      p.kv = wg - item * KVH;
+      p.chunk = item;
+      p.len = len;
+      p.n_tiles = tiles;
+    }
+    return p;
+  }
   int first = 0;
   for (int g0 = 0; g0 < B; g0 += 64) {
     const RaggedLane r = ragged_lane(seq_lens, g0, B, L_valid, BN, cs, dense);

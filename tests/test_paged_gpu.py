@@ -111,6 +111,9 @@ def test_flash_paged_matches_contiguous(H, KVH, lens, S, page_size, block_n, dty
         (32, 8, [12000, 3100, 7777, 4096], [256, 64, 300, 1], 16, 0, None, True),  # vec pass 1 (wave kernel)
         (32, 8, [12000, 3100, 7777, 4096], [256, 64, 300, 1], 16, 0, "gqa", True),  # general pass 1
         (16, 2, [1, 33, 500, 1000], [7, 40, 256, 1000], 8, 32, None, True),        # block_n 32, GH 8
+        (64, 8, [1, 65, 2000, 2999], [7, 40, 256, 1000], 8, 64, None, True),       # block_n 64, GH 8
+        (64, 8, [5000, 257], [256, 40], 16, 256, None, True),                      # GH 8, few tiles
+        (64, 8, [2990], [300], 64, 64, None, True),                                # one sequence
         (32, 8, [5000, 9000], [100, 0], 512, 0, None, True),                       # S = 0 for one sequence
         (32, 8, [1000, 8000, 2000], [256, 256, 256], 64, 0, None, False),          # mixed block sizes
     ],
