@@ -66,9 +66,11 @@ def test_causal_attention_strided():
     q, k, v = qkv.split([H, KVH, KVH], dim=2)
     want = _ref(q, k, v)
     _check(causal_attention(q, k, v), want, v, torch.bfloat16)
-    cache = torch.full((B, P + 9, KVH, 128), float("nan"), device="cuda", dtype=torch.bfloat16)
-    cache[:, :P] = k
-    _check(causal_attention(q, cache[:, :P], v), want, v, torch.bfloat16)
+    # the prompt's part of caches whose tails hold anything: a V row read past
+    # the end would show (0 * NaN), a K row only where its score is not masked
+    ck, cv = (torch.full((B, P + 9, KVH, 128), float("nan"), device="cuda", dtype=torch.bfloat16) for _ in range(2))
+    ck[:, :P], cv[:, :P] = k, v
+    _check(causal_attention(q, ck[:, :P], cv[:, :P]), want, v, torch.bfloat16)
     odd = torch.empty(B * P * H * 128 + 1, device="cuda", dtype=torch.bfloat16)[1:].view(B, P, H, 128)
     odd.copy_(q)
     _check(causal_attention(odd, k, v), want, v, torch.bfloat16)
@@ -152,12 +154,54 @@ def test_attention_huge_scores():
         _check_decode(ExactDecodeBackend().decode(q[:, -1], k, v, L), _ref_decode(q[:, -1], k, v, L), v, bf)
 
 
-def test_causal_attention_keeps_autograd():
-    """With gradients asked for, the torch expressions run and differentiate."""
-    print("\n[case] causal attention under autograd", flush=True)
-    q, k, v = (torch.randn(1, 40, h, 128, device="cuda", dtype=torch.bfloat16, requires_grad=True) for h in (4, 1, 1))
+def test_attention_keeps_autograd():
+    """With gradients asked for of tensors the kernels would take, the torch
+    expressions run: the outputs are differentiable.  The causal attention's
+    backward is not run in bf16 (its batched products would have transposed
+    right operands); the same expressions differentiate in float32."""
+    print("\n[case] attention under autograd", flush=True)
+    g = torch.Generator().manual_seed(9)
+    q, k, v = (torch.randn(1, 40, h, 128, generator=g).to("cuda", torch.bfloat16).requires_grad_() for h in (4, 1, 1))
+    with torch.no_grad():
+        kernel = causal_attention(q, k, v)
+    out = causal_attention(q, k, v)
+    assert out.grad_fn is not None and kernel.grad_fn is None
+    # the kernel's tolerance for both, and the torch path's scores rounded to bf16: |q . k| < 64 here,
+    # so off by 64 x 2^-9 before the scale of 128^-1/2
+    eps, vmax = 2.0 ** -8, v.detach().float().abs().max()
+    assert ((out - kernel).float().abs() <= 2 * (2 * eps + 2e-4 + 64 * 2.0 ** -9 / math.sqrt(128)) * vmax).all()
     causal_attention(q.float(), k.float(), v.float()).sum().backward()
     assert all(t.grad is not None and torch.isfinite(t.grad).all() for t in (q, k, v))
+
+    leaves = [t.detach().clone().requires_grad_() for t in (q[:, -1], k, v)]
+    w = torch.randn(1, 4, 128, generator=g).to("cuda", torch.bfloat16)
+    dec = ExactDecodeBackend().decode(*leaves, 33)
+    assert dec.grad_fn is not None
+    (dec * w).float().sum().backward()
+    d = [t.detach().double().cpu().requires_grad_() for t in leaves]
+    p = torch.softmax(torch.einsum("hd,ld->hl", d[0][0], d[1][0, :33, 0]) / math.sqrt(128), -1)
+    ((p @ d[2][0, :33, 0]) * w[0].double().cpu()).sum().backward()
+    for got, want in zip(leaves, d):
+        # the gradient in bf16 of a bf16 output: one rounding of each, float32 between
+        assert (got.grad.double().cpu() - want.grad).norm() <= 2.0 ** -7 * want.grad.norm()
+
+
+def test_attention_on_a_stream_of_its_own():
+    """The kernels run on the current stream, behind what that stream wrote."""
+    print("\n[case] attention on a side stream", flush=True)
+    g = torch.Generator().manual_seed(10)
+    q, k, v = (torch.randn(2, 200, h, 128, generator=g).to("cuda", torch.bfloat16) for h in (8, 2, 2))
+    want, wantd = causal_attention(q, k, v), ExactDecodeBackend().decode(q[:, -1], k, v, 200)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        x = torch.randn(4096, 4096, device="cuda")
+        for _ in range(8):  # work in front, so that a launch elsewhere would come too early
+            x = x @ x * 1e-2
+        k2 = torch.zeros_like(k) + x[:1, :1].to(k.dtype).nan_to_num(0.0) * 0 + k
+        got, gotd = causal_attention(q, k2, v), ExactDecodeBackend().decode(q[:, -1], k2, v, 200)
+    torch.cuda.current_stream().wait_stream(side)
+    assert torch.equal(got, want) and torch.equal(gotd, wantd)
 
 
 def _ref_decode(q, k, v, L):
