@@ -12,6 +12,8 @@
 #include "santa_amd.h"
 #include "santa_internal.h"
 
+#include <algorithm>
+
 namespace santa {
 namespace rt {
 
@@ -588,23 +590,29 @@ extern "C" int santa_rt_add_rms_norm(void* h, const void* a, const void* w, void
   const bool vec = hidden % 8 == 0 && nv <= 4 * rt::kNormVecThreads &&
                    ((reinterpret_cast<uintptr_t>(h) | reinterpret_cast<uintptr_t>(a) |
                      reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(x)) % 16) == 0;
-  uint16_t* hp = static_cast<uint16_t*>(h);
-  const uint16_t* ap = static_cast<const uint16_t*>(a);
-  const uint16_t* wp = static_cast<const uint16_t*>(w);
-  uint16_t* xp = static_cast<uint16_t*>(x);
   const int add = a ? 1 : 0;
-  if (vec && nv <= rt::kNormVecThreads)
-    hipLaunchKernelGGL(rt::add_rms_norm_vec_kernel<1>, dim3(rows), dim3(rt::kNormVecThreads), 0, stream, hp, ap, wp,
-                       xp, hidden, eps, add);
-  else if (vec && nv <= 2 * rt::kNormVecThreads)
-    hipLaunchKernelGGL(rt::add_rms_norm_vec_kernel<2>, dim3(rows), dim3(rt::kNormVecThreads), 0, stream, hp, ap, wp,
-                       xp, hidden, eps, add);
-  else if (vec)
-    hipLaunchKernelGGL(rt::add_rms_norm_vec_kernel<4>, dim3(rows), dim3(rt::kNormVecThreads), 0, stream, hp, ap, wp,
-                       xp, hidden, eps, add);
-  else
-    hipLaunchKernelGGL(rt::add_rms_norm_kernel, dim3(rows), dim3(rt::kNormThreads), 0, stream, hp, ap, wp, xp, hidden,
-                       eps, add);
+  // a launch holds fewer than 2^32 threads and drops the rest without an error
+  constexpr int kRows = 1 << 22;
+  for (long long r0 = 0; r0 < rows; r0 += kRows) {
+    const dim3 grid(static_cast<unsigned>(std::min<long long>(kRows, rows - r0)));
+    const size_t at = static_cast<size_t>(r0) * hidden;
+    uint16_t* hp = static_cast<uint16_t*>(h) + at;
+    const uint16_t* ap = a ? static_cast<const uint16_t*>(a) + at : nullptr;
+    const uint16_t* wp = static_cast<const uint16_t*>(w);
+    uint16_t* xp = static_cast<uint16_t*>(x) + at;
+    if (vec && nv <= rt::kNormVecThreads)
+      hipLaunchKernelGGL(rt::add_rms_norm_vec_kernel<1>, grid, dim3(rt::kNormVecThreads), 0, stream, hp, ap, wp, xp,
+                         hidden, eps, add);
+    else if (vec && nv <= 2 * rt::kNormVecThreads)
+      hipLaunchKernelGGL(rt::add_rms_norm_vec_kernel<2>, grid, dim3(rt::kNormVecThreads), 0, stream, hp, ap, wp, xp,
+                         hidden, eps, add);
+    else if (vec)
+      hipLaunchKernelGGL(rt::add_rms_norm_vec_kernel<4>, grid, dim3(rt::kNormVecThreads), 0, stream, hp, ap, wp, xp,
+                         hidden, eps, add);
+    else
+      hipLaunchKernelGGL(rt::add_rms_norm_kernel, grid, dim3(rt::kNormThreads), 0, stream, hp, ap, wp, xp, hidden,
+                         eps, add);
+  }
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return set_error(SANTA_ERR_HIP, "add_rms_norm launch failed: %s", hipGetErrorString(e));
   return clear_error();

@@ -64,6 +64,24 @@ def test_add_rms_norm(rows, hidden):
     _ulp_close(x0, _rms_norm(h, w, 1e-5), 2)
 
 
+@pytest.mark.parametrize("hidden", [8, 12])
+def test_add_rms_norm_many_rows(hidden):
+    """More rows than one launch holds (2^32 threads: 2^23 rows of the vector
+    form, 2^24 of the scalar one), as a prefill of many prompts of a narrow
+    model has: the ends and the seams between launches."""
+    rows = (1 << 24) + 3
+    print(f"\n[case] add_rms_norm rows={rows} hidden={hidden}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(hidden)
+    h = torch.randn(rows, hidden, device=DEV, generator=g, dtype=torch.bfloat16)
+    w = torch.ones(hidden, device=DEV, dtype=torch.bfloat16)
+    x = _FusedOps.add_rms_norm(h, None, w, 1e-5)
+    torch.cuda.synchronize()
+    for at in (0, 1 << 22, 1 << 23, (1 << 24) - 2, rows - 4):
+        part = slice(max(at - 4, 0), at + 4)
+        _ulp_close(x[part], _rms_norm(h[part], w, 1e-5), 2)
+    assert torch.isfinite(x).all()
+
+
 @pytest.mark.parametrize("B,P,H,KVH,D", [(1, 1, 32, 8, 128), (2, 33, 7, 1, 128), (3, 100, 4, 2, 64), (1, 130, 5, 5, 16)])
 def test_rope_write_rows(B, P, H, KVH, D):
     """A prefill's positions: bit for bit the torch expressions, rows of the
