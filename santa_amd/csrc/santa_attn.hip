@@ -7,6 +7,7 @@
 #include "santa_amd.h"
 #include "santa_internal.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace santa {
@@ -566,21 +567,28 @@ extern "C" int santa_rt_causal_attention(const void* q, const void* k, const voi
   constexpr int NW = 4;
   const int GH = H / KVH;
   const long long units = static_cast<long long>((P + 31) / 32) * GH;
-  const long long W = (units + NW - 1) / NW, NG = static_cast<long long>(B) * KVH;
-  if (units > 0x7fffff00LL || W * NG > 0x7fffffffLL)
+  const long long W = (units + NW - 1) / NW;
+  // a launch holds fewer than 2^32 threads and drops the rest without an error:
+  // at most this many sequences each
+  const long long per_seq = W * KVH;
+  const long long fit = (1LL << 32) / (64 * NW) - 1;
+  if (units > 0x7fffff00LL || per_seq > fit)
     return set_error(SANTA_ERR_INVALID, "causal_attention: too many positions");
   const float scale_log2 = 1.44269504088896340736f / sqrtf(static_cast<float>(D));
-  const dim3 grid(static_cast<unsigned>(W * NG)), block(64 * NW);
-  const uint16_t *qp = static_cast<const uint16_t*>(q), *kp = static_cast<const uint16_t*>(k),
-                 *vp = static_cast<const uint16_t*>(v);
-  if (dtype == SANTA_BF16)
-    hipLaunchKernelGGL((attn::causal_attention_kernel<true, NW>), grid, block, 0, stream, qp, kp, vp,
-                       static_cast<uint16_t*>(out), sq, sk, sv, so, P, GH, KVH, static_cast<int>(NG),
-                       static_cast<int>(W), scale_log2);
-  else
-    hipLaunchKernelGGL((attn::causal_attention_kernel<false, NW>), grid, block, 0, stream, qp, kp, vp,
-                       static_cast<uint16_t*>(out), sq, sk, sv, so, P, GH, KVH, static_cast<int>(NG),
-                       static_cast<int>(W), scale_log2);
+  const dim3 block(64 * NW);
+  for (long long b0 = 0, step = fit / per_seq; b0 < B; b0 += step) {
+    const long long n = std::min<long long>(step, B - b0) * KVH;
+    const dim3 grid(static_cast<unsigned>(W * n));
+    const uint16_t *qp = static_cast<const uint16_t*>(q) + b0 * sq.b, *kp = static_cast<const uint16_t*>(k) + b0 * sk.b,
+                   *vp = static_cast<const uint16_t*>(v) + b0 * sv.b;
+    uint16_t* op = static_cast<uint16_t*>(out) + b0 * so.b;
+    if (dtype == SANTA_BF16)
+      hipLaunchKernelGGL((attn::causal_attention_kernel<true, NW>), grid, block, 0, stream, qp, kp, vp, op, sq, sk, sv,
+                         so, P, GH, KVH, static_cast<int>(n), static_cast<int>(W), scale_log2);
+    else
+      hipLaunchKernelGGL((attn::causal_attention_kernel<false, NW>), grid, block, 0, stream, qp, kp, vp, op, sq, sk,
+                         sv, so, P, GH, KVH, static_cast<int>(n), static_cast<int>(W), scale_log2);
+  }
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return set_error(SANTA_ERR_HIP, "causal_attention launch failed: %s", hipGetErrorString(e));
   return clear_error();
@@ -609,35 +617,40 @@ extern "C" int santa_rt_exact_decode(const void* q, const void* k, const void* v
   const int GH = H / KVH, groups = (GH + 7) / 8;
   int chunk, cpg;
   attn::plan_decode(B, L, KVH, groups, &chunk, &cpg);
-  const long long items = static_cast<long long>(B) * KVH * groups * cpg;
-  const long long grid = (items + attn::kDecWaves - 1) / attn::kDecWaves;
-  if (grid > 0x7fffffffLL || static_cast<long long>(B) * H > 0x7fffffffLL)
-    return set_error(SANTA_ERR_INVALID, "exact_decode: batch too large");
+  // a launch holds fewer than 2^32 threads: at most this many sequences each
+  // (a wave per item, 256 threads a head in the merge)
+  const long long per_seq = static_cast<long long>(KVH) * groups * cpg;
+  const long long step = std::min((1LL << 25) / per_seq, (1LL << 23) / H);
+  if (step == 0) return set_error(SANTA_ERR_INVALID, "exact_decode: too many heads");
   const float scale_log2 = 1.44269504088896340736f / sqrtf(static_cast<float>(D));
-  const uint16_t *qp = static_cast<const uint16_t*>(q), *kp = static_cast<const uint16_t*>(k),
-                 *vp = static_cast<const uint16_t*>(v);
-  float* part = static_cast<float*>(workspace);
-  auto launch = [&](auto bf, auto ghp) {
-    constexpr bool BF16 = decltype(bf)::value;
-    constexpr int GHP = decltype(ghp)::value;
-    hipLaunchKernelGGL((attn::exact_decode_kernel<BF16, GHP>), dim3(static_cast<unsigned>(grid)),
-                       dim3(64 * attn::kDecWaves), 0, stream, qp, kp, vp, sk, sv, L, H, KVH, GH, groups, chunk, cpg,
-                       items, scale_log2, part);
-  };
-  auto pick = [&](auto bf) {
-    if (GH == 1) launch(bf, std::integral_constant<int, 1>{});
-    else if (GH == 2) launch(bf, std::integral_constant<int, 2>{});
-    else if (GH <= 4) launch(bf, std::integral_constant<int, 4>{});
-    else launch(bf, std::integral_constant<int, 8>{});
-  };
-  if (dtype == SANTA_BF16) {
-    pick(std::true_type{});
-    hipLaunchKernelGGL(attn::exact_merge_kernel<true>, dim3(static_cast<unsigned>(B) * H), dim3(256), 0, stream, part,
-                       cpg, static_cast<uint16_t*>(out));
-  } else {
-    pick(std::false_type{});
-    hipLaunchKernelGGL(attn::exact_merge_kernel<false>, dim3(static_cast<unsigned>(B) * H), dim3(256), 0, stream, part,
-                       cpg, static_cast<uint16_t*>(out));
+  for (long long b0 = 0; b0 < B; b0 += step) {
+    const long long n = std::min<long long>(step, B - b0);
+    const long long items = n * per_seq;
+    const dim3 grid(static_cast<unsigned>((items + attn::kDecWaves - 1) / attn::kDecWaves));
+    const dim3 heads(static_cast<unsigned>(n * H));
+    const uint16_t *qp = static_cast<const uint16_t*>(q) + b0 * H * D, *kp = static_cast<const uint16_t*>(k) + b0 * sk.b,
+                   *vp = static_cast<const uint16_t*>(v) + b0 * sv.b;
+    uint16_t* op = static_cast<uint16_t*>(out) + b0 * H * D;
+    float* part = static_cast<float*>(workspace) + b0 * H * cpg * attn::kPartStride;
+    auto launch = [&](auto bf, auto ghp) {
+      constexpr bool BF16 = decltype(bf)::value;
+      constexpr int GHP = decltype(ghp)::value;
+      hipLaunchKernelGGL((attn::exact_decode_kernel<BF16, GHP>), grid, dim3(64 * attn::kDecWaves), 0, stream, qp, kp,
+                         vp, sk, sv, L, H, KVH, GH, groups, chunk, cpg, items, scale_log2, part);
+    };
+    auto pick = [&](auto bf) {
+      if (GH == 1) launch(bf, std::integral_constant<int, 1>{});
+      else if (GH == 2) launch(bf, std::integral_constant<int, 2>{});
+      else if (GH <= 4) launch(bf, std::integral_constant<int, 4>{});
+      else launch(bf, std::integral_constant<int, 8>{});
+    };
+    if (dtype == SANTA_BF16) {
+      pick(std::true_type{});
+      hipLaunchKernelGGL(attn::exact_merge_kernel<true>, heads, dim3(256), 0, stream, part, cpg, op);
+    } else {
+      pick(std::false_type{});
+      hipLaunchKernelGGL(attn::exact_merge_kernel<false>, heads, dim3(256), 0, stream, part, cpg, op);
+    }
   }
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return set_error(SANTA_ERR_HIP, "exact_decode launch failed: %s", hipGetErrorString(e));

@@ -186,6 +186,16 @@ def test_attention_keeps_autograd():
         assert (got.grad.double().cpu() - want.grad).norm() <= 2.0 ** -7 * want.grad.norm()
 
 
+def test_attention_many_short_sequences():
+    """More workgroups than one launch holds threads for (2^32): one position
+    each, so the output is v."""
+    B = (1 << 24) + 3
+    print(f"\n[case] attention of {B} sequences of one position", flush=True)
+    q, k, v = (torch.randn(B, 1, 1, 128, device="cuda", dtype=torch.bfloat16) for _ in range(3))
+    assert torch.equal(causal_attention(q, k, v), v)
+    assert torch.equal(ExactDecodeBackend().decode(q[:, 0], k, v, 1), v[:, 0])
+
+
 def test_attention_on_a_stream_of_its_own():
     """The kernels run on the current stream, behind what that stream wrote."""
     print("\n[case] attention on a side stream", flush=True)
