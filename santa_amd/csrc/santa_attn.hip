@@ -120,10 +120,10 @@ struct Strides {
 // reads without bank conflicts.
 //
 // Bound by the matrix cores and the softmax's vector work beside them.  At
-// B = 2, P = 4096, 32q/8kv the call takes 289 us, 954 TFLOP/s over the causal
-// pairs (a large library matrix product reaches 1,349 on this card); the torch
-// expressions it replaces (all P x P scores of a query chunk, written and read
-// back five times over) took 8,513 us.
+// B = 2, P = 4096, 32q/8kv the call takes 280 to 310 us on one card or another,
+// 890 to 980 TFLOP/s over the causal pairs (a large library matrix product
+// reaches 1,349); the torch expressions it replaces (all P x P scores of a query
+// chunk, written and read back five times over) took 8,536 us.
 //
 // The workgroups of one (sequence, KV head) are NG apart, so with NG a
 // multiple of 8 they share an XCD and its L2 holds their K and V; the longest
@@ -311,10 +311,11 @@ __global__ __launch_bounds__(64 * NW, 2) void causal_attention_kernel(
 // this step's are summed, so 8 to 16 KiB per wave are in flight throughout.
 // The KV heads of a chunk are neighbours in launch order (8 waves of a
 // workgroup), so whole NHD rows are read at about the same time.  Bound by
-// reading K and V once: B = 8, 32k, 32q/8kv takes 171 us with its merge (6.27
-// TB/s), 32q/32kv at 8k 168 us (6.39 TB/s); eight heads per KV head double the
-// vector work per row (219 us, 4.90 TB/s).  B = 4, 4k: 21 us against 155 us for
-// the torch products on float32 copies of both caches it replaces.
+// reading K and V once (us per call with the merge, K and V tensors of their
+// own): B = 8, 32k, 32q/8kv 168 (6.4 TB/s), 32q/32kv at 8k 168 (6.4 TB/s); eight
+// heads per KV head double the vector work per row (64q/8kv 202 to 216, 5.0 to 5.3
+// TB/s).  The torch products on float32 copies of both caches it replaces took
+// 1,679, 1,797 and 2,000; B = 4, 4k: 21 against 135.
 constexpr int kDecWaves = 8;
 constexpr int kDecStep = 32;              // positions per step
 constexpr int kPartStride = kD + 2;       // chunk partial: max (log2 units), mass, numerator[128]

@@ -346,8 +346,9 @@ __device__ __forceinline__ size_t paged_row(const PageTable& pt, int page, int n
 // A wave's row-group addresses, one group per lane (the two halves of a 64-bit
 // address), and group i's as a scalar: one vector pass of address arithmetic a
 // tile and two readlanes a load, where a page id read back per load cost it
-// about a dozen scalar instructions of 64-bit shifts and products (8 sequences
-// of 8k-48k over 16-token pages 109.0 -> 105.0 us per step).
+// about a dozen scalar instructions of 64-bit shifts and products (santa_flash, 8
+// sequences of 8k-48k over 16-token pages, us per call: 32q/8kv 106.7 -> 104.9,
+// 64q/8kv 165.3 -> 158.4; two of 4k-9k, on tile_kernel, 33.9 -> 33.2).
 struct LaneAddr {
   uint32_t lo, hi;
 };

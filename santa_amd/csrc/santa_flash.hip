@@ -1548,11 +1548,11 @@ __global__ __launch_bounds__(ROWS ? 512 : kThreads, ROWS ? 1 : 2) void wave_kern
 //
 // Bound by each wave's chain (scores, tail, gathers) at two waves per SIMD.  A
 // chunk planned for a single wave goes to one: four waves per such chunk of three
-// tiles leave most of their lanes without rows (B = 16: 61 us).  us per step at S =
-// 128 and 1,500 tokens, tile_kernel -> strip_kernel: B = 8 29.0 -> 20.1, B = 16
-// 63.1 -> 23.8, B = 32 105.6 -> 35.4; GH 8, B = 2 40.2 -> 27.0, B = 4 62.2 -> 35.2,
-// B = 16 153.2 -> 38.6, B = 32 253.4 -> 59.2; 16 ragged sequences of 300-1,500 (S =
-// 256) 57.0 -> 28.4, GH 8 127.7 -> 48.1.
+// tiles leave most of their lanes without rows (B = 16: 61 us).  us per call at S =
+// 128 and 1,500 tokens, tile_kernel -> strip_kernel: B = 8 29.4 -> 21.6, B = 16
+// 63.7 -> 25.8, B = 32 105.6 -> 37.9; GH 8, B = 2 38.8 -> 27.1, B = 4 59.3 -> 36.2,
+// B = 16 149.1 -> 40.0, B = 32 249.7 -> 61.0; 16 ragged sequences of 300-1,500 (S =
+// 256) 56.4 -> 27.8, GH 8 122.5 -> 44.9.
 constexpr int kStripRows = 128;
 
 // Sum of the four (or eight) warps' sums held at lanes N * w of each 16-lane row,

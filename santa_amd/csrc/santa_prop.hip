@@ -738,8 +738,8 @@ struct PropWs {
   int cs, cpg, n_wg;
   bool pad8;  // groups of 5-7 heads on the tuned pass 2
 };
-// Groups of 5-7 heads at D = 128 and block_n 256 run the tuned GH 8 pass 2 over
-// the tile-major stash (per-tile work of two waves' heads interleaved and the
+// Groups of 5-7 heads at D = 128 and block_n 256 run the tuned GH 8 pass 2 (its
+// PAD form) over the tile-major stash (per-tile work of two waves' heads interleaved and the
 // stash two tiles ahead, where the generic form walks a head at a time): 28q/4kv,
 // B = 8 at 32k, pass 2 28.4 -> 23.2 us.  The debug form (counts) stays generic.
 // From half a resident round of (kv, tile) items; below it the generic form's plan

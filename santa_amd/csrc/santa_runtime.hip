@@ -1,8 +1,9 @@
-// santa_runtime.hip -- fused elementwise kernels of the model-level decode
-// step (santa_amd/runtime.py): the residual add with the RMSNorm that
-// follows it, RoPE of q and k with the step's cache write, and the SwiGLU
-// product.  Each replaces a chain of small torch kernels (about 26 per layer
-// and step) with one launch and keeps torch's bf16 semantics: values are
+// santa_runtime.hip -- the model-level runtime's kernels beside its attention
+// (santa_amd/runtime.py), for the decode step and the prefill: the residual add
+// with the RMSNorm that follows it, RoPE of q and k with the cache write, the
+// SwiGLU product, the decode step's few-row weight products and argmax, and the
+// head's float32 logits.  The elementwise ones each replace a chain of small torch
+// kernels (about 26 per layer and step) and keep torch's bf16 semantics: values are
 // rounded to bf16 where the torch expression rounds them, and the norm is
 // computed in float32 as in the torch expression.  The counterpart in the
 // reference is the HF model's own decoder layer

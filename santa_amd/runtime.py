@@ -62,11 +62,12 @@ def _rms_norm(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
 
 
 class _FusedOps:
-    """The library's fused decode-step kernels (santa_rt_* in santa_amd.h):
-    residual add + RMSNorm, RoPE of q and k with the cache write, SwiGLU.
-    Used for tensors on a GPU; the torch expressions above stay the CPU path
-    and the prefill's.  A GPU decode step fails loudly if the library is not
-    built."""
+    """The library's kernels for the model (santa_rt_* in santa_amd.h):
+    residual add + RMSNorm, RoPE of q and k with the cache write, SwiGLU, the
+    few-row weight products, the exact attention.  Used for tensors on a GPU by
+    the decode step, the prefill and the attention functions, which fail
+    loudly there if the library is not built; the torch expressions stay the
+    CPU path and that of calls the kernels do not take."""
 
     _lib = None
 
@@ -195,8 +196,10 @@ class _FusedOps:
 
     @classmethod
     def logits(cls, x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-        """x @ w.T in float32 for few rows of x (santa_rt_linear_f32: the
-        float32 sums; F.linear widened where the shape does not fit it)."""
+        """x @ w.T as float32.  For few rows of x (linear_fits: up to 8 rows of
+        up to 8192 columns) the product's float32 sums (santa_rt_linear_f32);
+        for more, F.linear's result in x's type, widened: a bf16 model's logits
+        are then rounded to bf16, as without the kernel."""
         rows, K = x.shape
         if not (cls.linear_fits(rows, K) and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
                 and x.is_contiguous() and w.is_contiguous() and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0):
@@ -343,7 +346,8 @@ def causal_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, chunk
     """Exact causal GQA attention for a prefill: q [B, P, H, D], k/v
     [B, P, KVH, D] -> [B, P, H, D].  bf16 and f16 tensors of head_dim 128 on a
     GPU run as one kernel (float32 scores and softmax).  Otherwise, and under
-    autograd, query chunks of `chunk` positions; the products run on contiguous
+    autograd, tracing, dispatch modes or autocast to another type, query chunks
+    of `chunk` positions; the products run on contiguous
     operands only (K is transposed once per call into a contiguous copy and
     every chunk is scored against all of it, the future positions masked),
     scores in the input dtype, softmax in float32."""
@@ -482,7 +486,8 @@ class RandomLlama:
                 attn_chunk: int = 512) -> torch.Tensor:
         """Causal forward over the prompt tokens [B, P]; writes K/V of positions
         0..P-1 into the caches and returns the last position's logits [B, V]
-        (float32).  Attention is exact (causal_attention)."""
+        (float32; on a GPU the head's float32 sums for up to 8 prompts, rounded
+        to the model's type for more).  Attention is exact (causal_attention)."""
         s, D = self.shape, self.shape.head_dim
         B, P = tokens.shape
         pos = torch.arange(P, device=self.device)
@@ -553,7 +558,7 @@ class RandomLlama:
     def decode_step(self, token: torch.Tensor, pos: int, cache: NHDCache, backend) -> torch.Tensor:
         """One token per sequence (token [B]) at position pos: cache writes, the
         backend's attention over positions 0..pos, and the logits [B, V]
-        (float32) -- tutorial_code/runtime_common.py:501-571."""
+        (float32, as prefill's) -- tutorial_code/runtime_common.py:501-571."""
         s, D = self.shape, self.shape.head_dim
         B = token.shape[0]
         h = self.embed[token]  # [B, hidden]
